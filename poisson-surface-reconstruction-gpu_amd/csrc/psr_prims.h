@@ -56,8 +56,8 @@ constexpr int kSortTileKeys = 512;
 // Width of each pass's digit for keys of `bits` bits: the fewest passes of at
 // most 8 bits, the bits spread evenly over them (the last may be narrower).
 int sort_digit_bits(int bits);
-// Optional gather fused into the last pass: posOut[i] = posIn[v], nrmOut[i] =
-// nrmIn[v] for the value v that lands at i.
+// Optional gather fused into the last pass: posOut[i] = posIn[v] and, where
+// nrmOut is given, nrmOut[i] = nrmIn[v] for the value v that lands at i.
 struct SortGather {
     const float4* posIn;
     const float4* nrmIn;

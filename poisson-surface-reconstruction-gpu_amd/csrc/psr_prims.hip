@@ -179,7 +179,7 @@ __device__ __forceinline__ void radix_scatter_body(int psr_bid, int psr_nbid, co
             vout[pos] = val;
             if (g.posOut) {
                 g.posOut[pos] = g.posIn[val];
-                g.nrmOut[pos] = g.nrmIn[val];
+                if (g.nrmOut) g.nrmOut[pos] = g.nrmIn[val];
             }
         }
         __syncthreads();
