@@ -226,6 +226,7 @@ struct Ctx {
     int cgMaxWgs = 0;            // resident workgroups of the CG kernels with several rows per thread
     int cgMaxWgsRow = 0;         // resident workgroups of the one-row-per-thread CG kernels
     int cgMaxWgsMinres = 0;      // resident workgroups of the MINRES kernel (indefinite depths, mixed form)
+    int cgMaxWgsChip[3] = {};    // resident workgroups of its on-chip forms (4, 8 and 16 rows a thread)
     int cgRowsPerWg = 0;         // rows per CG workgroup (0: default)
     int cgRowTarget = 0;         // batch: rows a CG workgroup takes (0: the single-cloud plan)
     int cgSpinLimit = -1;        // spin bound of the CG barriers (-1: the default)

@@ -47,7 +47,8 @@ constexpr int kCgWaves = kCgThreads / PSR_WAVE;
 // depth 9 than at 2), the mixed generic CG for 3.
 constexpr int kCgFp32GenericWaves = 4, kCgMixedGenericWaves = 3;
 // The MINRES kernel (indefinite depths of the mixed form) carries only its
-// own path and is compiled for 4 waves per SIMD.
+// own path and is compiled for 4 waves per SIMD.  Its occupancy (5) also sets
+// the row blocks of the on-chip form, whose sums follow them.
 constexpr int kCgMinresWaves = 4;
 // The mixed form's inner CG ends when its residual has not reached a new
 // minimum for this many iterations, and its solution goes back to the
@@ -1431,6 +1432,472 @@ __global__ void __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu
 PSR_BATCHABLE_WAVES(cg_mixed_minres, kCgThreads, kCgMinresWaves)
 
 
+
+// --- MINRES with the vectors on chip -----------------------------------------
+// The same solve as cg_mixed_minres, bit for bit (rows to threads, order of the
+// sums and of every operation), for a depth whose operator stores the diagonal
+// and the six faces: each of its workgroups keeps its rows' vectors where it
+// works on them.  Per sweep cg_mixed_minres moves about 100 bytes a row through
+// the caches and gathers 14 uncached values a row; here
+//   * x, the two directions w and y' stay in registers, R rows a thread;
+//   * y_{k-1} is formed once per row, in LDS, where all neighbours in the
+//     workgroup read it (95% of them: a workgroup's rows are a patch of the
+//     surface in Morton order), and once per neighbour outside it (a ghost: its
+//     owner's record {y_{k-2}, y'_{k-1}}, one 8-byte load);
+//   * the six columns of a row are 16-bit LDS places, the weights are one
+//     constant per slot (checked row by row);
+//   * only rows with a neighbour outside the workgroup write a record.
+// A workgroup whose rows do not fit this (other weights, more ghosts than
+// places) reads its neighbours' records instead, row by row, and stores all of
+// its own.  10000 iterations at depth 9: 2.76M rows (displaced sphere) 872 ms
+// with every vector in memory, 174 ms here (17 us a sweep: about 11 us of LDS
+// reads and arithmetic, the rest the reduction); 723k rows 285 -> 75 ms, 141k
+// rows 136 -> 63 ms (6 us a sweep, nearly all of it the reduction).
+//
+// Group reduction: every workgroup stores its block total (two stamped slots);
+// four collector workgroups each fold one wave's share of the totals, in
+// group_allreduce's order, and publish it in kResultCopies copies; every
+// workgroup merges the four.
+constexpr int kResultCopies = 16;
+constexpr int kCollectors = kCgWaves;  // a collector per wave of the fold
+constexpr int kFoldParts = 5;  // groups of at most kFoldParts * kCgThreads workgroups
+constexpr size_t minres_result_slots() { return size_t(2) * kResultCopies * kCollectors * 2; }  // of a group
+// Sum of the group's block totals `mine`, as group_allreduce folds them.  slots:
+// [2][G][2] block totals, then [2][kResultCopies][kCollectors][2] wave totals,
+// by phase parity, zero before the launch; a slot holds two words of payload and
+// the phase.  The block's stores of the sweep have completed (its waves waited
+// for them before the barrier that formed `mine`).
+__device__ __forceinline__ bool collect_comp2(const Comp2& mine, Comp2& out, float4* slots, int G, int local,
+                                              unsigned& phase, unsigned spinLimit, int* errFlag, Comp2* sh,
+                                              Comp2* part) {
+    __shared__ int shOk;
+    ++phase;
+    const float stamp = __uint_as_float(phase);
+    const int lane = __lane_id(), wave = threadIdx.x / PSR_WAVE;
+    const __amdgpu_buffer_rsrc_t in = vec_rsrc(slots + size_t(phase & 1u) * 2 * G, sizeof(float4) * 2 * size_t(G));
+    float4* results = slots + size_t(4) * G + size_t(phase & 1u) * kResultCopies * kCollectors * 2;
+    const __amdgpu_buffer_rsrc_t res = vec_rsrc(results, sizeof(float4) * kResultCopies * kCollectors * 2);
+    if (threadIdx.x < 2)
+        st_vec4(in, local * 2 + int(threadIdx.x),
+                threadIdx.x == 0 ? make_float4(mine.gs, mine.gc, stamp, 0.f) : make_float4(mine.ds, mine.dc, stamp, 0.f));
+    auto give_up = [&](unsigned spins) {
+        if (spins < spinLimit && ((spins & 63u) != 63u || !__hip_atomic_load(errFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+            return false;
+        __hip_atomic_store(errFlag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    };
+    for (int w = local; w < kCollectors; w += G) {
+        // thread (wave j, lane) reads the total of workgroup 64 w + lane + 256 j
+        // (and j + 4 beyond 1024 workgroups)
+        if (threadIdx.x == 0) shOk = 1;
+        __syncthreads();
+        for (int j = wave; j < kFoldParts; j += kCgWaves) {
+            const int k = PSR_WAVE * w + lane + kCgThreads * j;
+            Comp2 c{0.f, 0.f, 0.f, 0.f};
+            if (k < G) {
+                for (unsigned spins = 0;; ++spins) {
+                    const float4 a = ld_vec4(in, 2 * k), b = ld_vec4(in, 2 * k + 1);
+                    if (__float_as_uint(a.z) == phase && __float_as_uint(b.z) == phase) {
+                        c = Comp2{a.x, a.y, b.x, b.y};
+                        break;
+                    }
+                    if (give_up(spins)) {
+                        shOk = 0;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
+            part[j * PSR_WAVE + lane] = c;
+        }
+        __syncthreads();
+        if (shOk == 0) return false;
+        if (wave == 0) {
+            Comp2 t{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; PSR_WAVE * w + kCgThreads * j < G; ++j)
+                if (PSR_WAVE * w + lane + kCgThreads * j < G) comp2_merge(t, part[j * PSR_WAVE + lane]);
+            t = wave_comp2(t);
+            if (lane < 2 * kResultCopies)
+                st_vec4(res, ((lane >> 1) * kCollectors + w) * 2 + (lane & 1),
+                        (lane & 1) == 0 ? make_float4(t.gs, t.gc, stamp, 0.f) : make_float4(t.ds, t.dc, stamp, 0.f));
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        const int at = (local % kResultCopies) * kCollectors * 2 + lane;
+        bool ok = true;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (unsigned spins = 0;; ++spins) {
+            if (lane < 2 * kCollectors) v = ld_vec4(res, at);
+            if (__ballot(lane < 2 * kCollectors && __float_as_uint(v.z) != phase) == 0) break;
+            if (__ballot(give_up(spins)) != 0) {
+                ok = false;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (lane < 2 * kCollectors) {
+            float* d = (lane & 1) ? &sh[lane >> 1].ds : &sh[lane >> 1].gs;
+            d[0] = v.x;
+            d[1] = v.y;
+        }
+        if (lane == 0) shOk = ok ? 1 : 0;
+    }
+    __syncthreads();
+    out = sh[0];
+    for (int k = 1; k < kCollectors; ++k) comp2_merge(out, sh[k]);
+    const bool ok = shOk != 0;
+    __syncthreads();
+    return ok;
+}
+
+constexpr unsigned kFaceSlots = 1u << 4 | 1u << 10 | 1u << 12 | 1u << 13 | 1u << 14 | 1u << 16 | 1u << 22;
+// Ghost places of a workgroup: about 1000-1900 of 4096 rows' neighbours lie
+// outside it on the displaced sphere, 600-1200 of 2048 rows'.
+template <int R>
+constexpr int minres_ghosts() { return R == 16 ? 3072 : (R == 8 ? 2048 : 1536); }
+
+template <int R>
+__device__ __forceinline__ void cg_minres_chip(int psr_bid, const CgParams& P, const int* __restrict__ neigh,
+                                               const float* __restrict__ val, const float* __restrict__ b, float* x,
+                                               float* rOut, float2* rec, float* __restrict__ avScratch,
+                                               double* partialD, float4* slotsAll, GroupCtl* ctlAll,
+                                               int* __restrict__ iters, double* __restrict__ resid,
+                                               double* __restrict__ trueRel, int* errFlag,
+                                               const unsigned* __restrict__ slotMasks, const int* __restrict__ q1Fired) {
+    constexpr int kRows = R * kCgThreads, kGhosts = minres_ghosts<R>(), kZero = kRows + kGhosts;
+    static_assert(kGhosts % kCgThreads == 0, "whole rounds of ghosts");
+    static_assert(4 * kZero < 65536, "16-bit byte offsets");
+    static_assert(sizeof(Comp2) * PSR_WAVE * kFoldParts <= sizeof(float) * kGhosts, "the fold works in the ghosts' place");
+    __shared__ __align__(16) float ly[kRows + kGhosts + 1];  // y_{k-1} of the rows, of the ghosts, and a zero
+    __shared__ int lg[kGhosts];                // the ghosts' rows
+    __shared__ unsigned lw[7];
+    __shared__ int shGhosts, shSlow;
+    __shared__ double shd[kCgWaves];
+    __shared__ Comp2 shc[kCgWaves];
+    __shared__ int shFlag;
+    __shared__ double shResD;
+    int gi = 0;
+    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
+    const CgGroup G = P.g[gi];
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x);
+    const int r0 = G.rowBegin + local * G.rowsPerWg;
+    const int rows = max(0, min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0);  // at most kRows (host)
+    const int M = P.M;
+    double* partD = partialD + 2 * G.firstWg;
+    float4* slots = slotsAll + minres_result_slots() * gi + size_t(4) * G.firstWg;
+    GroupCtl* ctl = ctlAll + gi;
+    unsigned phase = 0, phaseC = 0;
+    const bool multi = G.wgs > 1;
+    const unsigned slotMask = slotMasks[G.depth];
+    auto sum_double = [&](double v, double& out) -> bool {
+        if (multi) __builtin_amdgcn_s_waitcnt(0);  // every wave's stores complete before the total
+        double s = block_sum_double(v, shd);
+        if (!multi) {
+            out = s;
+            return true;
+        }
+        return group_allreduce(s, out, partD, ctl, phase, G.wgs, local, P.spinLimit, errFlag, &shFlag, &shResD,
+                               [&](const double* parts, int n) { return fold_double(parts, n, shd); });
+    };
+
+    auto y_at = [&](unsigned byteOffset) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(ly) + byteOffset); };
+    // Row l's siblings lie at l ^ 4, l ^ 2 and l ^ 1 (x, y, z); the slots of its other three faces are the same for
+    // all rows of a thread (256 rows apart).  Those faces' columns as byte offsets into ly: x and y in one word, the
+    // z of two rows in another.
+    const bool bx = (t & 4) != 0, by = (t & 2) != 0, bz = (t & 1) != 0;
+    if (t < 7) lw[t] = 0u;
+    if (t == 0) shGhosts = 0, shSlow = slotMask != kFaceSlots ? 1 : 0, ly[kZero] = 0.f;
+    __syncthreads();
+    unsigned placeXY[R], placeZ[(R + 1) / 2];
+    unsigned boundary = 0u;  // bit k: row k has a neighbour outside the workgroup, and so a reader there
+    {
+        const int slotOf[7] = {bx ? 22 : 4, by ? 16 : 10, bz ? 14 : 12, bx ? 4 : 22, by ? 10 : 16, bz ? 12 : 14, 13};
+        float w[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        unsigned bad = 0u;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int l = k * kCgThreads + t, i = r0 + max(0, min(l, rows - 1));
+            const bool own = l < rows;
+            unsigned at[3];
+#pragma unroll
+            for (int q = 0; q < 7; ++q) {
+                const size_t e = size_t(slotOf[q]) * M + i;
+                const float v = val[e];
+                const int j = neigh[e];
+                bad |= own && v != 0.f && w[q] != 0.f && w[q] != v ? 1u : 0u;
+                if (own && v != 0.f) w[q] = v;
+                if (q >= 3) {  // a sibling or the row itself
+                    const int flip = q == 3 ? 4 : (q == 4 ? 2 : (q == 5 ? 1 : 0));
+                    bad |= own && (v == 0.f || j != r0 + (l ^ flip) || (l ^ flip) >= rows) ? 1u : 0u;
+                    continue;
+                }
+                const bool outside = own && j >= 0 && unsigned(j - r0) >= unsigned(rows);
+                if (outside) boundary |= 1u << k;
+                const bool stored = own && v != 0.f;
+                int p = stored ? j - r0 : kZero;
+                if (stored && outside) {
+                    const int h = atomicAdd(&shGhosts, 1);
+                    p = kRows + min(h, kGhosts - 1);
+                    if (h < kGhosts) lg[h] = j;
+                }
+                bad |= stored && j < 0 ? 1u : 0u;
+                at[q] = unsigned(4 * p) & 0xffffu;
+            }
+            placeXY[k] = at[0] | at[1] << 16;
+            placeZ[k / 2] = k % 2 == 0 ? at[2] : placeZ[k / 2] | at[2] << 16;
+            // packed here and now: the rows' state fills the registers
+            asm volatile("" : "+v"(placeXY[k]), "+v"(placeZ[k / 2]), "+v"(boundary), "+v"(bad) : : "memory");
+#pragma unroll
+            for (int q = 0; q < 7; ++q) asm volatile("" : "+v"(w[q]));
+        }
+        const int wordOf[7] = {bx ? 5 : 0, by ? 4 : 1, bz ? 3 : 2, bx ? 0 : 5, by ? 1 : 4, bz ? 2 : 3, 6};
+#pragma unroll
+        for (int q = 0; q < 7; ++q)
+            if (w[q] != 0.f) atomicMax(&lw[wordOf[q]], __float_as_uint(w[q]));
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 7; ++q)
+            if (w[q] != 0.f && __float_as_uint(w[q]) != lw[wordOf[q]]) bad = 1u;
+        if (bad) shSlow = 1;
+        __syncthreads();
+    }
+    const int ghosts = __builtin_amdgcn_readfirstlane(shGhosts);
+    const bool slow = __builtin_amdgcn_readfirstlane(shSlow) != 0 || ghosts > kGhosts;
+    // neighbour tables that the level-local child 0 rule changed need not be symmetric
+    if (slow || *q1Fired != 0) {
+        boundary = 0u;
+        for (int k = 0; k < R; ++k) boundary |= k * kCgThreads + t < rows ? 1u << k : 0u;
+    }
+    float wq[7];
+#pragma unroll
+    for (int q = 0; q < 7; ++q) wq[q] = __uint_as_float(__builtin_amdgcn_readfirstlane(lw[q]));
+
+    // x = 0; ||b||^2 in FP64 (the outer residual of x = 0 is b itself)
+    float xr[R];
+    double loc = 0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) xr[k] = 0.f;
+#pragma unroll 1
+    for (int l = t; l < rows; l += kCgThreads) {
+        const int i = r0 + l;
+        {
+            st_shared(&x[i], 0.f);
+            const double bi = b[i];
+            loc += bi * bi;
+        }
+    }
+    double bb;
+    if (!sum_double(loc, bb)) return;
+    double rr = bb, rel = bb > 0 ? 1.0 : 0.0;
+    const float* rhs = b;
+    int total = 0, outer = 0;
+    float gamma = 0.f;
+    while (rel > P.relTol && outer < P.maxOuter && total < P.maxIter) {
+        const double tgt = fmax(0.5 * P.relTol * sqrt(bb), 1e-6 * sqrt(rr));
+        const float beta1 = float(sqrt(rr));
+        const float tgtf = float(tgt);
+        float beta = beta1, oldb = 1.f, cPrev = 0.f;
+        float cs = -1.f, sn = 0.f, dbar = 0.f, epsln = 0.f, phibar = beta1;
+        float lagEps = 0.f, lagDelta = 0.f, lagGamma = 1.f, lagPhi = 0.f;
+        int it = 1, kdone = 0;
+        // y_{-1} = 0 and y'_0 = rhs make the first sweep one like the others
+        float yp[R], w1[R], w2[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            int l = k * kCgThreads + t;
+            asm volatile("" : "+v"(l));  // no address is kept from loop to loop
+            const int i = r0 + l;
+            yp[k] = l < rows ? ld_shared(&rhs[i]) : 0.f;
+            w1[k] = w2[k] = 0.f;
+            ly[l] = 0.f;
+            if (l < rows) st_vec2(vec_rsrc(rec, sizeof(float2) * size_t(M)), i, make_float2(0.f, yp[k]));
+        }
+        double fence;
+        if (!sum_double(0.0, fence)) return;  // the records are read by other workgroups
+        while (beta1 > tgtf && total < P.maxIter) {
+            // record buffer (it + 1) & 1 holds {y_{it-2}, y'_{it-1}}, it & 1 receives {y_{it-1}, y'_it}
+            const __amdgpu_buffer_rsrc_t in = vec_rsrc(rec + size_t((it + 1) & 1) * M, sizeof(float2) * size_t(M));
+            const __amdgpu_buffer_rsrc_t onto = vec_rsrc(rec + size_t(it & 1) * M, sizeof(float2) * size_t(M));
+            const float invB = 1.f / beta;
+            const float r1c = it >= 2 ? beta / oldb : 0.f;
+            const float invOld = 1.f / oldb;
+            // the rows' offsets and bounds are formed anew every sweep, not kept
+            int tt = t, base = r0 + t;
+            unsigned bnd = boundary;
+            asm volatile("" : "+v"(tt), "+v"(base), "+v"(bnd));
+            // the ghosts' records are on their way while the rows' y are formed
+            constexpr int kEarly = 6;
+            float2 g[kEarly];
+            if (!slow) {
+#pragma unroll
+                for (int m = 0; m < kEarly; ++m) {
+                    const int h = m * kCgThreads + tt;
+                    g[m] = h < ghosts ? ld_vec2(in, lg[h]) : make_float2(0.f, 0.f);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const int l = k * kCgThreads + t;
+                const float r1 = ly[l];  // y_{it-2}
+                // the previous iteration's direction and update (zero in the first sweep)
+                const float num = __fmaf_rn(-lagDelta, w2[k], __fmaf_rn(r1, invOld, -__fmul_rn(lagEps, w1[k])));
+                const float wk = num / lagGamma;
+                xr[k] = __fmaf_rn(lagPhi, wk, xr[k]);
+                w1[k] = w2[k];
+                w2[k] = wk;
+                ly[l] = __fmaf_rn(-cPrev, r1, yp[k]);
+                yp[k] = r1;
+                // the state stays in its registers from sweep to sweep
+                asm volatile("" : "+v"(xr[k]), "+v"(w1[k]), "+v"(w2[k]), "+v"(yp[k]));
+            }
+            if (!slow) {
+#pragma unroll
+                for (int m = 0; m < kEarly; ++m) {
+                    const int h = m * kCgThreads + tt;
+                    if (h < ghosts) ly[kRows + h] = __fmaf_rn(-cPrev, g[m].x, g[m].y);
+                }
+                for (int h = kEarly * kCgThreads + tt; h < ghosts; h += kCgThreads) {
+                    const float2 n = ld_vec2(in, lg[h]);
+                    ly[kRows + h] = __fmaf_rn(-cPrev, n.x, n.y);
+                }
+            } else {
+                for (int i = r0 + t; i < r0 + rows; i += kCgThreads) {
+                    float av = 0.f;
+#pragma unroll 1
+                    for (int q = 0; q < 27; ++q) {
+                        const float v = val[size_t(q) * M + i];
+                        if (v == 0.f) continue;  // a term of weight zero adds nothing
+                        const float2 n = ld_vec2(in, neigh[size_t(q) * M + i]);
+                        av = __fmaf_rn(v, __fmaf_rn(-cPrev, n.x, n.y), av);
+                    }
+                    avScratch[i] = av;
+                }
+            }
+            __syncthreads();
+            Comp2 dl{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                const int l = k * kCgThreads + t;
+                const float yi = ly[l];
+                // unpacked anew every sweep: 3 R addresses do not fit the registers
+                unsigned pxy = placeXY[k], pz = placeZ[k / 2];
+                asm volatile("" : "+v"(pxy), "+v"(pz));
+                const float xe = y_at(pxy & 0xffffu), ye = y_at(pxy >> 16), ze = y_at(k % 2 == 0 ? pz & 0xffffu : pz >> 16);
+                const float xs = ly[k * kCgThreads + (tt ^ 4)], ys = ly[k * kCgThreads + (tt ^ 2)],
+                            zs = ly[k * kCgThreads + (tt ^ 1)];
+                float av = __fmaf_rn(wq[0], bx ? xs : xe, 0.f);
+                av = __fmaf_rn(wq[1], by ? ys : ye, av);
+                av = __fmaf_rn(wq[2], bz ? zs : ze, av);
+                av = __fmaf_rn(wq[6], yi, av);
+                av = __fmaf_rn(wq[3], bz ? ze : zs, av);
+                av = __fmaf_rn(wq[4], by ? ye : ys, av);
+                av = __fmaf_rn(wq[5], bx ? xe : xs, av);
+                if (slow) av = rows - tt > k * kCgThreads ? avScratch[base + k * kCgThreads] : 0.f;
+                // rows past the workgroup's last are zero throughout and add nothing to the sums
+                yp[k] = __fmaf_rn(-r1c, yp[k], __fmul_rn(av, invB));
+                dot2_acc(dl.gs, dl.gc, __fmul_rn(yi, invB), yp[k]);
+                dot2_acc(dl.ds, dl.dc, yp[k], yp[k]);
+                if (bnd >> k & 1u) st_vec2(onto, base + k * kCgThreads, make_float2(yi, yp[k]));
+                asm volatile("" : "+v"(yp[k]), "+v"(dl.gs), "+v"(dl.gc), "+v"(dl.ds), "+v"(dl.dc));
+            }
+            dl = wave_comp2(dl);
+            __builtin_amdgcn_s_waitcnt(0);  // the records have left before the total does
+            if (__lane_id() == 0) shc[t / PSR_WAVE] = dl;
+            __syncthreads();
+            Comp2 gsum = shc[0];
+            for (int k = 1; k < kCgWaves; ++k) comp2_merge(gsum, shc[k]);
+            __syncthreads();
+            if (multi && !collect_comp2(gsum, gsum, slots, G.wgs, local, phaseC, P.spinLimit, errFlag, shc,
+                                        reinterpret_cast<Comp2*>(ly + kRows)))
+                return;
+            const float alfa = gsum.gs + gsum.gc, yy = gsum.ds + gsum.dc;
+            // one scalar per workgroup: kept in scalar registers between the sweeps
+            auto uni = [](float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); };
+            const float betaN = sqrtf(fmaxf(__fmaf_rn(-alfa, alfa, yy), 0.f));
+            const float oldeps = epsln;
+            const float delta = __fmaf_rn(cs, dbar, __fmul_rn(sn, alfa));
+            const float gbar = __fmaf_rn(dbar, sn, -__fmul_rn(cs, alfa));
+            epsln = uni(sn * betaN);
+            dbar = uni(-cs * betaN);
+            const float gam = fmaxf(sqrtf(__fmaf_rn(gbar, gbar, __fmul_rn(betaN, betaN))), 1e-30f);
+            cs = uni(gbar / gam);
+            sn = uni(betaN / gam);
+            const float phi = cs * phibar;
+            phibar = uni(sn * phibar);
+            lagEps = uni(oldeps);
+            lagDelta = uni(delta);
+            lagGamma = uni(gam);
+            lagPhi = uni(phi);
+            cPrev = uni(alfa / beta);
+            oldb = beta;
+            beta = uni(betaN);
+            ++kdone;
+            gamma = phibar * phibar;
+            if (!(phibar > tgtf) || total + kdone >= P.maxIter || !(betaN > 0.f)) break;
+            ++it;
+        }
+        if (kdone > 0) {
+            // the last iteration's update: v = y_{it-1} / beta_it
+            const float invOld = 1.f / oldb;
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+                int l = k * kCgThreads + t;
+                asm volatile("" : "+v"(l));
+                const float num = __fmaf_rn(-lagDelta, w2[k], __fmaf_rn(ly[l], invOld, -__fmul_rn(lagEps, w1[k])));
+                xr[k] = __fmaf_rn(lagPhi, num / lagGamma, xr[k]);
+                if (l < rows) st_shared(&x[r0 + l], xr[k]);
+            }
+        }
+        total += kdone;
+        ++outer;
+        if (kdone == 0) break;
+        // orders x before the outer residual reads neighbours' x
+        if (!sum_double(0.0, fence)) return;
+        // outer residual in FP64
+        loc = 0;
+        for (int i = r0 + t; i < r0 + rows; i += kCgThreads) {
+            double acc = b[i];
+#pragma unroll 1
+            for (int q = 0; q < 27; ++q) {
+                const float v = val[size_t(q) * M + i];
+                if (v != 0.f) acc -= double(v) * double(ld_shared(&x[neigh[size_t(q) * M + i]]));  // the product is exact
+            }
+            st_shared(&rOut[i], float(acc));
+            loc += acc * acc;
+        }
+        if (!sum_double(loc, rr)) return;
+        rel = bb > 0 ? sqrt(rr / bb) : 0.0;
+        rhs = rOut;
+    }
+    if (local == 0 && t == 0) {
+        iters[G.depth] = total;
+        iters[PSR_MAX_DEPTH + 1 + G.depth] = outer;
+        resid[G.depth] = sqrt(double(gamma));
+        trueRel[G.depth] = rel;
+    }
+}
+// R rows a thread at most, and the waves per SIMD its registers allow (with
+// the launch's residency): 16 rows and 3 waves hold 3.1M rows, 8 rows and 5
+// waves all depths of workgroups of 2048 rows or fewer.
+#define PSR_MINRES_CHIP(NAME, R, WAVES)                                                                                 \
+    template <class... A>                                                                                               \
+    __device__ __forceinline__ void NAME##_body(int bid, int, const A&... a) {                                          \
+        cg_minres_chip<R>(bid, a...);                                                                                   \
+    }                                                                                                                   \
+    __global__ void __launch_bounds__(kCgThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) NAME(                     \
+        CgParams P, const int* __restrict__ neigh, const float* __restrict__ val, const float* __restrict__ b,          \
+        float* x, float* rOut, float2* rec, float* __restrict__ avScratch, double* partialD, float4* slots,             \
+        GroupCtl* ctlAll, int* __restrict__ iters, double* __restrict__ resid, double* __restrict__ trueRel,            \
+        int* errFlag, const unsigned* __restrict__ slotMasks, const int* __restrict__ q1Fired) {                        \
+        cg_minres_chip<R>(blockIdx.x, P, neigh, val, b, x, rOut, rec, avScratch, partialD, slots, ctlAll, iters, resid, \
+                          trueRel, errFlag, slotMasks, q1Fired);                                                        \
+    }                                                                                                                   \
+    PSR_BATCHABLE_WAVES(NAME, kCgThreads, WAVES)
+PSR_MINRES_CHIP(cg_minres_chip16, 16, 3)
+PSR_MINRES_CHIP(cg_minres_chip8, 8, 5)
+PSR_MINRES_CHIP(cg_minres_chip4, 4, 5)
+
 // --- implicit function at points (LaplacianSolver.cu:85-118, 269-305) ------
 // Neighbour columns: d_x of neighbour i of every node, and, when the
 // level-local child 0 rule changed a parent, its basis parameters as well, so
@@ -1599,6 +2066,12 @@ void solve_depths(Ctx& c) {
         c.cgMaxWgsRow = std::max(0, perRow * cus);
         c.cgMaxWgs = std::max(1, perGen * cus);
         c.cgMaxWgsMinres = std::max(1, perMinres * cus);
+        c.cgMaxWgsChip[0] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip4),
+                                            multi_queue_kernel_of<cg_minres_chip4_k>(cg_minres_chip4));
+        c.cgMaxWgsChip[1] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip8),
+                                            multi_queue_kernel_of<cg_minres_chip8_k>(cg_minres_chip8));
+        c.cgMaxWgsChip[2] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip16),
+                                            multi_queue_kernel_of<cg_minres_chip16_k>(cg_minres_chip16));
     }
     // the mixed form solves indefinite depths with MINRES, in a launch of its
     // own (the MINRES kernel) after the CG launch of the other depths
@@ -1656,7 +2129,19 @@ void solve_depths(Ctx& c) {
         g.indef = isMinres[d] ? 1 : 0;
         w += g.wgs;
     }
-    if (wg > (rowForm ? c.cgMaxWgsRow : c.cgMaxWgs) || wgM > c.cgMaxWgsMinres)
+    // The MINRES launch keeps its vectors on chip when its row blocks fit the
+    // rows a thread holds and all its workgroups are resident in that form: up
+    // to 3.1M rows here.  The row blocks, and so the sums, are the same either
+    // way.
+    int chip = -1;
+    if (PM.ngroups > 0) {
+        int widest = 0;
+        for (int k = 0; k < PM.ngroups; ++k) widest = std::max(widest, PM.g[k].rowsPerWg);
+        const int want = widest <= 4 * kCgThreads ? 0 : (widest <= 8 * kCgThreads ? 1 : 2);
+        if (widest <= 16 * kCgThreads && wgM <= c.cgMaxWgsChip[want] && wgM <= kFoldParts * kCgThreads) chip = want;
+    }
+    const int capMinres = chip >= 0 ? c.cgMaxWgsChip[chip] : c.cgMaxWgsMinres;
+    if (wg > (rowForm ? c.cgMaxWgsRow : c.cgMaxWgs) || wgM > capMinres)
         throw std::runtime_error("CG launch exceeds the resident workgroup budget");
     c.stats.cg_workgroups = uint32_t(wg + wgM);
     double* partial = c.buf<double>("cg_partial", size_t(2) * (wg + wgM));
@@ -1666,13 +2151,16 @@ void solve_depths(Ctx& c) {
     double* resid = res->cgResid;
     double* trueRel = res->cgTrueRel;
     int* err = &res->cgErr;
-    float4* slots = rowForm && mixed ? c.buf<float4>("cg_slots", size_t(4) * wg) : nullptr;
+    // slots of the row form's groups, or of the on-chip MINRES's
+    const size_t slotCount = rowForm && mixed ? size_t(4) * wg
+                                              : (chip >= 0 ? size_t(4) * wgM + PM.ngroups * minres_result_slots() : 0);
+    float4* slots = slotCount ? c.buf<float4>("cg_slots", slotCount) : nullptr;
     // The group controls and slots start at zero: the neighbour-column kernel
     // clears them after every solve, so they need a launch of their own only
     // when the last call on this context did not complete or the slots moved.
     // The CG writes every depth's results itself; its error flag is cleared
     // with the operator counts (by the vector-field kernel).
-    const size_t slotWords = slots ? size_t(16) * wg : 0;
+    const size_t slotWords = 4 * slotCount;
     if (!c.cgClean || slots != c.cgSlots || slotWords != c.cgSlotWords)
         zero_spans({{ctl, size_t(ctlWords)}, {slots, slotWords}}, s);
     c.cgClean = false;
@@ -1688,8 +2176,7 @@ void solve_depths(Ctx& c) {
     // the two launches of a split solve run one after the other on the stream:
     // the account holds the larger
     const long long cap = rowForm ? c.cgMaxWgsRow : c.cgMaxWgs;
-    const long long units = std::max((wg * kCgUnits + cap - 1) / cap,
-                                     (wgM * kCgUnits + c.cgMaxWgsMinres - 1) / c.cgMaxWgsMinres);
+    const long long units = std::max((wg * kCgUnits + cap - 1) / cap, (wgM * kCgUnits + capMinres - 1) / capMinres);
     // While a batch records, the batch merges every cloud's solve into launches
     // that fit the resident budget and accounts for them itself.
     const bool recording = current_recorder() != nullptr;
@@ -1713,8 +2200,10 @@ void solve_depths(Ctx& c) {
         PSR_HIP_CHECK(hipEventRecord(c.ev[8], s));
     }
     if (rowForm && mixed) P.spinLimit = 1u << 22;
+    if (chip >= 0) PM.spinLimit = 1u << 24;  // polls of about a microsecond; a batch's group may wait for the solves before it
     if (c.cgSpinLimit >= 0) P.spinLimit = PM.spinLimit = unsigned(c.cgSpinLimit);
     static const char siteMixedRow = 0, siteMixedGen = 0, siteMinres = 0, siteRow = 0, siteGen = 0;
+    static const char siteChip[3] = {0, 0, 0};
     if (mixed) {
         P.relTol = PM.relTol = c.cfg.refine_rel_tol;
         P.maxOuter = PM.maxOuter = std::max(1, c.cfg.refine_max_outer);
@@ -1725,7 +2214,8 @@ void solve_depths(Ctx& c) {
             launch_kernel<cg_mixed_row_k>(&siteMixedRow, cg_mixed_row, wg, 0, s, true, P, o.neigh, val, c.fld.div,
                                           c.fld.dx, rOut, state, slots, iters, resid, trueRel, err);
         } else {
-            float* rbuf = c.buf<float>("cg_rbuf", size_t(2) * M);
+            // also the on-chip MINRES's two buffers of records
+            float* rbuf = c.buf<float>("cg_rbuf", size_t(chip >= 0 ? 4 : 2) * M);
             float* wbuf = c.buf<float>("cg_wbuf", size_t(2) * M);
             float* sbuf = c.buf<float>("cg_sbuf", size_t(2) * M);
             float* pvec = c.buf<float>("cg_pa", M);
@@ -1734,7 +2224,15 @@ void solve_depths(Ctx& c) {
                                                      val, c.fld.div, c.fld.dx, rOut, rbuf, wbuf, sbuf, pvec, partial,
                                                      partialC, ctl, iters, resid, trueRel, err, res->cgSlotMask);
             // the MINRES launch uses the group controls and partials after the CG launch's
-            if (PM.ngroups > 0)
+            auto launch_chip = [&](auto k, auto kernel, const char* site) {
+                launch_kernel<decltype(k)>(site, kernel, wgM, 0, s, true, PM, o.neigh, val, c.fld.div, c.fld.dx, rOut,
+                                           reinterpret_cast<float2*>(rbuf), sbuf, partial + size_t(2) * wg, slots,
+                                           ctl + P.ngroups, iters, resid, trueRel, err, res->cgSlotMask, o.q1Fired);
+            };
+            if (chip == 0) launch_chip(cg_minres_chip4_k{}, cg_minres_chip4, &siteChip[0]);
+            else if (chip == 1) launch_chip(cg_minres_chip8_k{}, cg_minres_chip8, &siteChip[1]);
+            else if (chip == 2) launch_chip(cg_minres_chip16_k{}, cg_minres_chip16, &siteChip[2]);
+            else if (PM.ngroups > 0)
                 launch_kernel<cg_mixed_minres_k>(&siteMinres, cg_mixed_minres, wgM, 0, s, true, PM, o.neigh, val,
                                                  c.fld.div, c.fld.dx, rOut, rbuf, wbuf, sbuf, pvec,
                                                  partial + size_t(2) * wg, partialC + size_t(2) * wg,
