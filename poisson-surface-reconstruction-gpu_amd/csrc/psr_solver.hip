@@ -7,6 +7,7 @@
 #include <chrono>
 #include <stdexcept>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 namespace psr {
@@ -237,17 +238,6 @@ __device__ __forceinline__ void st_vec2(__amdgpu_buffer_rsrc_t r, int idx, float
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r,
                                           idx * 8, 0, kCoherent);
 }
-__device__ __forceinline__ float3 ld_vec3(__amdgpu_buffer_rsrc_t r, int idx) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b96(r, idx * 12, 0, kCoherent);
-    return make_float3(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]));
-}
-__device__ __forceinline__ void st_vec3(__amdgpu_buffer_rsrc_t r, int idx, float3 v) {
-    __attribute__((ext_vector_type(3))) unsigned u;
-    u[0] = __float_as_uint(v.x);
-    u[1] = __float_as_uint(v.y);
-    u[2] = __float_as_uint(v.z);
-    __builtin_amdgcn_raw_buffer_store_b96(u, r, idx * 12, 0, kCoherent);
-}
 __device__ __forceinline__ float4 ld_vec4(__amdgpu_buffer_rsrc_t r, int idx) {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, idx * 16, 0, kCoherent));
 }
@@ -256,223 +246,501 @@ __device__ __forceinline__ void st_vec4(__amdgpu_buffer_rsrc_t r, int idx, float
                                            idx * 16, 0, kCoherent);
 }
 
-// Atomic-free group all-reduce of the mixed one-row kernel (measured faster
-// there than the arrival counter of group_allreduce; the FP32 kernel, with two
-// reductions and little work between them, is faster with the counter).  Each
-// workgroup stores its block total in its own 16-byte slot(s) of the group's
-// region, stamped with the phase (one store per slot, so a reader sees a slot
-// whole); every
-// workgroup polls the group's slots until all carry the phase and then folds
-// them in the same fixed order, so every workgroup holds the same bits.  Slots
-// are double-buffered by phase parity (a workgroup runs at most one phase
-// ahead of the slowest) and zeroed before the launch (phases start at 1).
-// S: slots per workgroup (two payload words each); thread t polls the slots
-// of workgroups t and t + kCgThreads.
-constexpr int kPollPerThread = 2;  // groups of up to kPollPerThread * kCgThreads workgroups
-// Every workgroup owns kSlotStride slots per parity whatever S an exchange
-// uses: the layout of a phase never overlaps that of the other parity, so a
-// workgroup that has passed phase p and writes phase p + 1 cannot overwrite
-// a phase-p slot that a slower workgroup has yet to read.  (With a stride of
-// S, an S = 2 exchange right after an S = 1 one wrote into the S = 1 region
-// of the other parity, and a slow reader could wait for a stamp that was
-// already gone.)
-constexpr int kSlotStride = 2;
-template <int S>
-__device__ __forceinline__ bool slot_exchange(float4* region, int G, int local, unsigned& phase,
-                                              const unsigned (&mine)[2 * S], float4 (&got)[kPollPerThread][S],
-                                              unsigned spinLimit, int* errFlag) {
-    static_assert(S <= kSlotStride, "slots per workgroup");
-    ++phase;
-    const __amdgpu_buffer_rsrc_t rs =
-        vec_rsrc(region + size_t(phase & 1u) * G * kSlotStride, sizeof(float4) * size_t(G) * kSlotStride);
-    const float stamp = __uint_as_float(phase);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int h = 0; h < S; ++h)
-            st_vec4(rs, local * kSlotStride + h,
-                    make_float4(__uint_as_float(mine[2 * h]), __uint_as_float(mine[2 * h + 1]), stamp, 0.f));
-    }
-    for (unsigned spins = 0;; ++spins) {
-        int ok = 1;
-#pragma unroll
-        for (int j = 0; j < kPollPerThread; ++j) {
-            const int k = int(threadIdx.x) + j * kCgThreads;
-            if (k < G) {
-#pragma unroll
-                for (int h = 0; h < S; ++h) {
-                    got[j][h] = ld_vec4(rs, k * kSlotStride + h);
-                    ok &= __float_as_uint(got[j][h].z) == phase ? 1 : 0;
-                }
-            }
-        }
-        if (__syncthreads_and(ok)) return true;
-        if (spins >= spinLimit) {
-            if (threadIdx.x == 0) __hip_atomic_store(errFlag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-        if ((spins & 63u) == 63u) {
-            const int e =
-                threadIdx.x == 0 ? __hip_atomic_load(errFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-            if (__syncthreads_or(e)) return false;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
-}
+// --- one row per thread -------------------------------------------------------
+// Both forms' kernels for depths whose rows all have a thread (to about 390k
+// rows in all): a workgroup takes kRowThreads rows, the row's vectors stay in
+// registers, and what its neighbours read of it (p, or the next residual) is
+// formed once, in LDS.  A workgroup's rows are a patch of the surface (Morton
+// order), so 87% of their stored entries lie inside it; each row outside that
+// some entry names (a ghost: about half as many as rows) is read once per
+// sweep, as one record, and its value formed beside the own rows'.  The
+// weights are one constant per slot (the operator depends on the offset only;
+// checked row by row), held in scalar registers; a row's columns are 26 16-bit
+// places in LDS.  Only rows with a neighbour outside write records.
+// Where the level-local child 0 rule changed the neighbour tables the weights
+// may differ from row to row: such a workgroup reads each row's own, and what
+// has no place from memory (the slow form of the product).
+// Bound by the reductions' memory round trips (about 2 us each) and the
+// ghosts' (1 us).  Whole solves with 256 rows a workgroup, the stencil per row
+// and a record gathered per entry, and here: torus at depth 7 (71k rows) 146 ->
+// 107 us mixed, 582 -> 293 us FP32 (whose two sums per iteration went through
+// an arrival counter); ellipsoid at depth 8 (263k rows, several rows a thread
+// before) 638 -> 195 us and 1398 -> 458 us; sphere at depth 5 (7k rows) 327 ->
+// 209 us FP32.  Of these row_maps takes 13-30 us.
+constexpr int kRowThreads = 512, kRowWaves = kRowThreads / PSR_WAVE;
+// The sums' blocks: 256 rows, whatever the workgroup holds, so that they do not
+// depend on it.
+constexpr int kRowBlock = 256, kRowBlockWaves = kRowBlock / PSR_WAVE, kRowBlocks = kRowThreads / kRowBlock;
+constexpr int kRowMaxBlocks = 4 * kRowThreads;  // blocks of a group
+constexpr int kSlotStride = 2;                  // slots of a block and parity, whatever a sum uses
+constexpr int kGhostTable = 2048, kGhostMax = kRowThreads * 2;
+// Places are byte offsets into RowShared::v, two to a word; the top bit of the
+// last word marks a boundary row.
+constexpr int kPlaceGhosts = 4 * kRowThreads, kPlaceZero = 4 * (kRowThreads + kGhostMax), kPlaceMemory = 0x7ffc;
+static_assert(kPlaceZero < kPlaceMemory, "place range");
+constexpr unsigned kBoundaryBit = 1u << 31;
+// Waves per SIMD: four workgroups a CU (524k rows resident) in the FP32 form,
+// three (393k rows) in the mixed form, whose state is larger.
+constexpr int kRowFp32Waves = 8, kRowMixedWaves = 6;
 
-// Sum of the group's block totals (v: this workgroup's, the same in every
-// thread), folded as fold_double folds.
-__device__ __forceinline__ bool slot_sum_double(double v, double& out, float4* region, int G, int local,
-                                                unsigned& phase, unsigned spinLimit, int* errFlag, double* sh) {
-    const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
-    const unsigned mine[2] = {unsigned(u), unsigned(u >> 32)};
-    float4 got[kPollPerThread][1];
-    if (!slot_exchange<1>(region, G, local, phase, mine, got, spinLimit, errFlag)) return false;
-    double t = 0;
-#pragma unroll
-    for (int j = 0; j < kPollPerThread; ++j)
-        if (int(threadIdx.x) + j * kCgThreads < G)
-            t += __hiloint2double(__float_as_int(got[j][0].y), __float_as_int(got[j][0].x));
-    out = block_sum_double(t, sh);
-    return true;
-}
-
-// A row's 27 stencil entries, held in registers for the whole solve; a
-// dropped or missing entry reads the row itself with weight 0.
-struct Stencil {
-    float v[27];
-    int j[27];
-    __device__ __forceinline__ void load(const float* __restrict__ val, const int* __restrict__ neigh, int M, int i) {
-#pragma unroll
-        for (int q = 0; q < 27; ++q) {
-            v[q] = val[q * M + i];
-            const int c = neigh[q * M + i];
-            j[q] = (v[q] != 0.f) ? c : i;
-        }
-    }
+// What row_maps leaves for a workgroup of the row form (its ghosts' rows in a
+// list of kGhostMax, its rows' places in a table [13][M]).
+struct RowHead {
+    int ghosts;
+    int slow;     // weights per row, or neighbours without a place
+    float w[27];  // the slots' weights
+    int pad[3];
+};
+struct RowMapArgs {
+    const int* neigh;
+    const float* val;
+    const int* q1Fired;
+    unsigned* places;
+    int* ghosts;
+    RowHead* heads;
 };
 
-// The reference's CG (CGAlgorithm.cu:10-80), one launch for all depths, one
-// row per thread.  Per iteration k the record of row i in buffer k & 1 holds
-// {r_k, p_{k-1}}; a row forms its neighbours' p_k = r_k + beta p_{k-1} on the
-// fly, so the update of p and the product A p need no barrier in between
-// (CGAlgorithm.cu:37-53).  The row's stencil, x, r, p and A p stay in
-// registers; one 8-byte record per neighbour is read and one written per
-// iteration.
-__device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, const CgParams& P, const int* __restrict__ neigh,
-                                                          const float* __restrict__ val, const float* __restrict__ b,
-                                                          float* __restrict__ x, float2* state, double* partial,
-                                                          GroupCtl* ctlAll, int* __restrict__ iters,
-                                                          double* __restrict__ resid, int* errFlag) {
-    __shared__ double sh[kCgWaves];
-    __shared__ int shFlag;
-    __shared__ double shRes;
+// The maps of the row form's workgroups, a workgroup each (a launch of its own:
+// inside the CG kernel the table costs registers that its sweeps then lack).
+// Every stored neighbour inside the workgroup gets its row's place.  Those
+// outside (13% of the entries) are listed, shared out over the threads and
+// entered into a hash table, whose used positions are numbered and become the
+// ghosts' places.
+__device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& a) {
+    __shared__ unsigned short place[26][kRowThreads];       // kGhostMark | table position until the ghosts are numbered
+    __shared__ unsigned short list[26 * kRowThreads];       // entries outside: row << 5 | slot
+    __shared__ int key[kGhostTable];                        // ghost rows by hash, -1: free
+    __shared__ unsigned short number[kGhostTable];
+    __shared__ unsigned weight[27];
+    __shared__ int entries, ghosts, slow;
+    constexpr unsigned kGhostMark = 0x8000u;
+    static_assert(kRowThreads == 512, "nine bits of row, five of slot");
+    int gi = 0;
+    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
+    const CgGroup& G = P.g[gi];
+    const int t = int(threadIdx.x), M = P.M;
+    const int r0 = G.rowBegin + (psr_bid - G.firstWg) * G.rowsPerWg;
+    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0;
+    const bool own = t < rows;
+    const int i = r0 + min(t, rows - 1);
+    float v[27];
+    int j[27];
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {
+        v[q] = a.val[size_t(q) * M + i];
+        j[q] = a.neigh[size_t(q) * M + i];
+    }
+    for (int k = t; k < kGhostTable; k += kRowThreads) key[k] = -1;
+    if (t < 27) weight[t] = 0u;
+    if (t == 0) entries = 0, ghosts = 0, slow = 0;
+    __syncthreads();
+    unsigned bad = 0u, outside = 0u, ghost = 0u;  // ghost: slots with a stored neighbour outside
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {
+        const int l = j[q] - r0;
+        const bool inside = unsigned(l) < unsigned(rows), stored = own && v[q] != 0.f;
+        if (stored) weight[q] = __float_as_uint(v[q]);  // any row's
+        if (q == 13) {
+            if (own && (!stored || l != t)) bad = 1u;
+            continue;
+        }
+        const bool away = own && j[q] >= 0 && !inside;
+        if (away) outside = 1u;
+        if (away && stored) ghost |= 1u << q;
+        if (stored && j[q] < 0) bad = 1u;
+        place[q < 13 ? q : q - 1][t] =
+            static_cast<unsigned short>(!stored ? kPlaceZero : (inside ? 4 * l : kPlaceMemory));
+    }
+    // the entries outside, listed: a wave's at consecutive positions
+    const int count = __popc(ghost);
+    int inc = count;
+#pragma unroll
+    for (int off = 1; off < PSR_WAVE; off <<= 1) {
+        const int o = __shfl_up(inc, off, PSR_WAVE);
+        if (int(__lane_id()) >= off) inc += o;
+    }
+    int base = 0;
+    if (__lane_id() == PSR_WAVE - 1 && inc) base = atomicAdd(&entries, inc);
+    int at = __builtin_amdgcn_readlane(base, PSR_WAVE - 1) + inc - count;
+    for (unsigned m = ghost; m; m &= m - 1) list[at++] = static_cast<unsigned short>(t << 5 | __builtin_ctz(m));
+    __syncthreads();
+    for (int e = t; e < entries; e += kRowThreads) {
+        const int row = list[e] >> 5, q = list[e] & 31;
+        const int n = a.neigh[size_t(q) * M + r0 + row];
+        static_assert(kGhostTable == 1 << 11, "hash bits");
+        unsigned h = (unsigned(n) * 2654435761u) >> 21;
+        for (int tries = 0; tries < kGhostTable; ++tries, h = (h + 1) & (kGhostTable - 1)) {
+            const int old = atomicCAS(&key[h], -1, n);
+            if (old != -1 && old != n) continue;
+            place[q < 13 ? q : q - 1][row] = static_cast<unsigned short>(kGhostMark | h);
+            break;  // (a full table leaves kPlaceMemory)
+        }
+    }
+    __syncthreads();
+    // the positions in use are numbered wave by wave, and listed
+    int* rowsOf = a.ghosts + size_t(psr_bid) * kGhostMax;
+    for (int h = t; h < kGhostTable; h += kRowThreads) {
+        const int row = key[h];
+        const unsigned long long mask = __ballot(row >= 0);
+        int n = 0;
+        if (__lane_id() == 0 && mask) n = atomicAdd(&ghosts, __popcll(mask));
+        n = __builtin_amdgcn_readfirstlane(n) + __popcll(mask & ((1ull << __lane_id()) - 1ull));
+        number[h] = static_cast<unsigned short>(n);
+        if (row >= 0 && n < kGhostMax) rowsOf[n] = row;
+    }
+    __syncthreads();
+    // more ghosts than the list holds: every neighbour outside is read from memory
+    const bool overflow = ghosts > kGhostMax;
+    auto final_place = [&](int e) {
+        unsigned p = place[e][t];
+        if (p & kGhostMark) p = overflow ? unsigned(kPlaceMemory) : unsigned(kPlaceGhosts) + 4u * number[p & (kGhostTable - 1)];
+        if (own && p == unsigned(kPlaceMemory)) bad = 1u;
+        return p;
+    };
+    unsigned word = 0u;
+#pragma unroll
+    for (int e = 0; e < 26; e += 2) {
+        word = final_place(e) | final_place(e + 1) << 16;
+        if (own && e < 24) a.places[size_t(e / 2) * M + i] = word;
+    }
+#pragma unroll
+    for (int q = 0; q < 27; ++q)
+        if (own && v[q] != 0.f && __float_as_uint(v[q]) != weight[q]) bad = 1u;
+    if (bad) slow = 1;
+    __syncthreads();
+    // readers of a row outside its workgroup: symmetric where the tables are regular
+    const bool boundary = outside != 0u || *a.q1Fired != 0 || slow != 0;
+    if (own) a.places[size_t(12) * M + i] = word | (boundary ? kBoundaryBit : 0u);
+    RowHead& head = a.heads[psr_bid];
+    if (t < 27) head.w[t] = __uint_as_float(weight[t]);
+    if (t == 0) head.ghosts = overflow ? 0 : ghosts, head.slow = slow;
+}
+__global__ void __launch_bounds__(kRowThreads) row_maps(CgParams P, RowMapArgs a) {
+    row_maps_body(blockIdx.x, gridDim.x, P, a);
+}
+PSR_BATCHABLE(row_maps, kRowThreads)
+
+// A value that is the same in every lane, in scalar registers: the rows' state
+// needs the vector ones (a spilled one's reload would wait for the records'
+// stores ahead of it).
+__device__ __forceinline__ float uniform(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+__device__ __forceinline__ double uniform(double v) {
+    const long long b = __double_as_longlong(v);
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(int(b >> 32)), __builtin_amdgcn_readfirstlane(int(b)));
+}
+
+struct RowShared {
+    float v[kRowThreads + kGhostMax + 1];  // the rows' values, the ghosts', a zero
+    unsigned place[13][kRowThreads];       // the rows' places; a one-wave group's own weights where it has no rows
+    double sum[2][kRowWaves][2];           // wave sums, by the parity of the sum
+    double fold[kRowWaves][2];
+    int fail;
+};
+
+// A row's place in its group and what it needs of the stencil.
+struct RowMap {
+    int ghostRow[2];     // this thread's ghosts (places t and t + kRowThreads of them): row, or -1
+    bool boundary;       // a neighbour lies outside the workgroup, and so a reader of this row
+    bool slow;           // the same in the whole workgroup
+};
+
+// Row t's weight of slot q in a one-wave group of the slow form (as bits).
+__device__ __forceinline__ unsigned& row_own_weight(RowShared& sh, int q, int t) {
+    static_assert(kRowThreads >= 4 * PSR_WAVE && 13 * 3 >= 27, "the weights fit beside a wave's places");
+    return sh.place[q / 3][PSR_WAVE * (1 + q % 3) + t];
+}
+
+__device__ __forceinline__ RowMap row_map(RowShared& sh, const RowMapArgs& a, int bid, int r0, int rows, int M, bool oneWave,
+                                          float (&w)[27]) {
+    RowMap m;
+    const int t = int(threadIdx.x), i = r0 + min(t, rows - 1);
+    const bool own = t < rows;
+    const RowHead& head = a.heads[bid];
+    const int ghosts = __builtin_amdgcn_readfirstlane(head.ghosts);
+    m.slow = __builtin_amdgcn_readfirstlane(head.slow) != 0;
+#pragma unroll
+    for (int q = 0; q < 27; ++q) w[q] = uniform(head.w[q]);
+#pragma unroll
+    for (int e = 0; e < 13; ++e) {
+        const unsigned p = a.places[size_t(e) * M + i];
+        if (e == 12) m.boundary = own && (p & kBoundaryBit) != 0u;
+        sh.place[e][t] = p & ~(e == 12 ? kBoundaryBit : 0u);
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        const int e = t + g * kRowThreads;
+        m.ghostRow[g] = e < ghosts ? a.ghosts[size_t(bid) * kGhostMax + e] : -1;
+    }
+    if (m.slow && oneWave && t < PSR_WAVE) {
+        // such a group may take thousands of sweeps: its weights beside its values
+#pragma unroll 1
+        for (int q = 0; q < 27; ++q) row_own_weight(sh, q, t) = own ? __float_as_uint(a.val[size_t(q) * M + i]) : 0u;
+    }
+    if (t == 0) sh.fail = 0, sh.v[kPlaceZero / 4] = 0.f;
+    __syncthreads();
+    return m;
+}
+
+// sum over the slots in order of weight x value, acc = term(acc, weight, value),
+// the values from LDS (`self`: the row's own); a thread without a row gets
+// something, which it must not use.  memory(e): the value of the
+// neighbour in entry e of the table where it has no place (slow form only).
+template <class T, class Term, class Memory>
+__device__ __forceinline__ T row_product(const RowMap& m, const RowMapArgs& a, RowShared& sh, const float (&w)[27],
+                                         float self, bool own, bool oneWave, int i, int M, T acc, Term term, Memory memory) {
+    auto placed = [&](unsigned p) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sh.v) + p); };
+    if (!m.slow) {
+        // half of the neighbours' values are read together, then summed
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int first = half ? 14 : 0, count = half ? 12 : 14;
+            float n[14];
+#pragma unroll
+            for (int e = 0; e < count; e += 2) {
+                const unsigned p = sh.place[(first + e) / 2][threadIdx.x];
+                n[e] = placed(p & 0xffffu);
+                n[e + 1] = placed(p >> 16);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < count; ++e) {
+                if (first + e == 13) acc = term(acc, w[13], self);  // slot 13, the row itself, comes before entry 13
+                acc = term(acc, w[first + e < 13 ? first + e : first + e + 1], n[e]);
+            }
+        }
+        return acc;
+    }
+    if (!own) return acc;
+    const int t = int(threadIdx.x);
+#pragma unroll 1
+    for (int c = 0; c < 27; c += 9) {
+        float v[9];
+        asm volatile("" : "+v"(i));  // addresses are formed anew, not kept from sweep to sweep
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+            v[k] = oneWave ? __uint_as_float(row_own_weight(sh, c + k, t)) : (a.val + size_t(c + k) * M)[unsigned(i)];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            const int q = c + k;
+            if (v[k] == 0.f) continue;  // adds nothing
+            float n = self;
+            if (q != 13) {
+                const int e = q < 13 ? q : q - 1;
+                const unsigned p = (sh.place[e / 2][t] >> (e & 1 ? 16 : 0)) & 0xffffu;
+                n = p == unsigned(kPlaceMemory) ? memory(size_t(q) * M + i) : placed(p);
+            }
+            acc = term(acc, v[k], n);
+        }
+    }
+    return acc;
+}
+
+// One group's sums: where its slots lie and how far it is.
+struct RowGroup {
+    float4* region;    // [2 parities][blocks][kSlotStride] slots
+    int blocks;        // of the group
+    int firstBlock;    // this workgroup's first
+    int ownBlocks;     // and how many it has
+    bool multi, oneWave;
+    unsigned phase, parity;
+    unsigned spinLimit;
+    int* errFlag;
+};
+
+// Sums v[n] over the group's rows, the same bits in every thread of every
+// workgroup: wave sums, blocks of four waves, then the blocks in the order of
+// 64 a wave.  A block's total goes to its slot(s), 8 bytes of payload stamped
+// with the phase in one 16-byte store; every workgroup reads all blocks' slots,
+// one lane a slot, each wave until its own have come, and folds them: no
+// atomics, one memory round trip after the last workgroup's store.  Slots
+// alternate with the parity of the phase (a workgroup runs at most one phase
+// ahead of the slowest) and start at zero (phases start at 1).  Every store of
+// the workgroup before the call completes before its slots are stored: whoever
+// has seen a phase's slots reads that phase's records.
+template <int N>
+__device__ __forceinline__ bool row_group_sum(double (&v)[N], RowShared& sh, RowGroup& g) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) v[n] = wave_sum_f64(v[n]);
+    if (g.oneWave) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) v[n] = uniform(v[n]);
+        wave_sync_memory();
+        return true;
+    }
+    const int lane = int(__lane_id()), wave = threadIdx.x / PSR_WAVE;
+    g.parity ^= 1u;
+    if (g.multi) __builtin_amdgcn_s_waitcnt(0);
+    if (lane == 0) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) sh.sum[g.parity][wave][n] = v[n];
+    }
+    __syncthreads();
+    auto block_total = [&](int b, int n) {
+        double s = 0;
+        for (int k = 0; k < kRowBlockWaves; ++k) s += sh.sum[g.parity][b * kRowBlockWaves + k][n];
+        return s;
+    };
+    if (!g.multi) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            double s = block_total(0, n);
+            for (int b = 1; b < kRowBlocks; ++b) s += block_total(b, n);
+            v[n] = uniform(s);
+        }
+        return true;
+    }
+    ++g.phase;
+    const __amdgpu_buffer_rsrc_t rs = vec_rsrc(g.region + size_t(g.phase & 1u) * g.blocks * kSlotStride,
+                                               sizeof(float4) * size_t(g.blocks) * kSlotStride);
+    const float stamp = __uint_as_float(g.phase);
+    if (int(threadIdx.x) < N * g.ownBlocks) {
+        const int b = int(threadIdx.x) / N, n = int(threadIdx.x) % N;
+        const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(block_total(b, n)));
+        st_vec4(rs, (g.firstBlock + b) * kSlotStride + n,
+                make_float4(__uint_as_float(unsigned(u)), __uint_as_float(unsigned(u >> 32)), stamp, 0.f));
+    }
+    double part[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) part[n] = 0.0;
+    for (int k = int(threadIdx.x); k - int(threadIdx.x) < g.blocks; k += kRowThreads) {
+        const bool mine = k < g.blocks;
+        float4 got[N];
+        for (unsigned spins = 0;; ++spins) {
+            bool ready = true;
+            if (mine) {
+#pragma unroll
+                for (int n = 0; n < N; ++n) {
+                    got[n] = ld_vec4(rs, k * kSlotStride + n);
+                    ready = ready && __float_as_uint(got[n].z) == g.phase;
+                }
+            }
+            if (__ballot(!ready) == 0) break;
+            if (spins >= g.spinLimit || ((spins & 63u) == 63u && __hip_atomic_load(g.errFlag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                __hip_atomic_store(g.errFlag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                sh.fail = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (mine) {
+#pragma unroll
+            for (int n = 0; n < N; ++n) part[n] += __hiloint2double(__float_as_int(got[n].y), __float_as_int(got[n].x));
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        part[n] = wave_sum_f64(part[n]);
+        if (lane == 0) sh.fold[wave][n] = part[n];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        double s = 0;
+        for (int k = 0; k < kRowWaves; ++k) s += sh.fold[k][n];
+        v[n] = uniform(s);
+    }
+    return __builtin_amdgcn_readfirstlane(sh.fail) == 0;
+}
+
+__device__ __forceinline__ RowGroup row_group(const CgParams& P, const CgGroup& G, int local, float4* slots, int* errFlag) {
+    RowGroup g;
+    const int per = G.rowsPerWg > kRowBlock ? kRowBlocks : 1;  // blocks of a full workgroup
+    const int last = G.rows - (G.wgs - 1) * G.rowsPerWg;       // rows of the last
+    g.blocks = (G.wgs - 1) * per + (last > kRowBlock ? 2 : 1);
+    g.firstBlock = local * per;
+    g.ownBlocks = local + 1 < G.wgs ? per : g.blocks - g.firstBlock;
+    g.region = slots + size_t(2) * kRowBlocks * kSlotStride * G.firstWg;
+    g.multi = G.wgs > 1;
+    // a group of at most one wave of rows (the coarsest depths) iterates in
+    // wave 0 alone, with no workgroup barrier (a wave's sum equals the block's,
+    // whose other waves add exact zeros)
+    g.oneWave = !g.multi && G.rows <= PSR_WAVE;
+    g.phase = g.parity = 0u;
+    g.spinLimit = P.spinLimit;
+    g.errFlag = errFlag;
+    return g;
+}
+__device__ __forceinline__ void row_sync(const RowGroup& g) {
+    if (g.oneWave) wave_sync_memory();
+    else __syncthreads();
+}
+
+// The reference's CG (CGAlgorithm.cu:10-80), one launch for all depths.  Per
+// iteration k the record of row i in buffer k & 1 holds {r_k, p_{k-1}}; a
+// ghost's p_k = r_k + beta p_{k-1} is formed from it, so the update of p and
+// the product A p need no group barrier in between (CGAlgorithm.cu:37-53).
+__device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& maps,
+                                                 const float* __restrict__ b, float* __restrict__ x, float2* state,
+                                                 float4* slots, int* __restrict__ iters, double* __restrict__ resid,
+                                                 int* errFlag) {
+    __shared__ RowShared sh;
     int gi = 0;
     while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
     const CgGroup G = P.g[gi];
-    const int local = psr_bid - G.firstWg;
-    const int i = G.rowBegin + local * G.rowsPerWg + int(threadIdx.x);
-    const bool own = int(threadIdx.x) < G.rowsPerWg && i < G.rowBegin + G.rows;
-    const int M = P.M;
-    double* part = partial + 2 * G.firstWg;
-    GroupCtl* ctl = ctlAll + gi;
-    unsigned phase = 0;
-    // a group of one workgroup exchanges its records through LDS (its rows
-    // are the depth's, all in this workgroup): no memory round trip per sweep
-    __shared__ float2 lrec2[2][kCgThreads];
-    const bool multi = G.wgs > 1;
-    // a group of at most one wave of rows (the coarsest depths) iterates in
-    // wave 0 alone, with wave reductions and no workgroup barrier per step
-    // (a wave's sum equals the block's, whose other waves add exact zeros)
-    const bool oneWave = !multi && G.rows <= PSR_WAVE;
-    if (oneWave && int(threadIdx.x) >= PSR_WAVE) return;
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M;
+    const int r0 = G.rowBegin + local * G.rowsPerWg;
+    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0, i = r0 + t;
+    const bool own = t < rows;
+    RowGroup g = row_group(P, G, local, slots, errFlag);
+    float w[27];
+    const RowMap m = row_map(sh, maps, psr_bid, r0, rows, M, g.oneWave, w);
+    const int* __restrict__ neigh = maps.neigh;
+    if (g.oneWave && t >= PSR_WAVE) return;
     const __amdgpu_buffer_rsrc_t st = vec_rsrc(state, sizeof(float2) * 2 * size_t(M));
-    auto group_sum = [&](double v, double& out) -> bool {
-        if (oneWave) {
-            out = wave_sum_f64(v);
-            wave_sync_memory();
-            return true;
-        }
-        double s = block_sum_double(v, sh);
-        if (!multi) {
-            out = s;
-            return true;
-        }
-        return group_allreduce(s, out, part, ctl, phase, G.wgs, local, P.spinLimit, errFlag, &shFlag, &shRes,
-                               [&](const double* parts, int n) { return fold_double(parts, n, sh); });
-    };
-    Stencil sr;
-    if (own) sr.load(val, neigh, M, i);
     // x = 0, r = b, rr = r.r  (CGAlgorithm.cu:21-33 with x0 = 0)
-    float xi = 0.f, ri = 0.f, pi = 0.f, api = 0.f;
-    double loc = 0;
-    if (own) {
-        ri = b[i];
-        if (multi) st_vec2(st, i, make_float2(ri, 0.f));
-        else lrec2[0][threadIdx.x] = make_float2(ri, 0.f);
-        loc = double(ri * ri);
-    }
-    double rrD;
-    if (!group_sum(loc, rrD)) return;
-    float rr = float(rrD), rrOld = 1.f;
+    float xi = 0.f, ri = own ? b[i] : 0.f, pi = 0.f;
+    if (m.boundary) st_vec2(st, i, make_float2(ri, 0.f));
+    double sum[1] = {double(ri * ri)};
+    if (!row_group_sum<1>(sum, sh, g)) return;
+    float rr = uniform(float(sum[0])), rrOld = 1.f;
     int k = 1;
     while (rr > P.tolSq && k <= P.maxIter) {
-        const float beta = (k > 1) ? rr / rrOld : 0.f;
-        const int cur = ((k - 1) & 1) * M, nxt = M - cur, curL = (k - 1) & 1;
+        const float beta = uniform((k > 1) ? rr / rrOld : 0.f);
+        const int cur = ((k - 1) & 1) * M, nxt = M - cur;
         // p = r + beta p (CGAlgorithm.cu:37-43), Ap = A p (:47), p.Ap (:53)
-        double lpAp = 0;
-        if (own) {
-            float s = 0.f;
-            if (oneWave) {
-                // a straight-line LDS loop for the one-wave groups (the choice
-                // per slot below costs them two branches a slot)
+        float2 n[2];
 #pragma unroll
-                for (int q = 0; q < 27; ++q) {
-                    const float2 nb = lrec2[curL][sr.j[q] - G.rowBegin];
-                    s += sr.v[q] * p_next(nb.x, beta, nb.y);
-                }
-            } else {
+        for (int e = 0; e < 2; ++e)
+            if (m.ghostRow[e] >= 0) n[e] = ld_vec2(st, cur + m.ghostRow[e]);
+        pi = p_next(ri, beta, pi);
+        sh.v[t] = pi;
 #pragma unroll
-                for (int q = 0; q < 27; ++q) {
-                    const float2 nb = multi ? ld_vec2(st, cur + sr.j[q]) : lrec2[curL][sr.j[q] - G.rowBegin];
-                    s += sr.v[q] * p_next(nb.x, beta, nb.y);
-                }
-            }
-            pi = p_next(ri, beta, pi);
-            api = s;
-            lpAp = double(pi * s);
-        }
-        double pAp;
-        if (!group_sum(lpAp, pAp)) return;
-        const float alpha = float(double(rr) / pAp);
-        double lrr = 0;
-        if (own) {
-            xi = xi + alpha * pi;
-            ri = ri + (-alpha) * api;
-            if (multi) st_vec2(st, nxt + i, make_float2(ri, pi));
-            else lrec2[curL ^ 1][threadIdx.x] = make_float2(ri, pi);
-            lrr = double(ri * ri);
-        }
+        for (int e = 0; e < 2; ++e)
+            if (m.ghostRow[e] >= 0) sh.v[kRowThreads + e * kRowThreads + t] = p_next(n[e].x, beta, n[e].y);
+        row_sync(g);
+        auto term = [](float a, float wq, float v) { return __fmaf_rn(wq, v, a); };
+        auto memory = [&](size_t e) {
+            const float2 r = ld_vec2(st, cur + neigh[e]);
+            return p_next(r.x, beta, r.y);
+        };
+        const float api = row_product(m, maps, sh, w, pi, own, g.oneWave, i, M, 0.f, term, memory);
+        sum[0] = own ? double(pi * api) : 0.0;
+        if (!row_group_sum<1>(sum, sh, g)) return;
+        const float alpha = uniform(float(double(rr) / sum[0]));
+        xi = __fmaf_rn(alpha, pi, xi);
+        ri = own ? __fmaf_rn(-alpha, api, ri) : 0.f;
+        if (m.boundary) st_vec2(st, nxt + i, make_float2(ri, pi));
+        sum[0] = double(ri * ri);
         rrOld = rr;
-        double rrNew;
-        if (!group_sum(lrr, rrNew)) return;
-        rr = float(rrNew);
+        if (!row_group_sum<1>(sum, sh, g)) return;
+        rr = uniform(float(sum[0]));
         ++k;
     }
     if (own) x[i] = xi;
-    if (local == 0 && threadIdx.x == 0) {
+    if (local == 0 && t == 0) {
         iters[G.depth] = k - 1;
         iters[PSR_MAX_DEPTH + 1 + G.depth] = 1;
         resid[G.depth] = sqrt(double(rr));
     }
 }
-__global__ void __launch_bounds__(kCgThreads) cg_fp32_row(CgParams P, const int* __restrict__ neigh,
-                                                          const float* __restrict__ val, const float* __restrict__ b,
-                                                          float* __restrict__ x, float2* state, double* partial,
-                                                          GroupCtl* ctlAll, int* __restrict__ iters,
-                                                          double* __restrict__ resid, int* errFlag) {
-    cg_fp32_row_body(blockIdx.x, gridDim.x, P, neigh, val, b, x, state, partial, ctlAll, iters, resid, errFlag);
+__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kRowFp32Waves))) cg_fp32_row(
+    CgParams P, RowMapArgs maps, const float* __restrict__ b, float* __restrict__ x, float2* state, float4* slots,
+    int* __restrict__ iters, double* __restrict__ resid, int* errFlag) {
+    cg_fp32_row_body(blockIdx.x, gridDim.x, P, maps, b, x, state, slots, iters, resid, errFlag);
 }
-PSR_BATCHABLE(cg_fp32_row, kCgThreads)
+PSR_BATCHABLE_WAVES(cg_fp32_row, kRowThreads, kRowFp32Waves)
 
 
 // A group of one workgroup with at most one row a thread (the coarse depths,
@@ -734,143 +1002,54 @@ __device__ __forceinline__ Comp2 block_comp2(Comp2 v, Comp2* sh) {
     return t;
 }
 
-// The row form's two dot products, gamma = r.r and delta = w.r, summed in
-// FP64: a lane's product of two floats is exact in FP64, and the wave, block
-// and group sums take the order of wave_sum_f64, block_sum_double and
-// slot_sum_double, so gamma of a right-hand side b is ||b||^2 to the bit.
-struct Dots {
-    double g, d;
-};
-__device__ __forceinline__ Dots wave_sum_dots(Dots v) {
-    v.g += dpp_f64<kDppSwap1>(v.g);
-    v.d += dpp_f64<kDppSwap1>(v.d);
-    v.g += dpp_f64<kDppSwap2>(v.g);
-    v.d += dpp_f64<kDppSwap2>(v.d);
-    v.g += dpp_f64<kDppHalfMirror>(v.g);
-    v.d += dpp_f64<kDppHalfMirror>(v.d);
-    v.g += dpp_f64<kDppMirror>(v.g);
-    v.d += dpp_f64<kDppMirror>(v.d);
-    return Dots{(readlane_f64(v.g, 0) + readlane_f64(v.g, 16)) + (readlane_f64(v.g, 32) + readlane_f64(v.g, 48)),
-                (readlane_f64(v.d, 0) + readlane_f64(v.d, 16)) + (readlane_f64(v.d, 32) + readlane_f64(v.d, 48))};
-}
-// fenceStores: the block's earlier stores complete before its barrier (a
-// workgroup barrier alone does not wait for them); the wave's sum is formed
-// while they are in flight.
-__device__ __forceinline__ Dots block_sum_dots(Dots v, double2* sh, bool fenceStores = false) {
-    v = wave_sum_dots(v);
-    if (fenceStores) __builtin_amdgcn_s_waitcnt(0);
-    const int w = threadIdx.x / PSR_WAVE;
-    if (__lane_id() == 0) sh[w] = make_double2(v.g, v.d);
-    __syncthreads();
-    Dots s{0.0, 0.0};
-    for (int k = 0; k < kCgWaves; ++k) {
-        s.g += sh[k].x;
-        s.d += sh[k].y;
-    }
-    __syncthreads();
-    return s;
-}
-
-// Mixed form, one launch for all depths, one row per thread.  Per inner
-// iteration k the 12-byte record of row i in buffer k & 1 holds {r_k, w_k, s_{k-1}};
-// the row writes {r_{k+1}, w_{k+1}, s_k} to the other buffer, keeps its r, w,
-// s, p and x in registers (x is also stored for the outer residual) and its
-// stencil in LDS.
-__device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, const CgParams& P, const int* __restrict__ neigh,
-                                                           const float* __restrict__ val,
-                                                           const float* __restrict__ b, float* x, float* rOut,
-                                                           float3* state, float4* slots, int* __restrict__ iters,
-                                                           double* __restrict__ resid, double* __restrict__ trueRel,
-                                                           int* errFlag) {
-    __shared__ double shd[kCgWaves];
-    __shared__ double2 shp[kCgWaves];
-    __shared__ float lV[27][kCgThreads];  // the row's stencil, read from LDS every sweep
-    __shared__ int lJ[27][kCgThreads];
+// Mixed form, one launch for all depths, one row per thread.  The two dot
+// products, gamma = r.r and delta = w.r, are summed in FP64 (a product of two
+// floats is exact in FP64), so gamma of a right-hand side b is ||b||^2 to the
+// bit.  Per inner iteration k the record of row i in buffer k & 1 holds
+// {r_k, w_k, s_{k-1}, x_k}; the row writes {r_{k+1}, w_{k+1}, s_k, x_{k+1}} to
+// the other buffer.
+__device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& maps,
+                                                  const float* __restrict__ b, float* x, float* rOut, float4* state,
+                                                  float4* slots, int* __restrict__ iters, double* __restrict__ resid,
+                                                  double* __restrict__ trueRel, int* errFlag) {
+    __shared__ RowShared sh;
     int gi = 0;
     while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
     const CgGroup G = P.g[gi];
-    const int local = psr_bid - G.firstWg;
-    const int i = G.rowBegin + local * G.rowsPerWg + int(threadIdx.x);
-    const bool own = int(threadIdx.x) < G.rowsPerWg && i < G.rowBegin + G.rows;
-    const int M = P.M;
-    float4* region = slots + size_t(4) * G.firstWg;  // [2][wgs][2]
-    unsigned phase = 0;
-    // a group of one workgroup exchanges its records through LDS
-    __shared__ float3 lrec3[2][kCgThreads];
-    const bool multi = G.wgs > 1;
-    // a group of at most one wave of rows iterates in wave 0 alone (as in the
-    // FP32 row form)
-    const bool oneWave = !multi && G.rows <= PSR_WAVE;
-    if (oneWave && int(threadIdx.x) >= PSR_WAVE) return;
-    const __amdgpu_buffer_rsrc_t st = vec_rsrc(state, sizeof(float3) * 2 * size_t(M));
-    auto sum_double = [&](double v, double& out) -> bool {
-        if (oneWave) {
-            out = wave_sum_f64(v);
-            wave_sync_memory();
-            return true;
-        }
-        // the stores of x and of the outer residual complete before the slot
-        // (as the records before the dots' slot)
-        if (multi) __builtin_amdgcn_s_waitcnt(0);
-        double s = block_sum_double(v, shd);
-        if (!multi) {
-            out = s;
-            return true;
-        }
-        return slot_sum_double(s, out, region, G.wgs, local, phase, P.spinLimit, errFlag, shd);
-    };
-    auto sum_dots = [&](Dots v, Dots& out) -> bool {
-        if (oneWave) {
-            out = wave_sum_dots(v);
-            wave_sync_memory();
-            return true;
-        }
-        // Every wave's record stores complete before the barrier, so the slot
-        // stored after it is never seen before them: a workgroup that has seen
-        // every slot of a phase reads the records of that phase.
-        const Dots s = block_sum_dots(v, shp, multi);
-        if (!multi) {
-            out = s;
-            return true;
-        }
-        const unsigned long long ug = static_cast<unsigned long long>(__double_as_longlong(s.g));
-        const unsigned long long ud = static_cast<unsigned long long>(__double_as_longlong(s.d));
-        const unsigned mine[4] = {unsigned(ug), unsigned(ug >> 32), unsigned(ud), unsigned(ud >> 32)};
-        float4 got[kPollPerThread][2];
-        if (!slot_exchange<2>(region, G.wgs, local, phase, mine, got, P.spinLimit, errFlag)) return false;
-        Dots t{0.0, 0.0};
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M;
+    const int r0 = G.rowBegin + local * G.rowsPerWg;
+    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0, i = r0 + t;
+    const bool own = t < rows;
+    RowGroup g = row_group(P, G, local, slots, errFlag);
+    float w[27];
+    const RowMap m = row_map(sh, maps, psr_bid, r0, rows, M, g.oneWave, w);
+    const int* __restrict__ neigh = maps.neigh;
+    if (g.oneWave && t >= PSR_WAVE) return;
+    const __amdgpu_buffer_rsrc_t st = vec_rsrc(state, sizeof(float4) * 2 * size_t(M));
+    auto term = [](float a, float wq, float v) { return __fmaf_rn(wq, v, a); };
+    auto ghost_values = [&](auto value) {  // value(row) into the ghosts' places
+        float n[2];
 #pragma unroll
-        for (int j = 0; j < kPollPerThread; ++j)
-            if (int(threadIdx.x) + j * kCgThreads < G.wgs) {
-                t.g += __hiloint2double(__float_as_int(got[j][0].y), __float_as_int(got[j][0].x));
-                t.d += __hiloint2double(__float_as_int(got[j][1].y), __float_as_int(got[j][1].x));
-            }
-        out = block_sum_dots(t, shp);
-        return true;
-    };
-    if (own) {
-        Stencil sr;
-        sr.load(val, neigh, M, i);
-#pragma unroll
-        for (int q = 0; q < 27; ++q) {
-            lV[q][threadIdx.x] = sr.v[q];
-            lJ[q][threadIdx.x] = sr.j[q];
+        for (int e = 0; e < 2; ++e) {
+            int j = m.ghostRow[e];
+            asm volatile("" : "+v"(j));  // no address is kept from step to step
+            n[e] = j >= 0 ? value(j) : 0.f;
         }
-    }
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            if (m.ghostRow[e] >= 0) sh.v[kRowThreads + e * kRowThreads + t] = n[e];
+    };
     float xi = 0.f, ro = 0.f, wo = 0.f, so = 0.f, po = 0.f;
-    // x = 0.  ||b||^2 in FP64 (the outer residual of x = 0 is b itself) is
-    // gamma of the first outer step, whose sum is bit for bit that of b.b;
-    // a solve that takes no step sums it alone.
-    if (own) st_shared(&x[i], 0.f);
+    // ||b||^2 in FP64 (the outer residual of x = 0 is b itself) is gamma of the
+    // first outer step, whose sum is bit for bit that of b.b; a solve that
+    // takes no step sums it alone.
     double bb = 0;
     const bool stepping = P.maxOuter > 0 && P.maxIter > 0;
     if (!stepping) {
-        double loc = 0;
-        if (own) {
-            const double bi = b[i];
-            loc = bi * bi;
-        }
-        if (!sum_double(loc, bb)) return;
+        const double bi = own ? double(b[i]) : 0.0;
+        double loc[1] = {bi * bi};
+        if (!row_group_sum<1>(loc, sh, g)) return;
+        bb = loc[0];
     }
     double rr = bb, rel = (bb > 0 || stepping) ? 1.0 : 0.0;
     const float* rhs = b;
@@ -878,24 +1057,23 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
     float gamma = 0.f;
     while (rel > P.relTol && outer < P.maxOuter && total < P.maxIter) {
         // r_0 = rhs, w_0 = A r_0, s_{-1} = 0, p_{-1} = 0
-        Dots d0{0.0, 0.0};
-        if (own) {
-            float w = 0.f;
-#pragma unroll
-            for (int q = 0; q < 27; ++q) w = __fmaf_rn(lV[q][threadIdx.x], ld_shared(&rhs[lJ[q][threadIdx.x]]), w);
-            ro = ld_shared(&rhs[i]);
-            wo = w;
-            so = 0.f;
-            po = 0.f;
-            if (multi) st_vec3(st, i, make_float3(ro, w, 0.f));
-            else lrec3[0][threadIdx.x] = make_float3(ro, w, 0.f);
-            d0.g = double(ro) * double(ro);
-            d0.d = double(w) * double(ro);
+        int ii = i;
+        asm volatile("" : "+v"(ii));  // nor this row's
+        ro = own ? ld_shared(&rhs[ii]) : 0.f;
+        sh.v[t] = ro;
+        ghost_values([&](int j) { return ld_shared(&rhs[j]); });
+        row_sync(g);
+        {
+            auto memory = [&](size_t e) { return ld_shared(&rhs[neigh[e]]); };
+            wo = row_product(m, maps, sh, w, ro, own, g.oneWave, i, M, 0.f, term, memory);
+            if (!own) wo = 0.f;
         }
-        Dots g;
-        if (!sum_dots(d0, g)) return;
+        so = po = 0.f;
+        if (m.boundary) st_vec4(st, i, make_float4(ro, wo, 0.f, xi));
+        double d[2] = {double(ro) * double(ro), double(wo) * double(ro)};
+        if (!row_group_sum<2>(d, sh, g)) return;
         if (outer == 0) {
-            bb = rr = g.g;
+            bb = rr = d[0];
             if (!(bb > 0)) {
                 rel = 0.0;
                 break;
@@ -903,51 +1081,44 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
         }
         // inner target on the updated residual: half the tolerance left, no tighter than FP32 can follow
         const double tgt = fmax(0.5 * P.relTol * sqrt(bb), 1e-6 * sqrt(rr));
-        const float tgt2 = float(tgt * tgt);
-        gamma = float(g.g);
-        float delta = float(g.d);
-        float alpha = gamma / delta, beta = 0.f;
+        const float tgt2 = uniform(float(tgt * tgt));
+        gamma = uniform(float(d[0]));
+        const float delta = float(d[1]);
+        float alpha = uniform(gamma / delta), beta = 0.f;
         int k = 0, kBest = 0;
         float gBest = gamma, xBest = xi;
         while (gamma > tgt2 && total + k < P.maxIter && k - kBest < kCgStall) {
             const int cur = (k & 1) * M, nxt = M - cur;
-            Dots dl{0.0, 0.0};
-            if (own) {
-                float w = 0.f;
-                if (oneWave) {
-                    // a straight-line LDS loop for the one-wave groups
+            float4 n[2];
 #pragma unroll
-                    for (int q = 0; q < 27; ++q) {
-                        const float3 nb = lrec3[k & 1][lJ[q][threadIdx.x] - G.rowBegin];
-                        w = __fmaf_rn(lV[q][threadIdx.x], r_next(nb.x, alpha, s_next(nb.y, beta, nb.z)), w);
-                    }
-                } else {
+            for (int e = 0; e < 2; ++e)
+                if (m.ghostRow[e] >= 0) n[e] = ld_vec4(st, cur + m.ghostRow[e]);
+            const float si = s_next(wo, beta, so);
+            const float rni = r_next(ro, alpha, si);
+            po = __fmaf_rn(beta, po, ro);
+            xi = __fmaf_rn(alpha, po, xi);
+            sh.v[t] = rni;
 #pragma unroll
-                    for (int q = 0; q < 27; ++q) {
-                        const int jq = lJ[q][threadIdx.x];
-                        const float3 nb = multi ? ld_vec3(st, cur + jq) : lrec3[k & 1][jq - G.rowBegin];
-                        w = __fmaf_rn(lV[q][threadIdx.x], r_next(nb.x, alpha, s_next(nb.y, beta, nb.z)), w);
-                    }
-                }
-                const float si = s_next(wo, beta, so);
-                const float rni = r_next(ro, alpha, si);
-                // the record first: the exchange waits for it
-                if (multi) st_vec3(st, nxt + i, make_float3(rni, w, si));
-                else lrec3[(k & 1) ^ 1][threadIdx.x] = make_float3(rni, w, si);
-                po = __fmaf_rn(beta, po, ro);
-                xi = __fmaf_rn(alpha, po, xi);
-                st_shared(&x[i], xi);
-                ro = rni;
-                wo = w;
-                so = si;
-                dl.g = double(rni) * double(rni);
-                dl.d = double(w) * double(rni);
-            }
-            if (!sum_dots(dl, g)) return;
-            const float gNew = float(g.g), dNew = float(g.d);
+            for (int e = 0; e < 2; ++e)
+                if (m.ghostRow[e] >= 0)
+                    sh.v[kRowThreads + e * kRowThreads + t] = r_next(n[e].x, alpha, s_next(n[e].y, beta, n[e].z));
+            row_sync(g);
+            auto memory = [&](size_t e) {
+                const float4 r = ld_vec4(st, cur + neigh[e]);
+                return r_next(r.x, alpha, s_next(r.y, beta, r.z));
+            };
+            wo = row_product(m, maps, sh, w, rni, own, g.oneWave, i, M, 0.f, term, memory);
+            if (!own) wo = 0.f;
+            ro = rni;
+            so = si;
+            if (m.boundary) st_vec4(st, nxt + i, make_float4(rni, wo, si, xi));
+            d[0] = double(rni) * double(rni);
+            d[1] = double(wo) * double(rni);
+            if (!row_group_sum<2>(d, sh, g)) return;
+            const float gNew = uniform(float(d[0])), dNew = float(d[1]);
             const float bNew = gNew / gamma;
-            alpha = gNew / (dNew - bNew * gNew / alpha);
-            beta = bNew;
+            alpha = uniform(gNew / (dNew - bNew * gNew / alpha));
+            beta = uniform(bNew);
             gamma = gNew;
             ++k;
             if (gamma < gBest) {  // the same in every workgroup of the group
@@ -963,43 +1134,48 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
             // orders the restored x before the outer residual reads it
             gamma = gBest;
             xi = xBest;
-            if (own) st_shared(&x[i], xi);
-            double fence;
-            if (!sum_double(0.0, fence)) return;
+            if (m.boundary) st_vec4(st, (k & 1) * M + i, make_float4(0.f, 0.f, 0.f, xi));
+            double fence[1] = {0.0};
+            if (!row_group_sum<1>(fence, sh, g)) return;
         }
-        // outer residual in FP64
-        double loc = 0;
+        // outer residual in FP64, x from the rows and from the last sweep's records
+        const int last = (k & 1) * M;
+        if (g.oneWave) wave_sync_memory();
+        else __syncthreads();  // sh.v of the last product has been read
+        sh.v[t] = xi;
+        ghost_values([&](int j) { return ld_vec4(st, last + j).w; });
+        row_sync(g);
+        double loc[1] = {0.0};
         if (own) {
-            double acc = b[i];
-#pragma unroll
-            for (int q = 0; q < 27; ++q)
-                acc -= double(lV[q][threadIdx.x]) * double(ld_shared(&x[lJ[q][threadIdx.x]]));
-            st_shared(&rOut[i], float(acc));
-            loc = acc * acc;
+            auto term64 = [](double a, float wq, float v) { return a - double(wq) * double(v); };
+            auto memory = [&](size_t e) { return ld_vec4(st, last + neigh[e]).w; };
+            asm volatile("" : "+v"(ii));
+            const double acc = row_product(m, maps, sh, w, xi, own, g.oneWave, i, M, double(b[ii]), term64, memory);
+            st_shared(&rOut[ii], float(acc));
+            loc[0] = acc * acc;
         }
-        if (!sum_double(loc, rr)) return;
-        rel = bb > 0 ? sqrt(rr / bb) : 0.0;
+        if (!row_group_sum<1>(loc, sh, g)) return;
+        rr = loc[0];
+        rel = uniform(bb > 0 ? sqrt(rr / bb) : 0.0);
         rhs = rOut;
         // an inner solve that found no smaller residual leaves x as it was:
         // another outer step would repeat it
         if (kBest == 0) break;
     }
-    if (local == 0 && threadIdx.x == 0) {
+    if (own) x[i] = xi;
+    if (local == 0 && t == 0) {
         iters[G.depth] = total;
         iters[PSR_MAX_DEPTH + 1 + G.depth] = outer;
         resid[G.depth] = sqrt(double(gamma));
         trueRel[G.depth] = rel;
     }
 }
-__global__ void __launch_bounds__(kCgThreads) cg_mixed_row(CgParams P, const int* __restrict__ neigh,
-                                                           const float* __restrict__ val,
-                                                           const float* __restrict__ b, float* x, float* rOut,
-                                                           float3* state, float4* slots, int* __restrict__ iters,
-                                                           double* __restrict__ resid, double* __restrict__ trueRel,
-                                                           int* errFlag) {
-    cg_mixed_row_body(blockIdx.x, gridDim.x, P, neigh, val, b, x, rOut, state, slots, iters, resid, trueRel, errFlag);
+__global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kRowMixedWaves))) cg_mixed_row(
+    CgParams P, RowMapArgs maps, const float* __restrict__ b, float* x, float* rOut, float4* state, float4* slots,
+    int* __restrict__ iters, double* __restrict__ resid, double* __restrict__ trueRel, int* errFlag) {
+    cg_mixed_row_body(blockIdx.x, gridDim.x, P, maps, b, x, rOut, state, slots, iters, resid, trueRel, errFlag);
 }
-PSR_BATCHABLE(cg_mixed_row, kCgThreads)
+PSR_BATCHABLE_WAVES(cg_mixed_row, kRowThreads, kRowMixedWaves)
 
 
 // The mixed form's group of one workgroup with at most one row a thread,
@@ -2048,10 +2224,10 @@ void solve_depths(Ctx& c) {
     // smaller occupancy of the two forms, so that a plan made for one cloud
     // also fits the merged launch.
     if (c.cgMaxWgs <= 0) {
-        auto occupancy = [](const void* single, const void* batched) {
+        auto occupancy = [](const void* single, const void* batched, int threads) {
             int a = 0, b = 0;
-            PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, single, kCgThreads, 0));
-            PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, batched, kCgThreads, 0));
+            PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, single, threads, 0));
+            PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, batched, threads, 0));
             return std::min(a, b);
         };
         const void* rowQueue = mixed ? multi_queue_kernel_of<cg_mixed_row_k>(cg_mixed_row)
@@ -2059,19 +2235,19 @@ void solve_depths(Ctx& c) {
         const void* genQueue = mixed ? multi_queue_kernel_of<cg_mixed_all_depths_k>(cg_mixed_all_depths)
                                      : multi_queue_kernel_of<cg_all_depths_k>(cg_all_depths);
         int cus = 0;
-        const int perRow = occupancy(rowKernel, rowQueue), perGen = occupancy(genKernel, genQueue);
+        const int perRow = occupancy(rowKernel, rowQueue, kRowThreads), perGen = occupancy(genKernel, genQueue, kCgThreads);
         const int perMinres = occupancy(reinterpret_cast<const void*>(cg_mixed_minres),
-                                        multi_queue_kernel_of<cg_mixed_minres_k>(cg_mixed_minres));
+                                        multi_queue_kernel_of<cg_mixed_minres_k>(cg_mixed_minres), kCgThreads);
         PSR_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
         c.cgMaxWgsRow = std::max(0, perRow * cus);
         c.cgMaxWgs = std::max(1, perGen * cus);
         c.cgMaxWgsMinres = std::max(1, perMinres * cus);
         c.cgMaxWgsChip[0] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip4),
-                                            multi_queue_kernel_of<cg_minres_chip4_k>(cg_minres_chip4));
+                                            multi_queue_kernel_of<cg_minres_chip4_k>(cg_minres_chip4), kCgThreads);
         c.cgMaxWgsChip[1] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip8),
-                                            multi_queue_kernel_of<cg_minres_chip8_k>(cg_minres_chip8));
+                                            multi_queue_kernel_of<cg_minres_chip8_k>(cg_minres_chip8), kCgThreads);
         c.cgMaxWgsChip[2] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip16),
-                                            multi_queue_kernel_of<cg_minres_chip16_k>(cg_minres_chip16));
+                                            multi_queue_kernel_of<cg_minres_chip16_k>(cg_minres_chip16), kCgThreads);
     }
     // the mixed form solves indefinite depths with MINRES, in a launch of its
     // own (the MINRES kernel) after the CG launch of the other depths
@@ -2085,14 +2261,18 @@ void solve_depths(Ctx& c) {
         return w;
     };
     auto need = [&](int rpw) { return need_of(rpw, false) + need_of(rpw, true); };
-    // one row per thread (stencil in registers) when every group fits at
-    // kCgThreads rows per workgroup; otherwise widen the row blocks
-    int rowsPerWg = c.cgRowsPerWg > 0 ? c.cgRowsPerWg : kCgThreads;
-    bool rowForm = rowsPerWg <= kCgThreads && need(rowsPerWg) <= c.cgMaxWgsRow;
+    // One row per thread, kRowThreads rows a workgroup, when all workgroups are
+    // resident (about 390k rows) and every group's blocks fit the fold;
+    // otherwise several rows per thread, the row blocks widened until they fit.
+    int rowsPerWg = c.cgRowsPerWg > 0 ? c.cgRowsPerWg : kRowThreads;
+    auto blocks_of = [&](int rows, int rpw) { return int(div_up(unsigned(rows), unsigned(rpw))) * (rpw > kRowBlock ? 2 : 1); };
+    // (the override of the rows per workgroup reaches the several-rows form beyond 256)
+    bool rowForm = (c.cgRowsPerWg == 0 || c.cgRowsPerWg <= kRowBlock) && need(rowsPerWg) <= c.cgMaxWgsRow;
     for (int d = 0; d <= D; ++d)
-        if (div_up(L.count[d], kCgThreads) > unsigned(kPollPerThread * kCgThreads)) rowForm = false;
+        if (blocks_of(L.count[d], rowsPerWg) > kRowMaxBlocks) rowForm = false;
     // MINRES runs in the several-rows-per-thread form only
     if (anyIndef) rowForm = false;
+    if (!rowForm && c.cgRowsPerWg == 0) rowsPerWg = kCgThreads;
     int rowsPerWgMinres = rowsPerWg;
     if (!rowForm) {
         while (need_of(rowsPerWg, false) > c.cgMaxWgs) rowsPerWg *= 2;
@@ -2101,14 +2281,14 @@ void solve_depths(Ctx& c) {
     // A batch sets the rows a workgroup takes instead (cgRowTarget, from the
     // batch's total rows and the resident budget): a depth of n rows gets
     // ceil(n / target) workgroups of equal shares; one row per thread when
-    // every share fits 256 rows.
+    // every share fits the workgroup's threads.
     int capRows[PSR_MAX_DEPTH + 1];
     if (c.cgRowTarget > 0) {
         rowForm = true;
         for (int d = 0; d <= D; ++d) {
             const int w = std::max(1, int(div_up(L.count[d], unsigned(c.cgRowTarget))));
             capRows[d] = std::max(1, int(div_up(L.count[d], unsigned(w))));
-            if (capRows[d] > kCgThreads) rowForm = false;
+            if (capRows[d] > kRowThreads || blocks_of(L.count[d], capRows[d]) > kRowMaxBlocks) rowForm = false;
         }
         if (anyIndef) rowForm = false;
     }
@@ -2152,8 +2332,8 @@ void solve_depths(Ctx& c) {
     double* trueRel = res->cgTrueRel;
     int* err = &res->cgErr;
     // slots of the row form's groups, or of the on-chip MINRES's
-    const size_t slotCount = rowForm && mixed ? size_t(4) * wg
-                                              : (chip >= 0 ? size_t(4) * wgM + PM.ngroups * minres_result_slots() : 0);
+    const size_t slotCount = rowForm ? size_t(2) * kRowBlocks * kSlotStride * wg
+                                     : (chip >= 0 ? size_t(4) * wgM + PM.ngroups * minres_result_slots() : 0);
     float4* slots = slotCount ? c.buf<float4>("cg_slots", slotCount) : nullptr;
     // The group controls and slots start at zero: the neighbour-column kernel
     // clears them after every solve, so they need a launch of their own only
@@ -2199,9 +2379,16 @@ void solve_depths(Ctx& c) {
         }
         PSR_HIP_CHECK(hipEventRecord(c.ev[8], s));
     }
-    if (rowForm && mixed) P.spinLimit = 1u << 22;
+    if (rowForm) P.spinLimit = 1u << 22;
     if (chip >= 0) PM.spinLimit = 1u << 24;  // polls of about a microsecond; a batch's group may wait for the solves before it
     if (c.cgSpinLimit >= 0) P.spinLimit = PM.spinLimit = unsigned(c.cgSpinLimit);
+    RowMapArgs maps{o.neigh, val, o.q1Fired, nullptr, nullptr, nullptr};
+    if (rowForm) {
+        maps.places = c.buf<unsigned>("cg_places", size_t(13) * M);
+        maps.ghosts = c.buf<int>("cg_ghosts", size_t(kGhostMax) * wg);
+        maps.heads = c.buf<RowHead>("cg_heads", wg);
+        PSR_LAUNCH(row_maps, wg, 0, s, P, maps);
+    }
     static const char siteMixedRow = 0, siteMixedGen = 0, siteMinres = 0, siteRow = 0, siteGen = 0;
     static const char siteChip[3] = {0, 0, 0};
     if (mixed) {
@@ -2210,9 +2397,9 @@ void solve_depths(Ctx& c) {
         float* rOut = c.buf<float>("cg_rout", M);
         Comp2* partialC = c.buf<Comp2>("cg_partial_c", size_t(2) * (wg + wgM));
         if (rowForm) {
-            float3* state = c.buf<float3>("cg_state3", size_t(2) * M);
-            launch_kernel<cg_mixed_row_k>(&siteMixedRow, cg_mixed_row, wg, 0, s, true, P, o.neigh, val, c.fld.div,
-                                          c.fld.dx, rOut, state, slots, iters, resid, trueRel, err);
+            float4* state = c.buf<float4>("cg_state4", size_t(2) * M);
+            launch_kernel<cg_mixed_row_k>(&siteMixedRow, cg_mixed_row, wg, 0, s, true, P, maps, c.fld.div, c.fld.dx,
+                                          rOut, state, slots, iters, resid, trueRel, err);
         } else {
             // also the on-chip MINRES's two buffers of records
             float* rbuf = c.buf<float>("cg_rbuf", size_t(chip >= 0 ? 4 : 2) * M);
@@ -2240,8 +2427,8 @@ void solve_depths(Ctx& c) {
         }
     } else if (rowForm) {
         float2* state = c.buf<float2>("cg_state2", size_t(2) * M);
-        launch_kernel<cg_fp32_row_k>(&siteRow, cg_fp32_row, wg, 0, s, true, P, o.neigh, val, c.fld.div, c.fld.dx,
-                                     state, partial, ctl, iters, resid, err);
+        launch_kernel<cg_fp32_row_k>(&siteRow, cg_fp32_row, wg, 0, s, true, P, maps, c.fld.div, c.fld.dx, state, slots,
+                                     iters, resid, err);
     } else {
         float* r = c.buf<float>("cg_r", M);
         float* pA = c.buf<float>("cg_pa", M);
