@@ -275,12 +275,47 @@ __device__ __forceinline__ void points_chi_block(const PointsChiArgs& a, int blo
     }
 }
 
+// --- coarse divergence: the shares' fold -----------------------------------
+// Coarse nodes (few, each covering a large share of depth D): `parts`
+// workgroups each, every one summing a strided share of the node's terms; the
+// shares are folded in a fixed order, thread t of the fold node t's.
+constexpr int kMaxCoarse = 4;  // coarse depths 0..3
+struct CoarsePlan {
+    int depths;                      // coarse depths 0..depths-1
+    int blockStart[kMaxCoarse + 1];  // first workgroup (and partial) of each depth
+    int parts[kMaxCoarse];           // workgroups per node
+    int base[kMaxCoarse + 1];        // node range of each depth
+};
+struct DivFoldArgs {
+    CoarsePlan plan;
+    const double* partial;
+    float* div;
+};
+__device__ __forceinline__ void divergence_fold(const DivFoldArgs& a, int t) {
+    const CoarsePlan& P = a.plan;
+    if (t >= P.base[P.depths]) return;
+    int d = 0;
+    while (t >= P.base[d + 1]) ++d;
+    const int parts = P.parts[d];
+    const double* pp = a.partial + P.blockStart[d] + size_t(t - P.base[d]) * parts;
+    double s = 0;
+    for (int k = 0; k < parts; ++k) s += pp[k];
+    a.div[t] = float(s);
+}
+
 // --- operator (LaplacianSolver.cu:27-74) -----------------------------------
 // L(o, o') = <F,F>_x <F,F>_y <F,F>_z (<F',F'>_x + <F',F'>_y + <F',F'>_z) for the
 // same-depth neighbours o' of o; |L| <= 1e-6 is dropped (stored as 0); values
 // kept as float.  ELL layout [27][M] over all nodes; the column of slot i is
 // neigh[i][o] - base[depth].
 // Also counts the stored (nonzero) entries per depth into nnz (zeroed before).
+// On the regular grid an entry depends on the depth and the offset alone
+// (build_tables proves it of the tables at hand), so a row is 27 neighbour loads
+// and 27 stores; the entry per pair (a neighbour's index and twelve scattered
+// FP64 table values each) remains for the bent tables of the child 0 rule and for
+// tables it does not hold of.  The launch both share with the divergence: 200k
+// torus at depth 7 54 -> 50 us, 300k rotated torus at depth 8 176 -> 164 us, 32
+// clouds in one 1275 -> 1132 us.
 // Blocks of kAssembleThreads threads, launched beside the divergence's last
 // kernel (they need only the octree and the tables).
 constexpr int kAssembleThreads = 256;
@@ -295,7 +330,14 @@ struct AssembleArgs {
     float* val;
     int* nnz;        // per depth; the slot masks follow the CG error flag after it
     unsigned* slots;
+    const float* weights;  // [depth][27] entries by offset, or null
+    const int* q1Fired;    // the neighbour tables are not the regular grid's
 };
+// The operator's entry from the two functions' inner products per axis.
+__host__ __device__ __forceinline__ float operator_entry(double dx, double dy, double dz, double ex, double ey, double ez) {
+    const double e = dx * dy * dz * (ex + ey + ez);
+    return fabs(e) > double(1e-6f) ? float(e) : 0.f;
+}
 __device__ __forceinline__ void assemble_rows(const AssembleArgs& a, int block) {
     const Levels& L = a.L;
     const int M = a.M, res = a.res;
@@ -317,22 +359,36 @@ __device__ __forceinline__ void assemble_rows(const AssembleArgs& a, int block) 
     unsigned bits = 0u;
     if (valid) {
         const int j = t / M, o = t - j * M;
-        const int3 f1 = decode_func_index(enc[o], L.D);
-#pragma unroll 3
-        for (int i = 9 * j; i < 9 * j + 9; ++i) {
-            const int nb = neigh[i * M + o];
-            float v = 0.f;
-            if (nb != -1) {
-                const int3 f2 = decode_func_index(enc[nb], L.D);
-                size_t sx = size_t(f1.x) * res + f2.x, sy = size_t(f1.y) * res + f2.y, sz = size_t(f1.z) * res + f2.z;
-                double e = dot[sx] * dot[sy] * dot[sz] * (d2dot[sx] + d2dot[sy] + d2dot[sz]);
-                if (fabs(e) > double(1e-6f)) v = float(e);
-            }
-            val[i * M + o] = v;
-            c += v != 0.f;
-            bits |= v != 0.f ? 1u << i : 0u;
-        }
         d = depth_of(L, o);
+        if (a.weights && *a.q1Fired == 0) {
+            // on the regular grid an entry is its slot's constant: no table reads
+            int nb[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) nb[k] = neigh[(9 * j + k) * M + o];
+            const float* w = a.weights + 27 * d + 9 * j;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) {
+                const float v = nb[k] != -1 ? w[k] : 0.f;
+                val[(9 * j + k) * M + o] = v;
+                c += v != 0.f;
+                bits |= v != 0.f ? 1u << (9 * j + k) : 0u;
+            }
+        } else {
+            const int3 f1 = decode_func_index(enc[o], L.D);
+#pragma unroll 3
+            for (int i = 9 * j; i < 9 * j + 9; ++i) {
+                const int nb = neigh[i * M + o];
+                float v = 0.f;
+                if (nb != -1) {
+                    const int3 f2 = decode_func_index(enc[nb], L.D);
+                    size_t sx = size_t(f1.x) * res + f2.x, sy = size_t(f1.y) * res + f2.y, sz = size_t(f1.z) * res + f2.z;
+                    v = operator_entry(dot[sx], dot[sy], dot[sz], d2dot[sx], d2dot[sy], d2dot[sz]);
+                }
+                val[i * M + o] = v;
+                c += v != 0.f;
+                bits |= v != 0.f ? 1u << i : 0u;
+            }
+        }
     }
     // stored entries per depth: one LDS add per depth present in the wave
     unsigned long long active = __ballot(valid);

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 namespace psr {
 
@@ -83,6 +84,19 @@ __global__ void __launch_bounds__(256) build_tables_kernel(int res, double* __re
     dot[t] = r0;
     ddot[t] = r1;
     d2dot[t] = r2;
+}
+
+// band[k * res + f] = (dot, d2dot) of functions f and f + k - 1, where both
+// belong to one depth.
+__global__ void __launch_bounds__(256) gather_band(int res, int D, const double* __restrict__ dot,
+                                                   const double* __restrict__ d2dot, double2* __restrict__ band) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= 3 * res) return;
+    const int k = t / res, f = t - k * res, g = f + k - 1;
+    const int d = 31 - __clz(f + 1);
+    const bool in = g >= (1 << d) - 1 && g < (2 << d) - 1;
+    const size_t at = size_t(f) * res + size_t(in ? g : f);
+    band[t] = in ? make_double2(dot[at], d2dot[at]) : make_double2(0.0, 0.0);
 }
 
 // Concatenated ranges of the 27 neighbours of a node, held in LDS per wave.
@@ -269,17 +283,8 @@ __device__ __forceinline__ void divergence_fine_body(int psr_bid, int psr_nbid,
 }
 
 
-// Coarse nodes (few, each covering a large share of depth D): `parts`
-// workgroups each, every one summing a strided share of the node's terms; the
-// shares are folded in a fixed order by divergence_fold.
+// A coarse node's share of workgroup `part` (CoarsePlan; folded by divergence_fold).
 constexpr int kDivCoarseThreads = 256;
-constexpr int kMaxCoarse = 4;  // coarse depths 0..3
-struct CoarsePlan {
-    int depths;                      // coarse depths 0..depths-1
-    int blockStart[kMaxCoarse + 1];  // first workgroup (and partial) of each depth
-    int parts[kMaxCoarse];           // workgroups per node
-    int base[kMaxCoarse + 1];        // node range of each depth
-};
 template <class FieldT>
 __device__ __forceinline__ void divergence_coarse_body(int psr_bid, int psr_nbid, 
     const CoarsePlan& P, int M, int offD, int nD, int res, int D, const int* __restrict__ neigh,
@@ -401,26 +406,6 @@ struct divergence_all_k {
     __device__ __forceinline__ static void run(int bid, int nbid, const A&... a) { divergence_all_body<FieldT>(bid, nbid, a...); }
 };
 
-// The coarse nodes' divergence: thread t folds node t's shares, in order.
-__device__ __forceinline__ void divergence_fold_body(int psr_bid, int psr_nbid, const CoarsePlan& P,
-                                                     const double* __restrict__ partial, float* __restrict__ div) {
-    const int t = psr_bid * 256 + threadIdx.x;
-    if (t >= P.base[P.depths]) return;
-    int d = 0;
-    while (t >= P.base[d + 1]) ++d;
-    const int parts = P.parts[d];
-    const double* pp = partial + P.blockStart[d] + size_t(t - P.base[d]) * parts;
-    double s = 0;
-    for (int k = 0; k < parts; ++k) s += pp[k];
-    div[t] = float(s);
-}
-__global__ void __launch_bounds__(256) divergence_fold(CoarsePlan P, const double* __restrict__ partial,
-                                                       float* __restrict__ div) {
-    divergence_fold_body(blockIdx.x, gridDim.x, P, partial, div);
-}
-PSR_BATCHABLE(divergence_fold, 256)
-
-
 }  // namespace
 
 void build_tables(Ctx& c) {
@@ -434,6 +419,49 @@ void build_tables(Ctx& c) {
     t.d2dot = c.buf<double>("table_d2dot", n);
     build_tables_kernel<<<div_up(n, 256), 256, 0, c.stream>>>(res, t.dot, t.ddot, t.d2dot);
     PSR_HIP_CHECK(hipGetLastError());
+    // The inner products of each depth's functions with those at offsets -1, 0
+    // and 1 (a depth's functions are consecutive), copied out in one piece.
+    const int functions = res;  // of all depths
+    double2* band = c.buf<double2>("table_band", size_t(3) * functions);
+    gather_band<<<div_up(size_t(3) * functions, 256), 256, 0, c.stream>>>(res, D, t.dot, t.d2dot, band);
+    std::vector<double2> hb(size_t(3) * functions);
+    PSR_HIP_CHECK(hipMemcpyAsync(hb.data(), band, sizeof(double2) * hb.size(), hipMemcpyDeviceToHost, c.stream));
+    PSR_HIP_CHECK(hipStreamSynchronize(c.stream));
+    // The operator's entry of every depth and offset: the inner products at one
+    // offset differ from function to function in their last bits only, and the
+    // entry rounds to one float for every triple of them or the depth has no
+    // table of entries.
+    std::vector<float> weights(27 * size_t(D + 1), 0.f);
+    bool unique = true;
+    for (int d = 0; d <= D; ++d) {
+        std::vector<double2> distinct[3];
+        for (int k = 0; k < 3; ++k) {
+            for (int f = (1 << d) - 1; f < (2 << d) - 1; ++f) {
+                const int g = f + k - 1;
+                if (g < (1 << d) - 1 || g >= (2 << d) - 1) continue;
+                const double2 v = hb[size_t(k) * functions + f];
+                bool seen = false;
+                for (const double2& q : distinct[k]) seen = seen || (q.x == v.x && q.y == v.y);
+                if (!seen) distinct[k].push_back(v);
+            }
+        }
+        for (int q = 0; q < 27; ++q) {
+            bool first = true;
+            for (const double2& x : distinct[q / 9])
+                for (const double2& y : distinct[(q / 3) % 3])
+                    for (const double2& z : distinct[q % 3]) {
+                        const float e = operator_entry(x.x, y.x, z.x, x.y, y.y, z.y);
+                        if (first) weights[27 * size_t(d) + q] = e;
+                        else unique = unique && e == weights[27 * size_t(d) + q];
+                        first = false;
+                    }
+        }
+    }
+    if (unique) {
+        t.weights = c.buf<float>("table_weights", weights.size());
+        PSR_HIP_CHECK(hipMemcpyAsync(t.weights, weights.data(), sizeof(float) * weights.size(), hipMemcpyHostToDevice, c.stream));
+        PSR_HIP_CHECK(hipStreamSynchronize(c.stream));
+    }
     // Which depths' operators are indefinite once entries with |L| <= 1e-6 are
     // dropped (LaplacianSolver.cu:62).  An entry depends only on the neighbour
     // offset (the inner products are shift-invariant inside the domain), so a
@@ -446,11 +474,9 @@ void build_tables(Ctx& c) {
         const int f = (1 << d) - 1 + (1 << (d - 1));  // an interior function of depth d
         double dt[2], d2[2];
         for (int k = 0; k < 2; ++k) {
-            const size_t at = size_t(f) * res + size_t(f + k);
-            PSR_HIP_CHECK(hipMemcpyAsync(&dt[k], t.dot + at, sizeof(double), hipMemcpyDeviceToHost, c.stream));
-            PSR_HIP_CHECK(hipMemcpyAsync(&d2[k], t.d2dot + at, sizeof(double), hipMemcpyDeviceToHost, c.stream));
+            dt[k] = hb[size_t(1 + k) * functions + f].x;
+            d2[k] = hb[size_t(1 + k) * functions + f].y;
         }
-        PSR_HIP_CHECK(hipStreamSynchronize(c.stream));
         double L[2][2][2];  // by |offset| per axis
         for (int a = 0; a < 2; ++a)
             for (int b = 0; b < 2; ++b)
@@ -510,17 +536,18 @@ void field_stages(Ctx& c, FieldT* vf) {
         partial = c.buf<double>("div_partial", blocks);
     }
     // every depth's divergence and the operator's assembly (it needs only the
-    // octree and the tables) in one launch, then the coarse shares' fold
+    // octree and the tables) in one launch
     const int midCount = std::max(offD - coarseCount, 0);
     const DivRoles R{P.blockStart[kCoarse + 1], int(div_up(midCount, kDivWaves)), int(div_up(nD, 256))};
     const AssembleArgs aa{L,     M,     o.neigh, o.encIdx, c.tables.dot, c.tables.d2dot, c.tables.res,
-                          c.buf<float>("lap_val", size_t(27) * M), c.results()->cgNnz, c.results()->cgSlotMask};
+                          c.buf<float>("lap_val", size_t(27) * M), c.results()->cgNnz, c.results()->cgSlotMask,
+                          c.tables.weights, o.q1Fired};
     const int assembleBlocks = int(div_up(size_t(3) * M, kAssembleThreads));
     PSR_LAUNCH_K(divergence_all<FieldT>, divergence_all_k<FieldT>,
                  R.coarseBlocks + R.midBlocks + R.leafBlocks + assembleBlocks, 0, s, P, R, coarseCount, midCount, M,
                  offD, nD, c.tables.res, D, o.neigh, o.didx, o.dnum, o.encIdx, vf, c.tables.ddot, partial, c.fld.div,
                  aa);
-    PSR_LAUNCH(divergence_fold, div_up(coarseCount, 256), 0, s, P, partial, c.fld.div);
+    c.fld.foldArgs = DivFoldArgs{P, partial, c.fld.div};  // run by the solve's first kernel (solve_depths)
     PSR_HIP_CHECK(hipGetLastError());
 }
 

@@ -66,6 +66,10 @@ struct Tables {
     double* dot = nullptr;
     double* ddot = nullptr;
     double* d2dot = nullptr;
+    // The operator's entry per depth and neighbour slot, [depth][27], where every
+    // pair of functions at that offset gives the same float (checked over all of
+    // them when the tables are built); null where some depth has two values.
+    float* weights = nullptr;
 };
 
 // Point and node arrays of the octree (structure of arrays).
@@ -105,6 +109,7 @@ struct Field {
     float* dCol = nullptr;     // [27][M]: d_x of neighbour i of each node (0 where absent), 4 B a term
     double* isoSum = nullptr; // device scalar
     float iso = 0.f;
+    DivFoldArgs foldArgs{};   // the coarse nodes' divergence shares, folded by the solve's first kernel
     PointsChiArgs chiArgs{};  // the points' implicit values, launched with the mesh stage's first kernel
     int chiBlocks = 0;
 };

@@ -266,7 +266,7 @@ __device__ __forceinline__ void st_vec4(__amdgpu_buffer_rsrc_t r, int idx, float
 // 107 us mixed, 582 -> 293 us FP32 (whose two sums per iteration went through
 // an arrival counter); ellipsoid at depth 8 (263k rows, several rows a thread
 // before) 638 -> 195 us and 1398 -> 458 us; sphere at depth 5 (7k rows) 327 ->
-// 209 us FP32.  Of these row_maps takes 13-30 us.
+// 209 us FP32.  Of these the maps take 14-30 us.
 constexpr int kRowThreads = 512, kRowWaves = kRowThreads / PSR_WAVE;
 // The sums' blocks: 256 rows, whatever the workgroup holds, so that they do not
 // depend on it.
@@ -294,15 +294,16 @@ struct RowHead {
 struct RowMapArgs {
     const int* neigh;
     const float* val;
+    const float* weights;  // the operator's entries by depth and slot on the regular grid, or null
     const int* q1Fired;
     unsigned* places;
     int* ghosts;
     RowHead* heads;
 };
 
-// The maps of the row form's workgroups, a workgroup each (a launch of its own:
-// inside the CG kernel the table costs registers that its sweeps then lack).
-// Every stored neighbour inside the workgroup gets its row's place.  Those
+// The maps of the row form's workgroups, a workgroup each (ahead of the CG
+// kernel: inside it the table costs registers that its sweeps then lack; beside
+// the coarse divergence's fold, which leaves the GPU idle).  Every stored neighbour inside the workgroup gets its row's place.  Those
 // outside (13% of the entries) are listed, shared out over the threads and
 // entered into a hash table, whose used positions are numbered and become the
 // ghosts' places.
@@ -323,15 +324,21 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0;
     const bool own = t < rows;
     const int i = r0 + min(t, rows - 1);
+    // on the regular grid an entry is its slot's constant where the neighbour exists
+    const bool regular = a.weights && *a.q1Fired == 0;
     float v[27];
     int j[27];
 #pragma unroll
-    for (int q = 0; q < 27; ++q) {
-        v[q] = a.val[size_t(q) * M + i];
-        j[q] = a.neigh[size_t(q) * M + i];
+    for (int q = 0; q < 27; ++q) j[q] = a.neigh[size_t(q) * M + i];
+    if (regular) {
+#pragma unroll
+        for (int q = 0; q < 27; ++q) v[q] = j[q] >= 0 ? a.weights[27 * G.depth + q] : 0.f;
+    } else {
+#pragma unroll
+        for (int q = 0; q < 27; ++q) v[q] = a.val[size_t(q) * M + i];
     }
     for (int k = t; k < kGhostTable; k += kRowThreads) key[k] = -1;
-    if (t < 27) weight[t] = 0u;
+    if (t < 27) weight[t] = regular ? __float_as_uint(a.weights[27 * G.depth + t]) : 0u;
     if (t == 0) entries = 0, ghosts = 0, slow = 0;
     __syncthreads();
     unsigned bad = 0u, outside = 0u, ghost = 0u;  // ghost: slots with a stored neighbour outside
@@ -339,7 +346,7 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     for (int q = 0; q < 27; ++q) {
         const int l = j[q] - r0;
         const bool inside = unsigned(l) < unsigned(rows), stored = own && v[q] != 0.f;
-        if (stored) weight[q] = __float_as_uint(v[q]);  // any row's
+        if (!regular && stored) weight[q] = __float_as_uint(v[q]);  // any row's
         if (q == 13) {
             if (own && (!stored || l != t)) bad = 1u;
             continue;
@@ -403,9 +410,11 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
         word = final_place(e) | final_place(e + 1) << 16;
         if (own && e < 24) a.places[size_t(e / 2) * M + i] = word;
     }
+    if (!regular) {
 #pragma unroll
-    for (int q = 0; q < 27; ++q)
-        if (own && v[q] != 0.f && __float_as_uint(v[q]) != weight[q]) bad = 1u;
+        for (int q = 0; q < 27; ++q)
+            if (own && v[q] != 0.f && __float_as_uint(v[q]) != weight[q]) bad = 1u;
+    }
     if (bad) slow = 1;
     __syncthreads();
     // readers of a row outside its workgroup: symmetric where the tables are regular
@@ -415,10 +424,22 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     if (t < 27) head.w[t] = __uint_as_float(weight[t]);
     if (t == 0) head.ghosts = overflow ? 0 : ghosts, head.slow = slow;
 }
-__global__ void __launch_bounds__(kRowThreads) row_maps(CgParams P, RowMapArgs a) {
-    row_maps_body(blockIdx.x, gridDim.x, P, a);
+// The solve's first kernel: the fold of the coarse nodes' divergence, and the
+// row form's maps (mapBlocks of them; none for the other forms) beside it.  Both
+// are chains of loads in a few workgroups, 4 and 13 us as a launch each on a small
+// cloud and 14 us together.  On the regular grid the maps leave the entries unread
+// (a row's are its slots' constants where the neighbour exists): a batch of 32
+// depth-7 clouds, whose maps and assembly this and assemble_rows shorten, 11.7 ->
+// 10.3 ms a call.
+__device__ __forceinline__ void solve_prepare_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& a,
+                                                   int mapBlocks, const DivFoldArgs& fold) {
+    if (psr_bid < mapBlocks) row_maps_body(psr_bid, psr_nbid, P, a);
+    else divergence_fold(fold, (psr_bid - mapBlocks) * kRowThreads + int(threadIdx.x));
 }
-PSR_BATCHABLE(row_maps, kRowThreads)
+__global__ void __launch_bounds__(kRowThreads) solve_prepare(CgParams P, RowMapArgs a, int mapBlocks, DivFoldArgs fold) {
+    solve_prepare_body(blockIdx.x, gridDim.x, P, a, mapBlocks, fold);
+}
+PSR_BATCHABLE(solve_prepare, kRowThreads)
 
 // A value that is the same in every lane, in scalar registers: the rows' state
 // needs the vector ones (a spilled one's reload would wait for the records'
@@ -2348,6 +2369,16 @@ void solve_depths(Ctx& c) {
     c.cgCtlWords = size_t(ctlWords);
     c.cgSlots = slots;
     c.cgSlotWords = slotWords;
+    RowMapArgs maps{o.neigh, val, c.tables.weights, o.q1Fired, nullptr, nullptr, nullptr};
+    if (rowForm) {
+        maps.places = c.buf<unsigned>("cg_places", size_t(13) * M);
+        maps.ghosts = c.buf<int>("cg_ghosts", size_t(kGhostMax) * wg);
+        maps.heads = c.buf<RowHead>("cg_heads", wg);
+    }
+    const CoarsePlan& coarse = c.fld.foldArgs.plan;
+    const int mapBlocks = rowForm ? wg : 0;
+    PSR_LAUNCH(solve_prepare, mapBlocks + int(div_up(coarse.base[coarse.depths], kRowThreads)), 0, s, P, maps, mapBlocks,
+               c.fld.foldArgs);
     // CG kernels of different contexts (streams) never compete for residency
     // while spinning in their group barriers: a launch is queued only once the
     // launches still in flight leave room for all its workgroups beside them
@@ -2382,13 +2413,6 @@ void solve_depths(Ctx& c) {
     if (rowForm) P.spinLimit = 1u << 22;
     if (chip >= 0) PM.spinLimit = 1u << 24;  // polls of about a microsecond; a batch's group may wait for the solves before it
     if (c.cgSpinLimit >= 0) P.spinLimit = PM.spinLimit = unsigned(c.cgSpinLimit);
-    RowMapArgs maps{o.neigh, val, o.q1Fired, nullptr, nullptr, nullptr};
-    if (rowForm) {
-        maps.places = c.buf<unsigned>("cg_places", size_t(13) * M);
-        maps.ghosts = c.buf<int>("cg_ghosts", size_t(kGhostMax) * wg);
-        maps.heads = c.buf<RowHead>("cg_heads", wg);
-        PSR_LAUNCH(row_maps, wg, 0, s, P, maps);
-    }
     static const char siteMixedRow = 0, siteMixedGen = 0, siteMinres = 0, siteRow = 0, siteGen = 0;
     static const char siteChip[3] = {0, 0, 0};
     if (mixed) {
