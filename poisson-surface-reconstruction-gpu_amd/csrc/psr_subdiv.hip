@@ -783,6 +783,218 @@ constexpr auto sub_corner_values_small = sub_corner_values<false, kSmallThreads>
 
 
 
+// --- tiles without a sign change -------------------------------------------
+// Nearly all one-root tiles hold no crossing (300k points at depth 8: 1.1k of
+// 35.8k; the roots are large empty leaves beside the surface), and of such a
+// tile nothing but the sign is ever read.  On the regular octree a bound decides
+// it: inside a root's cube every function of the root's list is one quadratic
+// per axis (its pieces meet at cell boundaries of its own, coarser depth), so
+// the list's sum is one triquadratic there, whose 27 Bernstein coefficients
+// (sub_setup) restricted to a box enclose it; a halo node adds at most d_x
+// times the largest value of its function over the box.  A tile is definite
+// when the bound, widened by kBoundMargin of the sum of the terms' magnitudes
+// (567 terms at most, summed one by one: 3.4e-5, the coefficients' own rounding
+// 4e-5 at most), excludes the iso value at every point of its box and of the
+// points one further inside the root's cube, whichever cell of the root owns
+// them.  A tile is left out (state = its sign) when it is definite and so are,
+// with its sign, the tiles of other roots of its set that touch it: then none of
+// its cells' edges crosses, and neither does an edge elsewhere that ends at a
+// point it owns, so that those points' sign stands for their value.  NaN and
+// infinities are never definite.
+// Corner values, classification and tile scan of the 300k cloud at depth 8 695
+// -> 242 us, of the 200k torus at depth 7 119 -> 76 us, of 32 clouds 2271 ->
+// 1127 us, the bounds included.  Below kBoundTilesMin tiles the GPU takes nearly
+// all of them at once and the bound is not taken: its launch costs more than the
+// tiles left out (a call with 284 tiles 523 us without and 538 with it, with 4282
+// tiles 650 and 630).  A batch has the tiles of all its clouds in one launch.
+constexpr float kBoundMargin = 2e-4f;
+constexpr int kPolyWords = 32;  // per root: 27 coefficients, x-major, and the sum of the list's |d_x|
+constexpr int kBoundTilesMin = 2048;
+
+// Coefficients of the root lists over the roots' cubes, a root per wave.
+struct RootPolyArgs {
+    int nRoots;  // the roots of one-root tiles (first in the list), or 0
+    const float4* basis;
+    const float* dx;
+    float* poly;
+};
+
+// Part of the bound: a box of cells [lc, lc + ext) of a root's cube.
+struct BoxBound {
+    int p0[3], p1[3], c0[3], c1[3];  // within the root's cube: the points and the owner cells they can have
+    float lo, hi;                    // the list's sum over them
+    __device__ __forceinline__ BoxBound(int3 lc, int3 ext, int side, float coef) {
+        const int lane = __lane_id(), me = min(lane, 26);
+        const int l3[3] = {lc.x, lc.y, lc.z}, e3[3] = {ext.x, ext.y, ext.z}, idx[3] = {me / 9, (me / 3) % 3, me % 3};
+        const int stride[3] = {9, 3, 1};
+        const float inv = 1.0f / float(side);
+        float c = coef;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            p0[a] = max(l3[a] - 1, 0);
+            p1[a] = min(l3[a] + e3[a] + 1, side);
+            c0[a] = max(l3[a] - 2, 0);
+            c1[a] = min(l3[a] + e3[a] + 1, side - 1);
+            // the coefficients of the restriction to [u, v] (blossom), axis by axis
+            const float u = float(p0[a]) * inv, v = float(p1[a]) * inv;
+            const float s = idx[a] == 2 ? v : u, r = idx[a] == 0 ? u : v;
+            const int at = me - stride[a] * idx[a];
+            c = (1.f - s) * (1.f - r) * __shfl(c, at, PSR_WAVE) +
+                ((1.f - s) * r + s * (1.f - r)) * __shfl(c, at + stride[a], PSR_WAVE) +
+                s * r * __shfl(c, at + 2 * stride[a], PSR_WAVE);
+        }
+        lo = hi = c;
+#pragma unroll
+        for (int off = PSR_WAVE / 2; off > 0; off >>= 1) {
+            lo = fminf(lo, __shfl_xor(lo, off, PSR_WAVE));
+            hi = fmaxf(hi, __shfl_xor(hi, off, PSR_WAVE));
+        }
+        // (fminf drops a NaN; a NaN or infinite coefficient shows in the magnitude)
+    }
+    // +-1 where the values less iso have that sign, mag the sum of the terms'
+    // magnitudes, [neg, pos] the halo's sum
+    __device__ __forceinline__ int sign(float iso, float mag, float neg, float pos) const {
+        if (!(pos - neg < 3e38f)) return 0;
+        const float m = kBoundMargin * (mag + fabsf(iso) + pos - neg);
+        return lo + neg - iso > m ? 1 : (hi + pos - iso < -m ? -1 : 0);
+    }
+    // The halo at the faces `faces` (bit mask): the cells next to the root's cube
+    // (at Rc) that an owner cell can reach, one layer per face and depth (an
+    // edge's cells once per face: counted twice, the bound only widens), each
+    // with its function's largest value over the box (2/3 for all of them
+    // saves 18 us of 72 there and costs 35 in the tiles it leaves open).
+    __device__ __forceinline__ void halo(const Grid& g, int rd, int3 root, unsigned faces, float& neg, float& pos) const {
+        const int lane = __lane_id(), D = g.D, sh = D - rd, side = 1 << sh;
+        const int Rc[3] = {root.x, root.y, root.z};
+        const float inv = 1.0f / float(1 << D);
+        neg = pos = 0.f;
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+            if (!((faces >> f) & 1u)) continue;
+            const int a = f >> 1, a1 = a == 0 ? 1 : 0, a2 = a == 2 ? 1 : 2;
+            // from depth D - k on the owner cells touch this face of the cube
+            const int far = (f & 1) ? c1[a] ^ (side - 1) : c0[a];
+            for (int k = far == 0 ? 0 : 32 - __builtin_clz(far); k < sh; ++k) {
+                const int l = D - k, lim = 1 << l;
+                const int layer = (Rc[a] << (sh - k)) + ((f & 1) ? side >> k : -1);
+                if (layer < 0 || layer >= lim) break;  // the domain's face
+                const float* grid = g.dxAt + ((size_t(1) << (3 * l)) - 1) / 7;
+                const int sa = a == 0 ? 2 * l : (a == 1 ? l : 0), s1 = a1 == 0 ? 2 * l : l, s2 = a2 == 1 ? l : 0;
+                const int b1 = (Rc[a1] << (sh - k)) + (c0[a1] >> k) - 1, m1 = (c1[a1] >> k) - (c0[a1] >> k) + 3;
+                const int b2 = (Rc[a2] << (sh - k)) + (c0[a2] >> k) - 1, m2 = (c1[a2] >> k) - (c0[a2] >> k) + 3;
+                const float r = __builtin_amdgcn_rcpf(float(m2));  // (i + 1/2) / m2 is 1/44 or more from a whole number
+                for (int i = lane; i < m1 * m2; i += PSR_WAVE) {
+                    const int q1 = int((float(i) + 0.5f) * r), q2 = i - q1 * m2;
+                    const int n1 = b1 + q1, n2 = b2 + q2;
+                    float d = 0.f;
+                    if (unsigned(n1) < unsigned(lim) && unsigned(n2) < unsigned(lim))
+                        d = grid[(unsigned(layer) << sa) | (unsigned(n1) << s1) | (unsigned(n2) << s2)];
+                    if (d == 0.f) continue;
+                    const int n[3] = {layer, n1, n2}, ax[3] = {a, a1, a2};
+                    const float w = 1.0f / float(lim);
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        // the point of the box nearest the function's centre
+                        const float ctr = (0.5f + float(n[e])) * w;
+                        const float x0 = float((Rc[ax[e]] << sh) + p0[ax[e]]) * inv,
+                                    x1 = float((Rc[ax[e]] << sh) + p1[ax[e]]) * inv;
+                        d *= bspline(fmaxf(fmaxf(x0 - ctr, ctr - x1), 0.f) * float(lim));
+                    }
+                    pos += d > 0.f ? d : 0.f;
+                    neg += d > 0.f ? 0.f : d;  // a NaN too
+                }
+            }
+        }
+#pragma unroll
+        for (int off = PSR_WAVE / 2; off > 0; off >>= 1) {
+            pos += __shfl_xor(pos, off, PSR_WAVE);
+            neg += __shfl_xor(neg, off, PSR_WAVE);
+        }
+    }
+};
+
+// The sign of every one-root tile's values, 0 where the bound leaves it open.  A
+// workgroup takes 8 tiles; in roots of 16 tiles or more these are one box of 8 x
+// 16 x 16 cells, bounded first as a whole, a face of its halo per wave, and tile
+// by tile only where that leaves it open (a tile per wave alone: 72 against 59
+// us on 300k points at depth 8).
+constexpr int kBoundTiles = 8;
+constexpr int kBoundThreads = kBoundTiles * PSR_WAVE;
+__device__ __forceinline__ void sub_bound_body(int psr_bid, int psr_nbid, const Grid& g, const Tile* __restrict__ tiles,
+                                               int nOne, const float* __restrict__ poly,
+                                               const float* __restrict__ iso, int* __restrict__ sign,
+                                               int* __restrict__ state, int4* __restrict__ tileCnt) {
+    __shared__ float2 part[6];
+    // (the wave's index in a scalar register: the geometry is scalar work)
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / PSR_WAVE), lane = __lane_id();
+    const int t = min(psr_bid * kBoundTiles + wave, nOne - 1);
+    const Tile T = tiles[t];
+    const SetDesc S = g.sets[T.set];
+    const int4 rc = g.rootCell[T.root];
+    const int3 Rc = make_int3(rc.x, rc.y, rc.z);
+    const int sh = g.D - S.rd, side = 1 << sh;
+    const float* pr = poly + size_t(kPolyWords) * T.root;
+    const float coef = pr[min(lane, 26)], mag = pr[27], isoV = *iso;
+    const int rel = (T.start - S.dEnum) & ((1 << (3 * sh)) - 1);  // first cell within the root
+    int s = 0;
+    if (sh >= 4) {  // the same for the whole block: sets of such roots come first, 16 tiles or more a root
+        const BoxBound b(demorton(rel & ~(kBoundTiles * kTile - 1), sh), make_int3(8, 16, 16), side, coef);
+        float neg = 0.f, pos = 0.f;
+        const bool open = b.sign(isoV, mag, 0.f, 0.f) == 0;
+        if (!open && wave < 6) {
+            b.halo(g, S.rd, Rc, 1u << wave, neg, pos);
+            if (lane == 0) part[wave] = make_float2(neg, pos);
+        }
+        __syncthreads();
+        if (!open) {
+            neg = pos = 0.f;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) neg += part[f].x, pos += part[f].y;
+            s = b.sign(isoV, mag, neg, pos);
+        }
+    }
+    if (s == 0) {
+        const BoxBound b(demorton(rel, sh), make_int3(4, 8, 8), side, coef);
+        if (b.sign(isoV, mag, 0.f, 0.f) != 0) {
+            float neg, pos;
+            b.halo(g, S.rd, Rc, 0x3Fu, neg, pos);
+            s = b.sign(isoV, mag, neg, pos);
+        }
+    }
+    if (lane == 0 && psr_bid * kBoundTiles + wave < nOne) {
+        const bool out = s != 0 && S.nr == 1;
+        sign[t] = s;
+        state[t] = out ? s : 0;  // of a set of several roots: sub_corner_values_grid
+        if (out) tileCnt[t] = make_int4(0, 0, 0, 0);
+    }
+}
+__global__ void __launch_bounds__(kBoundThreads) sub_bound(Grid g, const Tile* __restrict__ tiles, int nOne,
+                                                           const float* __restrict__ poly,
+                                                           const float* __restrict__ iso, int* __restrict__ sign,
+                                                           int* __restrict__ state, int4* __restrict__ tileCnt) {
+    sub_bound_body(blockIdx.x, gridDim.x, g, tiles, nOne, poly, iso, sign, state, tileCnt);
+}
+PSR_BATCHABLE(sub_bound, kBoundThreads)
+
+// Whether a definite tile of sign s of a set of several roots is left out: the
+// tiles of other roots that touch it, among the 26 around it (tiles lie on one
+// grid), have its sign (asked by a whole wave, a neighbour per lane).
+__device__ __forceinline__ bool tile_left_out(const Grid& g, const Tile& T, const SetDesc& S,
+                                              const int* __restrict__ sign, int s) {
+    const int sh = g.D - S.rd, i = min(__lane_id(), 26);
+    const int3 lc = demorton((T.start - S.dEnum) & ((1 << (3 * sh)) - 1), sh);
+    const int x = lc.x + 4 * (i / 9 - 1), y = lc.y + 8 * ((i / 3) % 3 - 1), z = lc.z + 8 * (i % 3 - 1);
+    const int ax = x >> sh, ay = y >> sh, az = z >> sh;  // the root's cube, relative to this one
+    const int cube = nbr_index(ax, ay, az);
+    bool differs = false;
+    if (cube != 13 && ((g.rootSet[T.root] >> cube) & 1u)) {
+        const int q = g.rootNbr[27 * size_t(T.root) + cube] - S.rootOffset;
+        const int cell = (q << (3 * sh)) + morton(make_int3(x - (ax << sh), y - (ay << sh), z - (az << sh)), sh);
+        differs = sign[S.firstTile + cell / kTile] != s;
+    }
+    return __ballot(differs) == 0;
+}
+
 // Quotient by a small divisor through a multiply: exact for u * d < 2^32.
 struct SmallDiv {
     unsigned m;
@@ -809,10 +1021,12 @@ constexpr int kHaloPerThread = 4;     // halo entries per thread (<= 1024 for de
 // faster than at 5 (82 registers).  The batched form, which would spill 25
 // there, keeps the compiler's choice (the same batch time).
 constexpr int kCornerGridWaves = 7;
-__device__ __forceinline__ void sub_corner_values_grid_body(int psr_bid, int psr_nbid, const Grid& g, const Tile* __restrict__ tiles, int nVD,
-                                                                   const float* __restrict__ iso,
-                                                                   float* __restrict__ cval,
-                                                                   unsigned* __restrict__ ptOwner) {
+__device__ __forceinline__ void sub_corner_values_grid_body(int psr_bid, int psr_nbid, const Grid& g,
+                                                            const Tile* __restrict__ tiles, int nVD,
+                                                            const float* __restrict__ iso, float* __restrict__ cval,
+                                                            unsigned* __restrict__ ptOwner,
+                                                            const int* __restrict__ sign, int* __restrict__ state,
+                                                            int4* __restrict__ tileCnt) {
     extern __shared__ float4 ldsDyn[];  // grid_tile_words(D, rd) words
     __shared__ unsigned short lItem[kThreads * 8];  // owned (cell << 3 | corner), cell order
     __shared__ int lNbr[27];
@@ -821,7 +1035,18 @@ __device__ __forceinline__ void sub_corner_values_grid_body(int psr_bid, int psr
     __shared__ unsigned lSet;
     __shared__ unsigned lNz;  // bit l: some halo d_x of depth l is nonzero
     float* lds = reinterpret_cast<float*>(ldsDyn);
+    if (state && state[psr_bid] != 0) return;
     const Tile T = tiles[psr_bid];
+    if (state) {
+        const int s = sign[psr_bid];
+        if (s != 0 && tile_left_out(g, T, g.sets[T.set], sign, s)) {  // the same in every wave
+            if (threadIdx.x == 0) {
+                state[psr_bid] = s;
+                tileCnt[psr_bid] = make_int4(0, 0, 0, 0);
+            }
+            return;
+        }
+    }
     if (threadIdx.x < 27) lNbr[threadIdx.x] = g.rootNbr[27 * size_t(T.root) + threadIdx.x];
     if (threadIdx.x == 32) lSet = g.rootSet[T.root];
     if (threadIdx.x == 33) lNz = 0u;
@@ -945,9 +1170,8 @@ __device__ __forceinline__ void sub_corner_values_grid_body(int psr_bid, int psr
             const int3 p = make_int3(lo.x + pt / (kTy * kTz), lo.y + (pt / kTz) % kTy, lo.z + pt % kTz);
             int slot;
             const int e = owner_of_point(F, p, slot, ve);
-            // every point's value index, for sub_classify (when it has the map)
-            if (ptOwner)
-                ptOwner[size_t(psr_bid) * kPoints + pt] = e >= 0 ? unsigned(slot) * unsigned(nVD) + unsigned(e) : ~0u;
+            // every point's owner, for sub_classify (a set has less than 2^31 / 12 cells)
+            ptOwner[size_t(psr_bid) * kPoints + pt] = e >= 0 ? (unsigned(e) << 3) | unsigned(slot) : ~0u;
             if (e >= T.start && e < T.start + T.count) {
                 item[j] = ((e - T.start) << 3) | slot;
                 ++nOwn;
@@ -1008,11 +1232,11 @@ __device__ __forceinline__ void sub_corner_values_grid_body(int psr_bid, int psr
         cval[size_t(b) * nVD + e] = val - isoV;
     }
 }
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kCornerGridWaves))) sub_corner_values_grid(Grid g, const Tile* __restrict__ tiles, int nVD,
-                                                                   const float* __restrict__ iso,
-                                                                   float* __restrict__ cval,
-                                                                   unsigned* __restrict__ ptOwner) {
-    sub_corner_values_grid_body(blockIdx.x, gridDim.x, g, tiles, nVD, iso, cval, ptOwner);
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kCornerGridWaves)))
+    sub_corner_values_grid(Grid g, const Tile* __restrict__ tiles, int nVD, const float* __restrict__ iso,
+                           float* __restrict__ cval, unsigned* __restrict__ ptOwner, const int* __restrict__ sign,
+                           int* __restrict__ state, int4* __restrict__ tileCnt) {
+    sub_corner_values_grid_body(blockIdx.x, gridDim.x, g, tiles, nVD, iso, cval, ptOwner, sign, state, tileCnt);
 }
 PSR_BATCHABLE(sub_corner_values_grid, kThreads)
 
@@ -1239,7 +1463,8 @@ __device__ __forceinline__ void sub_classify_body(int psr_bid, int psr_nbid, con
                                                          const float* __restrict__ cval, float* __restrict__ vals,
                                                          unsigned* __restrict__ cellWord,
                                                          int* __restrict__ crossPrefix, int4* __restrict__ tileCnt,
-                                                         const unsigned* __restrict__ ptOwner, int nMapped) {
+                                                         const unsigned* __restrict__ ptOwner, int nMapped,
+                                                         const int* __restrict__ state) {
     __shared__ TileRoot lRoots[kMaxRootsPerTile];
     __shared__ int lNbr[kMaxRootsPerTile * 27];
     __shared__ unsigned lSet[kMaxRootsPerTile];
@@ -1247,6 +1472,7 @@ __device__ __forceinline__ void sub_classify_body(int psr_bid, int psr_nbid, con
     __shared__ float lVal[kClassifyPoints];
     __shared__ unsigned short lItem[kThreads * 12];  // crossing edges as (cell << 4 | edge), cell order
     __shared__ unsigned lOwn[kThreads];              // per cell: owned crossing edges, kept ones << 12
+    if (psr_bid < nMapped && state && state[psr_bid] != 0) return;  // left out: its counts are 0
     const Tile T = tiles[psr_bid];
     const SetDesc S = g.sets[T.set];
     const int D = g.D;
@@ -1262,8 +1488,17 @@ __device__ __forceinline__ void sub_classify_body(int psr_bid, int psr_nbid, con
     const int ex = tg.ext.x + 1, ey = tg.ext.y + 1, ez = tg.ext.z + 1, PP = ex * ey * ez;
     if (psr_bid < nMapped) {
         for (int t = threadIdx.x; t < kTilePoints; t += kThreads) {
-            const unsigned oi = ptOwner[size_t(psr_bid) * kTilePoints + t];
-            lVal[t] = oi != ~0u ? cval[oi] : 0.f;
+            const unsigned o = ptOwner[size_t(psr_bid) * kTilePoints + t];
+            const int e = int(o >> 3);
+            float v = 0.f;
+            if (o != ~0u) {
+                // a point of a tile that is left out: its sign
+                const int st = !state || (e >= T.start && e < T.start + T.count)
+                                   ? 0
+                                   : state[S.firstTile + (e - S.dEnum) / kTile];
+                v = st != 0 ? float(st) : cval[size_t(o & 7u) * nVD + e];
+            }
+            lVal[t] = v;
         }
     } else
     for (int t = threadIdx.x; t < tg.nRoots * PP; t += kThreads) {
@@ -1346,94 +1581,46 @@ __global__ void __launch_bounds__(kThreads) sub_classify(Grid g, const Tile* __r
                                                          const float* __restrict__ cval, float* __restrict__ vals,
                                                          unsigned* __restrict__ cellWord,
                                                          int* __restrict__ crossPrefix, int4* __restrict__ tileCnt,
-                                                         const unsigned* __restrict__ ptOwner, int nMapped) {
-    sub_classify_body(blockIdx.x, gridDim.x, g, tiles, nVD, cval, vals, cellWord, crossPrefix, tileCnt, ptOwner, nMapped);
+                                                         const unsigned* __restrict__ ptOwner, int nMapped,
+                                                         const int* __restrict__ state) {
+    sub_classify_body(blockIdx.x, gridDim.x, g, tiles, nVD, cval, vals, cellWord, crossPrefix, tileCnt, ptOwner, nMapped, state);
 }
 PSR_BATCHABLE(sub_classify, kThreads)
 
 
-// Exclusive scan of the per-tile counts in one workgroup; totals[0..2] are the
-// chunk's crossings, kept vertices and triangles; totals[3] = *keptMain, the
-// vertices kept by the depth-D batch.
-constexpr int kScanThreads = 1024;
+// Exclusive scan of the per-tile counts, kScanPer tiles a thread, the workgroups'
+// prefixes by look-back (in one workgroup, 36k tiles took 83 us); totals[0..2] are
+// the chunk's crossings, kept vertices and triangles (written by the tickets);
+// totals[3] = *keptMain, the vertices kept by the depth-D batch.
+constexpr int kScanThreads = 256;
+constexpr int kScanPer = 4;
 __device__ __forceinline__ void sub_tile_scan_body(int psr_bid, int psr_nbid, const int4* __restrict__ cnt, int n,
-                                                              int4* __restrict__ base, const int* __restrict__ keptMain,
-                                                              int* __restrict__ totals) {
-    constexpr int kW = kScanThreads / PSR_WAVE;
-    __shared__ int3 lSum3[kW];
-    const int per = (n + kScanThreads - 1) / kScanThreads;
-    const int i0 = min(n, int(threadIdx.x) * per), i1 = min(n, i0 + per);
-    // up to kPerMax counts a thread are held in registers, read at once
-    constexpr int kPerMax = 8;
-    const bool held = per <= kPerMax;
-    int4 v[kPerMax];
+                                                   const ScanTicket& ta, const ScanTicket& tb, const ScanTicket& tc,
+                                                   int4* __restrict__ base, const int* __restrict__ keptMain,
+                                                   int* __restrict__ totals) {
+    const int block = ticket_tile(ta);
+    const int i0 = (block * kScanThreads + int(threadIdx.x)) * kScanPer;
+    int4 v[kScanPer];
     int a = 0, b = 0, c = 0;
-    if (held) {
 #pragma unroll
-        for (int k = 0; k < kPerMax; ++k) v[k] = i0 + k < i1 ? cnt[i0 + k] : make_int4(0, 0, 0, 0);
+    for (int k = 0; k < kScanPer; ++k) v[k] = i0 + k < n ? cnt[i0 + k] : make_int4(0, 0, 0, 0);
 #pragma unroll
-        for (int k = 0; k < kPerMax; ++k) {
-            a += v[k].x;
-            b += v[k].y;
-            c += v[k].z;
-        }
-    } else {
-        for (int i = i0; i < i1; ++i) {
-            const int4 t = cnt[i];
-            a += t.x;
-            b += t.y;
-            c += t.z;
-        }
-    }
-    // the three exclusive scans in one pass over the block (one barrier pair)
-    const int lane = __lane_id(), w = threadIdx.x / PSR_WAVE;
-    int xa = a, xb = b, xc = c;
+    for (int k = 0; k < kScanPer; ++k) a += v[k].x, b += v[k].y, c += v[k].z;
+    ticket_prefix3<kScanThreads>(ta, tb, tc, block, a, b, c, a, b, c);
 #pragma unroll
-    for (int o = 1; o < PSR_WAVE; o <<= 1) {
-        const int ya = __shfl_up(xa, o, PSR_WAVE), yb = __shfl_up(xb, o, PSR_WAVE), yc = __shfl_up(xc, o, PSR_WAVE);
-        if (lane >= o) xa += ya, xb += yb, xc += yc;
+    for (int k = 0; k < kScanPer; ++k) {
+        if (i0 + k < n) base[i0 + k] = make_int4(a, b, c, 0);
+        a += v[k].x;
+        b += v[k].y;
+        c += v[k].z;
     }
-    if (lane == PSR_WAVE - 1) lSum3[w] = make_int3(xa, xb, xc);
-    __syncthreads();
-    int ta = 0, tb = 0, tc = 0, pa = 0, pb = 0, pc = 0;
-#pragma unroll
-    for (int k = 0; k < kW; ++k) {
-        const int3 t = lSum3[k];
-        if (k < w) pa += t.x, pb += t.y, pc += t.z;
-        ta += t.x, tb += t.y, tc += t.z;
-    }
-    a = pa + xa - a;
-    b = pb + xb - b;
-    c = pc + xc - c;
-    if (held) {
-#pragma unroll
-        for (int k = 0; k < kPerMax; ++k) {
-            if (i0 + k >= i1) break;
-            base[i0 + k] = make_int4(a, b, c, 0);
-            a += v[k].x;
-            b += v[k].y;
-            c += v[k].z;
-        }
-    } else {
-        for (int i = i0; i < i1; ++i) {
-            const int4 t = cnt[i];
-            base[i] = make_int4(a, b, c, 0);
-            a += t.x;
-            b += t.y;
-            c += t.z;
-        }
-    }
-    if (threadIdx.x == 0) {
-        totals[0] = ta;
-        totals[1] = tb;
-        totals[2] = tc;
-        totals[3] = *keptMain;
-    }
+    if (block == 0 && threadIdx.x == 0) totals[3] = *keptMain;
 }
-__global__ void __launch_bounds__(kScanThreads) sub_tile_scan(const int4* __restrict__ cnt, int n,
-                                                              int4* __restrict__ base, const int* __restrict__ keptMain,
+__global__ void __launch_bounds__(kScanThreads) sub_tile_scan(const int4* __restrict__ cnt, int n, ScanTicket ta,
+                                                              ScanTicket tb, ScanTicket tc, int4* __restrict__ base,
+                                                              const int* __restrict__ keptMain,
                                                               int* __restrict__ totals) {
-    sub_tile_scan_body(blockIdx.x, gridDim.x, cnt, n, base, keptMain, totals);
+    sub_tile_scan_body(blockIdx.x, gridDim.x, cnt, n, ta, tb, tc, base, keptMain, totals);
 }
 PSR_BATCHABLE(sub_tile_scan, kScanThreads)
 
@@ -1586,6 +1773,55 @@ __device__ __forceinline__ void root_records(const RootRecArgs& a, int block) {
     }
 }
 
+__device__ __forceinline__ void root_polynomials(const RootRecArgs& ra, const RootPolyArgs& a, int block) {
+    const int q = block * (kThreads / PSR_WAVE) + int(threadIdx.x) / PSR_WAVE, lane = __lane_id();
+    if (q >= a.nRoots) return;
+    const Levels& Lv = ra.Lv;
+    const int root = ra.roots[q];
+    int rd = 0;
+    while (rd < Lv.D && root >= Lv.base[rd + 1]) ++rd;
+    // lane u of the wave keeps chain node u
+    int chain = -1, node = root;
+    for (int u = 0; u <= rd; ++u) {
+        if (lane == u) chain = node;
+        node = node < 0 ? -1 : ra.parent[node];
+    }
+    const int3 c = demorton(ra.key[root] >> (3 * (Lv.D - rd)), rd);
+    const float w = 1.0f / float(1 << rd), x0 = float(c.x) * w, y0 = float(c.y) * w, z0 = float(c.z) * w;
+    float acc[27] = {0.f};
+    float mag = 0.f;
+    const int K = 27 * (rd + 1);
+    for (int k0 = 0; k0 < K; k0 += PSR_WAVE) {
+        const int k = k0 + lane, u = min(k / 27, rd);
+        const int cn = __shfl(chain, u, PSR_WAVE);
+        const int nb = k < K && cn >= 0 ? ra.neigh[size_t(k % 27) * ra.M + cn] : -1;
+        if (nb < 0) continue;
+        const float4 b = a.basis[nb];
+        const float d = a.dx[nb], invw = float(1 << (rd - u));
+        // Bernstein coefficients per axis: the ends, and twice the middle less their mean
+        float f[3][3];
+        const float lo[3] = {x0, y0, z0}, ctr[3] = {b.x, b.y, b.z};
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            f[e][0] = bspline((lo[e] - ctr[e]) * invw);
+            f[e][2] = bspline((lo[e] + w - ctr[e]) * invw);
+            f[e][1] = 2.f * bspline((lo[e] + 0.5f * w - ctr[e]) * invw) - 0.5f * (f[e][0] + f[e][2]);
+        }
+#pragma unroll
+        for (int i = 0; i < 27; ++i) acc[i] += d * f[0][i / 9] * f[1][(i / 3) % 3] * f[2][i % 3];
+        mag += fabsf(d);
+    }
+    float mine = 0.f;
+#pragma unroll
+    for (int i = 0; i < 28; ++i) {
+        float v = i < 27 ? acc[i < 27 ? i : 0] : mag;
+#pragma unroll
+        for (int off = PSR_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PSR_WAVE);
+        if (lane == i) mine = v;
+    }
+    if (lane < 28) a.poly[size_t(kPolyWords) * q + lane] = mine;
+}
+
 // d_x of every node at its cell of the dense grid of its depth.
 __device__ __forceinline__ void scatter_dx_grid_body(int psr_bid, int psr_nbid, int M, const Levels& L, const int* __restrict__ key,
                                                             const float* __restrict__ dx, float* __restrict__ grid) {
@@ -1684,21 +1920,21 @@ __device__ __forceinline__ void make_tiles(const TileArgs& a, int block) {
 
 // The subdivision's set-up in one launch: blocks [0, keepBlocks) compact the
 // vertices kept by the depth-D batch, the next rootBlocks blocks write the
-// root records, the remaining blocks expand the tiles (parts blocks per set).
+// root records, the next polyBlocks the root lists' polynomials, the remaining
+// blocks expand the tiles (parts blocks per set).
 __device__ __forceinline__ void sub_setup_body(int psr_bid, int psr_nbid, const KeepArgs& ka, int keepBlocks, const RootRecArgs& ra, int rootBlocks,
-                                                      const TileArgs& ta) {
-    const int b = psr_bid;
-    if (b < keepBlocks) {
-        keep_compact(ka);
-    } else if (b < keepBlocks + rootBlocks) {
-        root_records(ra, b - keepBlocks);
-    } else {
-        make_tiles(ta, b - keepBlocks - rootBlocks);
-    }
+                                                      const RootPolyArgs& pa, int polyBlocks, const TileArgs& ta) {
+    int b = psr_bid;
+    if (b < keepBlocks) return keep_compact(ka);
+    b -= keepBlocks;
+    if (b < rootBlocks) return root_records(ra, b);
+    b -= rootBlocks;
+    if (b < polyBlocks) return root_polynomials(ra, pa, b);
+    make_tiles(ta, b - polyBlocks);
 }
 __global__ void __launch_bounds__(kThreads) sub_setup(KeepArgs ka, int keepBlocks, RootRecArgs ra, int rootBlocks,
-                                                      TileArgs ta) {
-    sub_setup_body(blockIdx.x, gridDim.x, ka, keepBlocks, ra, rootBlocks, ta);
+                                                      RootPolyArgs pa, int polyBlocks, TileArgs ta) {
+    sub_setup_body(blockIdx.x, gridDim.x, ka, keepBlocks, ra, rootBlocks, pa, polyBlocks, ta);
 }
 PSR_BATCHABLE(sub_setup, kThreads)
 
@@ -1805,7 +2041,8 @@ void extract_mesh_b(Ctx& c) {
     const int keepBlocks = std::max(1, int(div_up(mm.nCross, kThreads)));
     const KeepArgs ka{mainV, mainKey, mm.nCross,
                       scan_ticket(c.scan_for_tiles(size_t(keepBlocks)), keepBlocks, keptMain), outV, outKey};
-    if (nSets == 0) PSR_LAUNCH(sub_setup, keepBlocks, 0, st, ka, keepBlocks, RootRecArgs{}, 0, TileArgs{});
+    if (nSets == 0) PSR_LAUNCH(sub_setup, keepBlocks, 0, st, ka, keepBlocks, RootRecArgs{}, 0, RootPolyArgs{}, 0,
+                               TileArgs{});
     if (deferred && nSets > 0) outT = c.buf_keep<int>("mesh_triangles", 3 * tCap, 3 * size_t(mm.nTri));
     if (nSets > 0) {
         const int* rootPos = mm.rootPos;
@@ -1818,8 +2055,17 @@ void extract_mesh_b(Ctx& c) {
         const RootRecArgs ra{mm.nRoots, M,        L,       finerDepth, mm.roots, rootPos,  o.neigh,
                              o.parent,  o.key,    rootNbr, rootChain,  rootCell, rootSet};
         const int rootBlocks = int(div_up(size_t(27) * mm.nRoots, kThreads));
+        int nOneRoots = 0;  // roots of one-root tiles
+        for (int d = 0; d <= D - 3; ++d) nOneRoots += mm.rootsPerDepth[d];
         // tiles read d_x from dense per-depth grids when the octree is geometric
         const bool denseHalo = !mm.q1Fired;
+        // the roots' polynomials, where the tiles are bounded
+        size_t oneTiles = 0;
+        for (int k = 0; k < nSets; ++k)
+            if (D - sets[k].rd >= 3) oneTiles += setCells[k] / kTile;
+        float* rootPoly = denseHalo && oneTiles >= size_t(current_recorder() ? 1 : kBoundTilesMin)
+                              ? c.buf<float>("sub_root_poly", size_t(kPolyWords) * nOneRoots)
+                              : nullptr;
         for (const SetDesc& S : sets) {
             int halo = 0;
             if (denseHalo && D - S.rd >= 3 &&
@@ -1891,7 +2137,9 @@ void extract_mesh_b(Ctx& c) {
                                   D, parts, dsets, reinterpret_cast<Tile*>(dAll + bSets),
                                   reinterpret_cast<Tile*>(dAll + bSets + bTiles)};
                 const int kb = s0 == 0 ? keepBlocks : 0, rb = s0 == 0 ? rootBlocks : 0;
-                PSR_LAUNCH(sub_setup, unsigned(kb + rb + nCs * parts), 0, st, ka, kb, ra, rb, ta);
+                const int pb = s0 == 0 && rootPoly ? int(div_up(size_t(nOneRoots), kThreads / PSR_WAVE)) : 0;
+                const RootPolyArgs pa{nOneRoots, o.basis, c.fld.dx, rootPoly};
+                PSR_LAUNCH(sub_setup, unsigned(kb + rb + pb + nCs * parts), 0, st, ka, kb, ra, rb, pa, pb, ta);
             }
             Tile* dtiles = reinterpret_cast<Tile*>(dAll + bSets);
             Tile* dsmall = reinterpret_cast<Tile*>(dAll + bSets + bTiles);
@@ -1906,17 +2154,21 @@ void extract_mesh_b(Ctx& c) {
             // the one-root tiles' point owners, found by sub_corner_values_grid
             // and reused by sub_classify (value indices slot * nVD + cell fit 32 bits)
             unsigned* ptOwner = nullptr;
-            int nMapped = 0;
+            int* state = nullptr;
             if (nOne > 0 && denseHalo) {
                 int words = 0;
                 for (int k = 0; k < nCs; ++k)
                     if (D - cs[k].rd >= 3) words = std::max(words, grid_tile_words(D, cs[k].rd));
-                if (size_t(8) * size_t(nVD) <= size_t(UINT32_MAX)) {
-                    ptOwner = c.buf<unsigned>("sub_point_owner", size_t(nOne) * kTilePoints);
-                    nMapped = nOne;
+                ptOwner = c.buf<unsigned>("sub_point_owner", size_t(nOne) * kTilePoints);
+                int* sign = nullptr;
+                if (rootPoly) {
+                    sign = c.buf<int>("sub_tile_sign", nOne);
+                    state = c.buf<int>("sub_tile_state", nOne);
+                    PSR_LAUNCH(sub_bound, div_up(nOne, kBoundTiles), 0, st, gr, dtiles, nOne,
+                               static_cast<const float*>(rootPoly), isoDev, sign, state, tileCnt);
                 }
                 PSR_LAUNCH(sub_corner_values_grid, nOne, sizeof(float) * words, st, gr, dtiles, nVD, isoDev, cval,
-                           ptOwner);
+                           ptOwner, static_cast<const int*>(sign), state, tileCnt);
             }
             else if (nOne > 0)
                 PSR_LAUNCH_K(sub_corner_values_one, sub_corner_values_one_k, nOne, 0, st, gr, dtiles, nVD, isoDev, cval);
@@ -1930,9 +2182,19 @@ void extract_mesh_b(Ctx& c) {
                 PSR_LAUNCH_K(sub_corner_values_small, sub_corner_values_small_k, nSmall, 0, st, gr, dsmall, nVD, isoDev, cval);
             }
             PSR_LAUNCH(sub_classify, nTiles, 0, st, gr, dtiles, nVD, cval, vals, cellWord, crossPre, tileCnt,
-                       static_cast<const unsigned*>(ptOwner), nMapped);
-            // totals: slots 0-3
-            PSR_LAUNCH(sub_tile_scan, 1, 0, st, tileCnt, nTiles, tileBase, keptMain, c.mail);
+                       static_cast<const unsigned*>(ptOwner), ptOwner ? nOne : 0, static_cast<const int*>(state));
+            {
+                // totals: slots 0-3; three scans on one ticket epoch, a status array each
+                const int blocks = int(div_up(nTiles, kScanThreads * kScanPer));
+                ScanState& scan = c.scan_for_tiles(size_t(3) * blocks);
+                const ScanTicket ta = scan_ticket(scan, blocks, c.mail + 0);
+                ScanTicket tb = ta, tc = ta;
+                tb.status += blocks;
+                tc.status += 2 * blocks;
+                tb.total = c.mail + 1;
+                tc.total = c.mail + 2;
+                PSR_LAUNCH(sub_tile_scan, blocks, 0, st, tileCnt, nTiles, ta, tb, tc, tileBase, keptMain, c.mail);
+            }
             if (deferred) {
                 PSR_LAUNCH(sub_emit, nTiles, 0, st, gr, dtiles, nVD, vals, cellWord, crossPre, tileCnt, tileBase,
                                                       keptMain, 0, mm.nTri, outV, outT, outKey);

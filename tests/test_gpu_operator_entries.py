@@ -29,16 +29,20 @@ def _kept(rec, D):
     return [int(((rows >= base[d]) & (rows < base[d + 1])).sum()) for d in range(D + 1)]
 
 
-@pytest.mark.parametrize("cloud,depth", [("sphere", 2), ("pair", 3), ("sphere", 5), ("torus", 7), ("torus", 8)])
+@pytest.mark.parametrize("cloud,depth", [("sphere", 2), ("bent", 7), ("sphere", 5), ("torus", 7), ("torus", 8)])
 def test_entries(pkg, cloud, depth):
     import residual_host
     import torch
-    xyz, nrm = pkg.synth.torus(n=60000) if cloud == "torus" else pkg.synth.sphere(n=64 if cloud == "pair" else 4000)
+    if cloud == "bent":
+        xyz, nrm = pkg.synth.batch64()[36]
+    else:
+        xyz, nrm = pkg.synth.torus(n=60000) if cloud == "torus" else pkg.synth.sphere(n=4000)
     rec = pkg.PoissonReconstruction(depth=depth, precision=1)
     rec.SolvePoissionReconstructionMesh(torch.from_numpy(xyz).cuda(), torch.from_numpy(nrm).cuda())
     st, kept, rel = rec.stats(), _kept(rec, depth), residual_host.true_relres(rec, depth)
     rec.close()
     print(cloud, depth, "q1", st["q1_fired"], "kept", kept, "relres", rel, flush=True)
+    assert st["q1_fired"] == (cloud == "bent")
     assert list(st["cg_nnz"])[:depth + 1] == kept
     rep = np.array(st["cg_true_relres"])[:depth + 1]
     assert np.all(np.abs(rep - rel) <= 1e-3 * np.maximum(rep, 1e-6))
