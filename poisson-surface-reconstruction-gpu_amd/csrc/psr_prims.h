@@ -67,7 +67,10 @@ struct SortGather {
 // Stable ascending sort of keys (only the low `bits` bits are examined) carrying
 // values.  The sorted data ends in (keys, vals): the four buffers are swapped
 // in place of a final copy, so keys/vals may come back as the former ktmp/vtmp.
+// src: the keys are read from there and the values are their positions (keys and
+// vals need not hold them), or null.
 void radix_sort_pairs(unsigned*& keys, unsigned*& vals, unsigned*& ktmp, unsigned*& vtmp, int n, int bits,
-                      int* scratch, bool firstHist, ScanState& st, const SortGather& g, hipStream_t s);
+                      int* scratch, bool firstHist, ScanState& st, const SortGather& g, hipStream_t s,
+                      const unsigned* src = nullptr);
 
 }  // namespace psr

@@ -159,7 +159,7 @@ __device__ __forceinline__ void radix_scatter_body(int psr_bid, int psr_nbid, co
         int i = base + it * kSortThreads + threadIdx.x;
         bool valid = i < n;
         unsigned key = valid ? kin[i] : 0u;
-        unsigned val = valid ? vin[i] : 0u;
+        unsigned val = valid && vin ? vin[i] : unsigned(i);  // no vin: the positions
         int d = int((key >> shift) & mask);
         unsigned long long peers = __ballot(valid);
 #pragma unroll
@@ -214,7 +214,8 @@ size_t sort_scratch_ints(size_t n) {
 }
 
 void radix_sort_pairs(unsigned*& keys, unsigned*& vals, unsigned*& ktmp, unsigned*& vtmp, int n, int bits,
-                      int* scratch, bool firstHist, ScanState& st, const SortGather& g, hipStream_t s) {
+                      int* scratch, bool firstHist, ScanState& st, const SortGather& g, hipStream_t s,
+                      const unsigned* src) {
     if (n <= 0) return;
     if (bits <= 0) return;
     int tiles = int(div_up(n, kSortTile));
@@ -224,10 +225,13 @@ void radix_sort_pairs(unsigned*& keys, unsigned*& vals, unsigned*& ktmp, unsigne
     for (int p = 0; p < passes; ++p) {
         const int shift = width * p, b = std::min(width, bits - shift);
         const unsigned mask = (1u << b) - 1u;
-        if (p > 0 || !firstHist) PSR_LAUNCH(radix_hist, tiles, 0, s, ka, n, shift, mask, tiles, hist);
+        const bool first = p == 0 && src;
+        const unsigned* kin = first ? src : ka;
+        const unsigned* vin = first ? nullptr : va;
+        if (p > 0 || !firstHist) PSR_LAUNCH(radix_hist, tiles, 0, s, kin, n, shift, mask, tiles, hist);
         scan_exclusive(hist, hist, int(mask + 1) * tiles, nullptr, st, s);
         const SortGather none{};
-        PSR_LAUNCH(radix_scatter, tiles, 0, s, ka, va, kb, vb, n, shift, mask, tiles, hist,
+        PSR_LAUNCH(radix_scatter, tiles, 0, s, kin, vin, kb, vb, n, shift, mask, tiles, hist,
                    p == passes - 1 ? g : none);
         std::swap(ka, kb);
         std::swap(va, vb);

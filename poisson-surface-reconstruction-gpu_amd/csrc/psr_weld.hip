@@ -6,14 +6,19 @@
 // own).  Every vertex of this build's mesh carries the global key of its
 // depth-D edge (segment_key); welding keeps one vertex per key:
 //   * (key, vertex) pairs sorted by key (stable: equal keys keep vertex order);
-//   * head flags where the key changes, their exclusive scan = welded index;
+//   * where the key changes a run begins, the runs before it = welded index;
 //   * the first vertex of each run (the lowest-numbered vertex on that edge)
 //     is kept, every vertex maps to its run's welded index, and triangle
 //     corners are remapped through that map.
+// Bound by its launches and the gaps between them (28k vertices are 100 KB): the
+// sort's first pass reads the mesh's keys in place, the keys' 23 bits at depth 7
+// take 3 passes where 32 took 4, and the runs are found, scanned and copied in
+// one launch, 11 launches where there were 17 (110 -> 86 us a call).
 // Welded vertices come out in ascending key order.
 #include "psr_internal.h"
 #include "psr_mesh_common.h"
 #include "psr_prims.h"
+#include "psr_tile_scan.h"
 
 #include <cstdio>
 #include <cstring>
@@ -29,34 +34,29 @@ constexpr int kThreads = 256;
 constexpr int kMailWeld = 44;  // mailbox slot of the welded vertex count
 static_assert(kMailWeld > kMailGeo + 2 && kMailWeld < kMailWords, "mailbox slot of the weld");
 
-__global__ void __launch_bounds__(kThreads) weld_init(const unsigned* __restrict__ key, int n,
-                                                      unsigned* __restrict__ k, unsigned* __restrict__ v) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    k[i] = key[i];
-    v[i] = unsigned(i);
-}
-
-__global__ void __launch_bounds__(kThreads) weld_heads(const unsigned* __restrict__ k, int n, int* __restrict__ head) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    head[i] = (i == 0 || k[i] != k[i - 1]) ? 1 : 0;
-}
-
-// Sorted position i: vertex v[i] maps to run grp[i] + head[i] - 1; a run's
-// first vertex is copied to it.
-__global__ void __launch_bounds__(kThreads) weld_vertices(const unsigned* __restrict__ v, const int* __restrict__ head,
-                                                          const int* __restrict__ grp, int n,
+// Sorted position i is a head where its key differs from the one before; the
+// heads' count before it (t: a scan over the launch's workgroups) is its run's
+// welded index.  Vertex v[i] maps to its run, whose first vertex is copied to it.
+__global__ void __launch_bounds__(kThreads) weld_vertices(const unsigned* __restrict__ k,
+                                                          const unsigned* __restrict__ v, int n, ScanTicket t,
                                                           const float* __restrict__ inV, int* __restrict__ remap,
                                                           float* __restrict__ outV) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
+    const int tile = ticket_tile(t), i = tile * kThreads + threadIdx.x;
+    const int h = i < n && (i == 0 || k[i] != k[i - 1]) ? 1 : 0;
+    const int src = i < n ? int(v[i]) : 0;
+    float x = 0.f, y = 0.f, z = 0.f;
+    if (h) {
+        x = inV[3 * size_t(src)];
+        y = inV[3 * size_t(src) + 1];
+        z = inV[3 * size_t(src) + 2];
+    }
+    const int g = ticket_prefix<kThreads>(t, tile, h) + h - 1;
     if (i >= n) return;
-    const int h = head[i], g = grp[i] + h - 1, src = int(v[i]);
     remap[src] = g;
     if (h) {
-        outV[3 * size_t(g)] = inV[3 * size_t(src)];
-        outV[3 * size_t(g) + 1] = inV[3 * size_t(src) + 1];
-        outV[3 * size_t(g) + 2] = inV[3 * size_t(src) + 2];
+        outV[3 * size_t(g)] = x;
+        outV[3 * size_t(g) + 1] = y;
+        outV[3 * size_t(g) + 2] = z;
     }
 }
 
@@ -264,18 +264,18 @@ void weld_mesh(Ctx& c) {
         unsigned* v = c.buf<unsigned>("weld_v", nv);
         unsigned* kt = c.buf<unsigned>("weld_kt", nv);
         unsigned* vt = c.buf<unsigned>("weld_vt", nv);
-        int* head = c.buf<int>("weld_head", nv);
-        int* grp = c.buf<int>("weld_grp", nv);
         int* remap = c.buf<int>("weld_remap", nv);
-        weld_init<<<div_up(nv, kThreads), kThreads, 0, s>>>(m.keys, nv, k, v);
+        // a key is below 3 (2^D + 1)^3 (segment_key)
+        const unsigned long long side = (1ull << c.cfg.depth) + 1, keyEnd = 3 * side * side * side;
+        int bits = 1;
+        while (bits < 32 && (keyEnd - 1) >> bits) ++bits;
         int* scratch = c.scratch_for(sort_scratch_ints(size_t(nv)));
-        radix_sort_pairs(k, v, kt, vt, nv, 32, scratch, false, c.scan_for(sort_scan_elems(size_t(nv))), SortGather{},
-                         s);
-        weld_heads<<<div_up(nv, kThreads), kThreads, 0, s>>>(k, nv, head);
+        radix_sort_pairs(k, v, kt, vt, nv, bits, scratch, false, c.scan_for(sort_scan_elems(size_t(nv))), SortGather{},
+                         s, m.keys);
         c.hostPinned[kMailWeld] = 0;
-        scan_exclusive(head, grp, nv, c.mail + kMailWeld, c.scan_for(size_t(nv)), s);
-        weld_vertices<<<div_up(nv, kThreads), kThreads, 0, s>>>(v, head, grp, nv, m.vertices, remap,
-                                                                m.weldedVertices);
+        const int tiles = int(div_up(nv, kThreads));
+        const ScanTicket t = scan_ticket(c.scan_for_tiles(size_t(tiles)), tiles, c.mail + kMailWeld);
+        weld_vertices<<<tiles, kThreads, 0, s>>>(k, v, nv, t, m.vertices, remap, m.weldedVertices);
         if (nt > 0)
             weld_triangles<<<div_up(size_t(3) * nt, kThreads), kThreads, 0, s>>>(m.triangles, size_t(3) * nt, nv,
                                                                                  remap, m.weldedTriangles);
