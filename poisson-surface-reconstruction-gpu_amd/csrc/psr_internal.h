@@ -251,12 +251,16 @@ struct Ctx {
     void clear_scan_error() { hostPinned[kMailScanErr] = 0; }
     bool scan_failed() const { return __atomic_load_n(&hostPinned[kMailScanErr], __ATOMIC_ACQUIRE) != 0; }
     // Waits for the stream by polling it: a blocking wait adds the host thread's
-    // wake-up latency to every read-back.  Errors surface through the final
-    // synchronisation.
+    // wake-up latency to every read-back.  The query that finds the stream empty
+    // is the wait: it says what a synchronisation would (every operation has
+    // completed, or the error of one that failed), and a synchronisation after it
+    // took 1 to 25 us (200k torus at depth 7, three waits: 676 -> 641 us a call;
+    // shorter calls the same).
     void wait() {
-        while (hipStreamQuery(stream) == hipErrorNotReady) {
+        hipError_t e;
+        while ((e = hipStreamQuery(stream)) == hipErrorNotReady) {
         }
-        PSR_HIP_CHECK(hipStreamSynchronize(stream));
+        PSR_HIP_CHECK(e);
     }
     // Pinned, mapped, coherent staging of at least `bytes` (device view in stageDev); only
     // reused after a stream synchronisation.
