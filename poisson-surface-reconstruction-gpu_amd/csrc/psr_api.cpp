@@ -463,18 +463,26 @@ int psr_export(psr_ctx* ctx, int id, void* dst, uint64_t bytes, uint64_t* needed
             if (needed) *needed = size_t(12) * nD;
             if (!dst) return PSR_OK;
             if (bytes < size_t(12) * nD) return PSR_ERR_CAPACITY;
-            std::vector<float> t(size_t(3) * nD);
-            if (c.fld.vhalf) {  // FP16 storage of V * 2^-(D+1)
-                std::vector<__half> h(size_t(3) * nD);
-                if (hipMemcpy(h.data(), c.fld.vhalf, 6 * size_t(nD), hipMemcpyDeviceToHost) != hipSuccess)
-                    return PSR_ERR_HIP;
-                for (size_t i = 0; i < h.size(); ++i) t[i] = __half2float(h[i]) * float(2 << D);
-            } else if (hipMemcpy(t.data(), c.fld.vfield, 12 * size_t(nD), hipMemcpyDeviceToHost) != hipSuccess) {
-                return PSR_ERR_HIP;
-            }
             float* out = static_cast<float*>(dst);
-            for (int i = 0; i < nD; ++i)
-                for (int a = 0; a < 3; ++a) out[3 * size_t(i) + a] = t[size_t(a) * nD + i];
+            if (c.fld.vhalf) {  // FP16 storage of V * 2^-(D+1)
+                std::vector<psr::FieldHalf> h(nD);
+                if (hipMemcpy(h.data(), c.fld.vhalf, sizeof(psr::FieldHalf) * size_t(nD), hipMemcpyDeviceToHost) != hipSuccess)
+                    return PSR_ERR_HIP;
+                for (size_t i = 0; i < h.size(); ++i) {
+                    out[3 * i] = __half2float(h[i].x) * float(2 << D);
+                    out[3 * i + 1] = __half2float(h[i].y) * float(2 << D);
+                    out[3 * i + 2] = __half2float(h[i].z) * float(2 << D);
+                }
+                return PSR_OK;
+            }
+            std::vector<float4> t(nD);
+            if (hipMemcpy(t.data(), c.fld.vfield, sizeof(float4) * size_t(nD), hipMemcpyDeviceToHost) != hipSuccess)
+                return PSR_ERR_HIP;
+            for (size_t i = 0; i < t.size(); ++i) {
+                out[3 * i] = t[i].x;
+                out[3 * i + 1] = t[i].y;
+                out[3 * i + 2] = t[i].z;
+            }
             return PSR_OK;
         }
         case PSR_ARRAY_DIVERGENCE: src = {c.fld.div, size_t(4) * M, 0}; break;

@@ -17,6 +17,7 @@ namespace {
 //   dot[a + res b]   = <F_a,  F_b>
 //   ddot[a + res b]  = <F_a', F_b>
 //   d2dot[a + res b] = <F_a', F_b'>
+// and ddotT, ddot transposed: the divergence of a node reads one row of it.
 // Each product is a polynomial of degree <= 4 between breakpoints; 3-point
 // Gauss-Legendre per piece integrates it exactly.
 __device__ double bsp_d(double u) {
@@ -39,7 +40,8 @@ __device__ void cw_of(int idx, double& c, double& w) {
 }
 
 __global__ void __launch_bounds__(256) build_tables_kernel(int res, double* __restrict__ dot,
-                                                           double* __restrict__ ddot, double* __restrict__ d2dot) {
+                                                           double* __restrict__ ddot, double* __restrict__ ddotT,
+                                                           double* __restrict__ d2dot) {
     long long t = (long long)blockIdx.x * 256 + threadIdx.x;
     if (t >= (long long)res * res) return;
     int a = int(t % res), b = int(t / res);
@@ -83,6 +85,7 @@ __global__ void __launch_bounds__(256) build_tables_kernel(int res, double* __re
     }
     dot[t] = r0;
     ddot[t] = r1;
+    ddotT[size_t(a) * res + b] = r1;
     d2dot[t] = r2;
 }
 
@@ -165,13 +168,23 @@ __device__ __forceinline__ int range_of(const NbRanges& r, int t) {
 // two depth-D nodes per wave, one per half: a node's chain of dependent loads
 // (neighbours, their point ranges, the points) is latency-bound, and the two
 // chains of a wave overlap.
-// Field storage: FP32, or FP16 holding V * 2^-(D+1) (the normals' scale, an
-// exact power of two, so the stored value is the FP16 rounding of the sum of
-// weighted unit normals).
-__device__ __forceinline__ void store_field(float* p, float v, float) { *p = v; }
-__device__ __forceinline__ void store_field(__half* p, float v, float invScale) { *p = __float2half_rn(v * invScale); }
-__device__ __forceinline__ float load_field(const float* p, float) { return *p; }
-__device__ __forceinline__ float load_field(const __half* p, float scale) { return __half2float(*p) * scale; }
+// Field storage, a vector per node: FP32, or FP16 holding V * 2^-(D+1) (the
+// normals' scale, an exact power of two, so the stored value is the FP16
+// rounding of the sum of weighted unit normals); the divergence reads a vector
+// with one load (FieldHalf, float4: the fourth component is unused).
+__device__ __forceinline__ void store_field(float4* p, float3 v, float) { *p = make_float4(v.x, v.y, v.z, 0.f); }
+__device__ __forceinline__ void store_field(FieldHalf* p, float3 v, float invScale) {
+    *p = FieldHalf{__float2half_rn(v.x * invScale), __float2half_rn(v.y * invScale), __float2half_rn(v.z * invScale),
+                   __half(0.f)};
+}
+__device__ __forceinline__ float3 load_field(const float4* p, float) {
+    const float4 v = *p;
+    return make_float3(v.x, v.y, v.z);
+}
+__device__ __forceinline__ float3 load_field(const FieldHalf* p, float scale) {
+    const FieldHalf v = *p;
+    return make_float3(__half2float(v.x) * scale, __half2float(v.y) * scale, __half2float(v.z) * scale);
+}
 
 constexpr int kVfWaves = 4;
 template <class FieldT>
@@ -217,10 +230,7 @@ __device__ __forceinline__ void vector_field_kernel_body(int psr_bid, int psr_nb
     ay = half_sum_f32(ay, half);
     az = half_sum_f32(az, half);
     if (hl == 0 && valid) {
-        const float inv = 1.0f / float(2 << D);
-        store_field(&vf[node], ax, inv);
-        store_field(&vf[nD + node], ay, inv);
-        store_field(&vf[2 * nD + node], az, inv);
+        store_field(&vf[node], make_float3(ax, ay, az), 1.0f / float(2 << D));
     }
 }
 template <class FieldT>
@@ -241,42 +251,82 @@ struct vector_field_kernel_k {
 // --- divergence (ComputeNodesDivergence.cu:25-136) -------------------------
 // b(o) = sum over the 27 neighbours' depth-D descendants j of
 //        V_j . (<F'_ox, F_jx>, <F'_oy, F_jy>, <F'_oz, F_jz>)     (reference Q3)
+// The rows of ddotT of a node's three functions: F_j's values lie beside those of
+// its neighbours, where a column of ddot has a cache line for each.
+struct DivRows {
+    const double *x, *y, *z;
+    __device__ __forceinline__ DivRows(const double* ddotT, int res, int3 fo)
+        : x(ddotT + size_t(fo.x) * res), y(ddotT + size_t(fo.y) * res), z(ddotT + size_t(fo.z) * res) {}
+};
 template <class FieldT>
-__device__ __forceinline__ double div_term(int j, int offD, int nD, int res, int D, int3 fo,
-                                           const int* __restrict__ enc, const FieldT* __restrict__ vf,
-                                           const double* __restrict__ ddot) {
-    const float sc = float(2 << D);
-    int3 fj = decode_func_index(enc[offD + j], D);
-    double s = double(load_field(&vf[j], sc)) * ddot[fo.x + res * fj.x];
-    s += double(load_field(&vf[nD + j], sc)) * ddot[fo.y + res * fj.y];
-    s += double(load_field(&vf[2 * nD + j], sc)) * ddot[fo.z + res * fj.z];
+__device__ __forceinline__ double div_term(int j, int offD, int D, const DivRows& rows, const int* __restrict__ enc,
+                                           const FieldT* __restrict__ vf) {
+    const int3 fj = decode_func_index(enc[offD + j], D);
+    const float3 v = load_field(&vf[j], float(2 << D));
+    double s = double(v.x) * rows.x[fj.x];
+    s += double(v.y) * rows.y[fj.y];
+    s += double(v.z) * rows.z[fj.z];
     return s;
 }
 
 constexpr int kDivWaves = 4;
+// The wave's three rows are copied to LDS where they are short (a term's table
+// values are three scattered 8-byte reads, which bound the kernel from the cache;
+// its vector and index are contiguous).  The launch with this, one load a vector
+// and the leaves' 9 table values: 200k torus at depth 7 51 -> 38 us, 20k sphere at
+// depth 6 25 -> 16 us, 300k points at depth 8 163 -> 141 us, 32 clouds 1141 -> 980.
+constexpr int kDivRow = 96;  // functions an axis kept in LDS: up to 5 levels above depth D
 template <class FieldT>
 __device__ __forceinline__ void divergence_fine_body(int psr_bid, int psr_nbid, 
     int begin, int count, int M, int offD, int nD, int res, int D, const int* __restrict__ neigh,
     const int* __restrict__ didx, const int* __restrict__ dnum, const int* __restrict__ enc,
-    const FieldT* __restrict__ vf, const double* __restrict__ ddot, float* __restrict__ div) {
+    const FieldT* __restrict__ vf, const double* __restrict__ ddotT, const int* __restrict__ q1Fired,
+    float* __restrict__ div) {
     // (two nodes per wave, as the vector field splats them, measured 64%
     // slower here: a node at depth 4 or 5 has hundreds to thousands of terms)
-    __shared__ NbRanges R[kDivWaves];
+    __shared__ NbRanges ranges[kDivWaves];
+    __shared__ double rowStore[kDivWaves][3 * kDivRow];
     int wid = threadIdx.x / PSR_WAVE, lane = __lane_id();
     int node = psr_bid * kDivWaves + wid;
     if (node >= count) return;
     int o = begin + node;
-    NbRanges& r = R[wid];
+    NbRanges& r = ranges[wid];
+    double* tab = rowStore[wid];
     int total = wave_ranges(r, neigh, M, o, lane, [&](int nb, int& first, int& len) {
         first = didx[nb];
         len = dnum[nb];
     });
     __builtin_amdgcn_wave_barrier();
-    int3 fo = decode_func_index(enc[o], D);
+    const int3 fo = decode_func_index(enc[o], D);
+    const DivRows rows(ddotT, res, fo);
     double acc = 0;
-    for (int t = lane; t < total; t += PSR_WAVE) {
-        int i = range_of(r, t);
-        acc += div_term(r.first[i] + (t - r.start[i]), offD, nD, res, D, fo, enc, vf, ddot);
+    // on the regular grid the descendants' functions are those of the node's cell
+    // and the cells beside it, 3 2^(D - d) an axis
+    const int d = 31 - __clz(fo.x + 1), k = D - d, R = 3 << k;
+    if (*q1Fired == 0 && R <= kDivRow) {
+        int f0[3];
+        const int f[3] = {fo.x, fo.y, fo.z};
+        const double* g[3] = {rows.x, rows.y, rows.z};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            f0[a] = (1 << D) - 1 + (f[a] - (1 << d)) * (1 << k);  // the first of the cell below
+            for (int u = lane; u < R; u += PSR_WAVE) tab[a * kDivRow + u] = g[a][min(max(f0[a] + u, 0), res - 1)];
+        }
+        __builtin_amdgcn_wave_barrier();
+        for (int t = lane; t < total; t += PSR_WAVE) {
+            const int i = range_of(r, t), j = r.first[i] + (t - r.start[i]);
+            const int3 fj = decode_func_index(enc[offD + j], D);
+            const float3 v = load_field(&vf[j], float(2 << D));
+            double s = double(v.x) * tab[fj.x - f0[0]];
+            s += double(v.y) * tab[kDivRow + fj.y - f0[1]];
+            s += double(v.z) * tab[2 * kDivRow + fj.z - f0[2]];
+            acc += s;
+        }
+    } else {
+        for (int t = lane; t < total; t += PSR_WAVE) {
+            int i = range_of(r, t);
+            acc += div_term(r.first[i] + (t - r.start[i]), offD, D, rows, enc, vf);
+        }
     }
     acc = wave_sum_f64(acc);
     if (lane == 0) div[o] = float(acc);
@@ -289,7 +339,7 @@ template <class FieldT>
 __device__ __forceinline__ void divergence_coarse_body(int psr_bid, int psr_nbid, 
     const CoarsePlan& P, int M, int offD, int nD, int res, int D, const int* __restrict__ neigh,
     const int* __restrict__ didx, const int* __restrict__ dnum, const int* __restrict__ enc,
-    const FieldT* __restrict__ vf, const double* __restrict__ ddot, double* __restrict__ partial) {
+    const FieldT* __restrict__ vf, const double* __restrict__ ddotT, double* __restrict__ partial) {
     int d = 0;
     while (d + 1 < P.depths && int(psr_bid) >= P.blockStart[d + 1]) ++d;
     const int parts = P.parts[d];
@@ -310,12 +360,12 @@ __device__ __forceinline__ void divergence_coarse_body(int psr_bid, int psr_nbid
     }
     __syncthreads();
     const int total = start[27];
-    const int3 fo = decode_func_index(enc[o], D);
+    const DivRows rows(ddotT, res, decode_func_index(enc[o], D));
     double acc = 0;
     int i = 0;
     for (int t = part * kDivCoarseThreads + threadIdx.x; t < total; t += parts * kDivCoarseThreads) {
         while (start[i + 1] <= t) ++i;
-        acc += div_term(first[i] + (t - start[i]), offD, nD, res, D, fo, enc, vf, ddot);
+        acc += div_term(first[i] + (t - start[i]), offD, D, rows, enc, vf);
     }
     acc = wave_sum_f64(acc);
     if (__lane_id() == 0) red[threadIdx.x / PSR_WAVE] = acc;
@@ -327,28 +377,53 @@ __device__ __forceinline__ void divergence_coarse_body(int psr_bid, int psr_nbid
     }
 }
 // Depth-D nodes: their neighbours are depth-D nodes, each its own only
-// descendant, so a thread sums the 27 terms of its node.  The first threads
-// also fold the coarse nodes' shares (thread t: coarse node t), in order.
-// Blocks from leafBlocks on assemble the operator instead (assemble_rows):
-// independent work that fills the GPU beside this kernel's few workgroups.
-// Depth-D nodes: their neighbours are depth-D nodes, each its own only
-// descendant, so a thread sums the 27 terms of its node.
+// descendant, so a thread sums the 27 terms of its node.  On the regular grid
+// neighbour i's functions are the node's own shifted by its offset, so that the
+// 81 table values are 9 and no neighbour's index is read.
 template <class FieldT>
 __device__ __forceinline__ void divergence_leaf_nodes(int block, int offD, int nD, int M, int res, int D,
                                                       const int* __restrict__ neigh, const int* __restrict__ enc,
                                                       const FieldT* __restrict__ vf,
-                                                      const double* __restrict__ ddot, float* __restrict__ div) {
+                                                      const double* __restrict__ ddotT,
+                                                      const int* __restrict__ q1Fired, float* __restrict__ div) {
     const int t = block * 256 + threadIdx.x;
     if (t >= nD) return;
     const int o = offD + t;
     const int3 fo = decode_func_index(enc[o], D);
-    int nb[27];
-#pragma unroll
-    for (int i = 0; i < 27; ++i) nb[i] = neigh[i * M + o];
+    const DivRows rows(ddotT, res, fo);
     double acc = 0;
+    if (*q1Fired == 0 && neigh[13 * M + o] == o) {
+        const float sc = float(2 << D);
+        double wy[3], wz[3];
 #pragma unroll
-    for (int i = 0; i < 27; ++i)
-        if (nb[i] != -1) acc += div_term(nb[i] - offD, offD, nD, res, D, fo, enc, vf, ddot);
+        for (int k = 0; k < 3; ++k) {  // past the domain: not used
+            wy[k] = rows.y[min(max(fo.y + k - 1, 0), res - 1)];
+            wz[k] = rows.z[min(max(fo.z + k - 1, 0), res - 1)];
+        }
+#pragma unroll 1
+        for (int x = 0; x < 3; ++x) {  // nine neighbours' loads in flight (27 take 12 more registers)
+            const double wx = rows.x[min(max(fo.x + x - 1, 0), res - 1)];
+            int nb[9];
+            float3 v[9];
+#pragma unroll
+            for (int i = 0; i < 9; ++i) nb[i] = neigh[(9 * x + i) * M + o];
+#pragma unroll
+            for (int i = 0; i < 9; ++i) v[i] = load_field(&vf[nb[i] != -1 ? nb[i] - offD : 0], sc);
+#pragma unroll
+            for (int i = 0; i < 9; ++i) {
+                double s = double(v[i].x) * wx;
+                s += double(v[i].y) * wy[i / 3];
+                s += double(v[i].z) * wz[i % 3];
+                if (nb[i] != -1) acc += s;
+            }
+        }
+    } else {
+#pragma unroll 3
+        for (int i = 0; i < 27; ++i) {
+            const int nb = neigh[i * M + o];
+            if (nb != -1) acc += div_term(nb - offD, offD, D, rows, enc, vf);
+        }
+    }
     div[o] = float(acc);
 }
 
@@ -368,24 +443,24 @@ __device__ __forceinline__ void divergence_all_body(int psr_bid, int psr_nbid, c
                                                     int begin, int count, int M, int offD, int nD, int res, int D,
                                                     const int* __restrict__ neigh, const int* __restrict__ didx,
                                                     const int* __restrict__ dnum, const int* __restrict__ enc,
-                                                    const FieldT* __restrict__ vf, const double* __restrict__ ddot,
+                                                    const FieldT* __restrict__ vf, const double* __restrict__ ddotT,
                                                     double* __restrict__ partial, float* __restrict__ div,
                                                     const AssembleArgs& aa) {
     int b = psr_bid;
     if (b < R.coarseBlocks) {
-        divergence_coarse_body<FieldT>(b, R.coarseBlocks, P, M, offD, nD, res, D, neigh, didx, dnum, enc, vf, ddot,
+        divergence_coarse_body<FieldT>(b, R.coarseBlocks, P, M, offD, nD, res, D, neigh, didx, dnum, enc, vf, ddotT,
                                        partial);
         return;
     }
     b -= R.coarseBlocks;
     if (b < R.midBlocks) {
         divergence_fine_body<FieldT>(b, R.midBlocks, begin, count, M, offD, nD, res, D, neigh, didx, dnum, enc, vf,
-                                     ddot, div);
+                                     ddotT, aa.q1Fired, div);
         return;
     }
     b -= R.midBlocks;
     if (b < R.leafBlocks) {
-        divergence_leaf_nodes<FieldT>(b, offD, nD, M, res, D, neigh, enc, vf, ddot, div);
+        divergence_leaf_nodes<FieldT>(b, offD, nD, M, res, D, neigh, enc, vf, ddotT, aa.q1Fired, div);
         return;
     }
     assemble_rows(aa, b - R.leafBlocks);
@@ -394,10 +469,10 @@ template <class FieldT>
 __global__ void __launch_bounds__(kDivCoarseThreads) divergence_all(
     CoarsePlan P, DivRoles R, int begin, int count, int M, int offD, int nD, int res, int D,
     const int* __restrict__ neigh, const int* __restrict__ didx, const int* __restrict__ dnum,
-    const int* __restrict__ enc, const FieldT* __restrict__ vf, const double* __restrict__ ddot,
+    const int* __restrict__ enc, const FieldT* __restrict__ vf, const double* __restrict__ ddotT,
     double* __restrict__ partial, float* __restrict__ div, AssembleArgs aa) {
     divergence_all_body<FieldT>(blockIdx.x, gridDim.x, P, R, begin, count, M, offD, nD, res, D, neigh, didx, dnum, enc,
-                                vf, ddot, partial, div, aa);
+                                vf, ddotT, partial, div, aa);
 }
 template <class FieldT>
 struct divergence_all_k {
@@ -416,8 +491,9 @@ void build_tables(Ctx& c) {
     size_t n = size_t(res) * res;
     t.dot = c.buf<double>("table_dot", n);
     t.ddot = c.buf<double>("table_ddot", n);
+    t.ddotT = c.buf<double>("table_ddot_t", n);
     t.d2dot = c.buf<double>("table_d2dot", n);
-    build_tables_kernel<<<div_up(n, 256), 256, 0, c.stream>>>(res, t.dot, t.ddot, t.d2dot);
+    build_tables_kernel<<<div_up(n, 256), 256, 0, c.stream>>>(res, t.dot, t.ddot, t.ddotT, t.d2dot);
     PSR_HIP_CHECK(hipGetLastError());
     // The inner products of each depth's functions with those at offsets -1, 0
     // and 1 (a depth's functions are consecutive), copied out in one piece.
@@ -545,7 +621,7 @@ void field_stages(Ctx& c, FieldT* vf) {
     const int assembleBlocks = int(div_up(size_t(3) * M, kAssembleThreads));
     PSR_LAUNCH_K(divergence_all<FieldT>, divergence_all_k<FieldT>,
                  R.coarseBlocks + R.midBlocks + R.leafBlocks + assembleBlocks, 0, s, P, R, coarseCount, midCount, M,
-                 offD, nD, c.tables.res, D, o.neigh, o.didx, o.dnum, o.encIdx, vf, c.tables.ddot, partial, c.fld.div,
+                 offD, nD, c.tables.res, D, o.neigh, o.didx, o.dnum, o.encIdx, vf, c.tables.ddotT, partial, c.fld.div,
                  aa);
     c.fld.foldArgs = DivFoldArgs{P, partial, c.fld.div};  // run by the solve's first kernel (solve_depths)
     PSR_HIP_CHECK(hipGetLastError());
@@ -559,11 +635,11 @@ void compute_field(Ctx& c) {
     c.fld.div = c.buf<float>("divergence", c.oct.M);
     if (c.cfg.precision == PSR_PRECISION_MIXED) {
         c.fld.vfield = nullptr;
-        c.fld.vhalf = c.buf<__half>("vfield_half", size_t(3) * nD);
+        c.fld.vhalf = c.buf<FieldHalf>("vfield_half", nD);
         field_stages(c, c.fld.vhalf);
     } else {
         c.fld.vhalf = nullptr;
-        c.fld.vfield = c.buf<float>("vfield", size_t(3) * nD);
+        c.fld.vfield = c.buf<float4>("vfield", nD);
         field_stages(c, c.fld.vfield);
     }
 }

@@ -65,6 +65,7 @@ struct Tables {
     int res = 0;
     double* dot = nullptr;
     double* ddot = nullptr;
+    double* ddotT = nullptr;  // ddot transposed
     double* d2dot = nullptr;
     // The operator's entry per depth and neighbour slot, [depth][27], where every
     // pair of functions at that offset gives the same float (checked over all of
@@ -98,9 +99,14 @@ struct Octree {
     float* normParams = nullptr;     // corner xyz, edge
 };
 
+// The vector field's stored vector in the mixed-precision form.
+struct alignas(8) FieldHalf {
+    __half x, y, z, w;
+};
+
 struct Field {
-    float* vfield = nullptr;  // [3][nD] (FP32 form)
-    __half* vhalf = nullptr;  // [3][nD], V * 2^-(D+1) (mixed-precision form)
+    float4* vfield = nullptr;    // a vector per depth-D node (FP32 form)
+    FieldHalf* vhalf = nullptr;  // V * 2^-(D+1) (mixed-precision form)
     float* div = nullptr;     // [M]
     float* dx = nullptr;      // [M]
     float* chiPts = nullptr;  // [N]
