@@ -138,7 +138,7 @@ def cg_kernel_name(st, precision):
     if st["cg_row_form"]:
         return "cg_mixed_row" if precision == "mixed" else "cg_fp32_row"
     if precision == "mixed":
-        return "cg_mixed_all_depths+cg_mixed_minres" if st["depth"] >= 9 else "cg_mixed_all_depths"
+        return "cg_mixed_all_depths+cg_minres_chip16" if st["depth"] >= 9 else "cg_mixed_all_depths"
     return "cg_all_depths"
 
 
@@ -151,16 +151,21 @@ def cg_algorithmic_bytes(st, precision):
     out; b, x, residual) + 28n per inner iteration (records {r, w, s} read and
     written, x out).  Several rows per thread (stencil read every sweep):
     FP32 (CGAlgorithm.cu:10-80) 8z + 48n per iteration; mixed 8n, then
-    16z + 32n per outer step and 8z + 40n per inner iteration."""
+    16z + 32n per outer step and 8z + 40n per inner iteration; a depth solved
+    with MINRES (9 and deeper) keeps stencil and vectors on chip, so that its
+    inner iterations move only the workgroups' outer records, which are not
+    counted."""
     total = 0
     row = bool(st["cg_row_form"])
-    for k, z, n, o in zip(st["cg_iterations"], st["cg_nnz"], st["nodes_per_depth"], st["cg_outer"]):
+    per_depth = zip(st["cg_iterations"], st["cg_nnz"], st["nodes_per_depth"], st["cg_outer"])
+    for d, (k, z, n, o) in enumerate(per_depth):
         if row and precision == "mixed":
             total += 8 * z + 8 * n + o * 28 * n + k * 28 * n
         elif row:
             total += 8 * z + 16 * n + k * 16 * n
         elif precision == "mixed":
-            total += 8 * n + o * (16 * z + 32 * n) + k * (8 * z + 40 * n)
+            inner = 0 if d >= 9 else k * (8 * z + 40 * n)
+            total += 8 * n + o * (16 * z + 32 * n) + inner
         else:
             total += k * (8 * z + 48 * n)
     return total
