@@ -487,7 +487,8 @@ __device__ __forceinline__ RowMap row_map(RowShared& sh, const RowMapArgs& a, in
     for (int e = 0; e < 13; ++e) {
         const unsigned p = a.places[size_t(e) * M + i];
         if (e == 12) m.boundary = own && (p & kBoundaryBit) != 0u;
-        sh.place[e][t] = p & ~(e == 12 ? kBoundaryBit : 0u);
+        // the other waves of a one-wave group have no rows, and wave 0 keeps its weights in their words
+        if (!oneWave || t < PSR_WAVE) sh.place[e][t] = p & ~(e == 12 ? kBoundaryBit : 0u);
     }
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
