@@ -257,9 +257,11 @@ __device__ __forceinline__ void st_vec4(__amdgpu_buffer_rsrc_t r, int idx, float
 // weights are one constant per slot (the operator depends on the offset only;
 // checked row by row), held in scalar registers; a row's columns are 26 16-bit
 // places in LDS.  Only rows with a neighbour outside write records.
-// Where the level-local child 0 rule changed the neighbour tables the weights
-// may differ from row to row: such a workgroup reads each row's own, and what
-// has no place from memory (the slow form of the product).
+// Where the level-local child 0 rule changed the neighbour tables a row may lack
+// its own entry, and in a tenth of such clouds a slot's weights differ from row
+// to row: such a workgroup reads each row's own (RowHead::kOwnWeights), a group
+// of one wave from LDS.  Neighbours outside that the ghost list cannot hold are
+// read from memory (RowHead::kMemoryPlaces).
 // Bound by the reductions' memory round trips (about 2 us each) and the
 // ghosts' (1 us).  Whole solves with 256 rows a workgroup, the stencil per row
 // and a record gathered per entry, and here: torus at depth 7 (71k rows) 146 ->
@@ -287,9 +289,10 @@ constexpr int kRowFp32Waves = 8, kRowMixedWaves = 6;
 // list of kGhostMax, its rows' places in a table [13][M]).
 struct RowHead {
     int ghosts;
-    int slow;     // weights per row, or neighbours without a place
+    int form;     // 0: what follows suffices
     float w[27];  // the slots' weights
     int pad[3];
+    static constexpr int kOwnWeights = 1, kMemoryPlaces = 2;  // bits of form
 };
 struct RowMapArgs {
     const int* neigh;
@@ -313,7 +316,7 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     __shared__ int key[kGhostTable];                        // ghost rows by hash, -1: free
     __shared__ unsigned short number[kGhostTable];
     __shared__ unsigned weight[27];
-    __shared__ int entries, ghosts, slow;
+    __shared__ int entries, ghosts, form;
     constexpr unsigned kGhostMark = 0x8000u;
     static_assert(kRowThreads == 512, "nine bits of row, five of slot");
     int gi = 0;
@@ -339,22 +342,22 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     }
     for (int k = t; k < kGhostTable; k += kRowThreads) key[k] = -1;
     if (t < 27) weight[t] = regular ? __float_as_uint(a.weights[27 * G.depth + t]) : 0u;
-    if (t == 0) entries = 0, ghosts = 0, slow = 0;
+    if (t == 0) entries = 0, ghosts = 0, form = 0;
     __syncthreads();
-    unsigned bad = 0u, outside = 0u, ghost = 0u;  // ghost: slots with a stored neighbour outside
+    int needs = 0;
+    unsigned outside = 0u, ghost = 0u;  // ghost: slots with a stored neighbour outside
 #pragma unroll
     for (int q = 0; q < 27; ++q) {
         const int l = j[q] - r0;
         const bool inside = unsigned(l) < unsigned(rows), stored = own && v[q] != 0.f;
         if (!regular && stored) weight[q] = __float_as_uint(v[q]);  // any row's
-        if (q == 13) {
-            if (own && (!stored || l != t)) bad = 1u;
+        if (q == 13) {  // the row itself or, below a parent the child 0 rule changed, nothing
+            if (own && !stored) needs |= RowHead::kOwnWeights;
             continue;
         }
         const bool away = own && j[q] >= 0 && !inside;
         if (away) outside = 1u;
         if (away && stored) ghost |= 1u << q;
-        if (stored && j[q] < 0) bad = 1u;
         place[q < 13 ? q : q - 1][t] =
             static_cast<unsigned short>(!stored ? kPlaceZero : (inside ? 4 * l : kPlaceMemory));
     }
@@ -401,7 +404,7 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     auto final_place = [&](int e) {
         unsigned p = place[e][t];
         if (p & kGhostMark) p = overflow ? unsigned(kPlaceMemory) : unsigned(kPlaceGhosts) + 4u * number[p & (kGhostTable - 1)];
-        if (own && p == unsigned(kPlaceMemory)) bad = 1u;
+        if (own && p == unsigned(kPlaceMemory)) needs |= RowHead::kMemoryPlaces;
         return p;
     };
     unsigned word = 0u;
@@ -413,16 +416,16 @@ __device__ __forceinline__ void row_maps_body(int psr_bid, int psr_nbid, const C
     if (!regular) {
 #pragma unroll
         for (int q = 0; q < 27; ++q)
-            if (own && v[q] != 0.f && __float_as_uint(v[q]) != weight[q]) bad = 1u;
+            if (own && v[q] != 0.f && __float_as_uint(v[q]) != weight[q]) needs |= RowHead::kOwnWeights;
     }
-    if (bad) slow = 1;
+    if (needs) atomicOr(&form, needs);
     __syncthreads();
     // readers of a row outside its workgroup: symmetric where the tables are regular
-    const bool boundary = outside != 0u || *a.q1Fired != 0 || slow != 0;
+    const bool boundary = outside != 0u || *a.q1Fired != 0 || form != 0;
     if (own) a.places[size_t(12) * M + i] = word | (boundary ? kBoundaryBit : 0u);
     RowHead& head = a.heads[psr_bid];
     if (t < 27) head.w[t] = __uint_as_float(weight[t]);
-    if (t == 0) head.ghosts = overflow ? 0 : ghosts, head.slow = slow;
+    if (t == 0) head.ghosts = overflow ? 0 : ghosts, head.form = form;
 }
 // The solve's first kernel: the fold of the coarse nodes' divergence, and the
 // row form's maps (mapBlocks of them; none for the other forms) beside it.  Both
@@ -453,67 +456,87 @@ __device__ __forceinline__ double uniform(double v) {
 }
 
 struct RowShared {
+    // the rows' places; or, in a one-wave group with own weights, lane t's 27
+    // weights and 13 words of places as chunks of four, [11][PSR_WAVE]
+    alignas(16) unsigned place[13][kRowThreads];
     float v[kRowThreads + kGhostMax + 1];  // the rows' values, the ghosts', a zero
-    unsigned place[13][kRowThreads];       // the rows' places; a one-wave group's own weights where it has no rows
     double sum[2][kRowWaves][2];           // wave sums, by the parity of the sum
     double fold[kRowWaves][2];
     int fail;
 };
+constexpr int kLaneChunks = 11, kLanePlaces = 28;  // words: 27 weights and a pad, then the places
+static_assert(kLaneChunks * 4 >= kLanePlaces + 13 && kLaneChunks * 4 * PSR_WAVE <= 13 * kRowThreads, "a lane's words fit");
+__device__ __forceinline__ unsigned& lane_word(RowShared& sh, int k, int t) {
+    return (&sh.place[0][0])[4 * (k / 4 * PSR_WAVE + t) + k % 4];
+}
 
 // A row's place in its group and what it needs of the stencil.
 struct RowMap {
     int ghostRow[2];     // this thread's ghosts (places t and t + kRowThreads of them): row, or -1
-    bool boundary;       // a neighbour lies outside the workgroup, and so a reader of this row
-    bool slow;           // the same in the whole workgroup
+    bool boundary;       // another workgroup may read this row
+    int form;            // RowHead::form, the same in the whole workgroup
+    bool lanes;          // the weights and places are in lane_word
 };
 
-// Row t's weight of slot q in a one-wave group of the slow form (as bits).
-__device__ __forceinline__ unsigned& row_own_weight(RowShared& sh, int q, int t) {
-    static_assert(kRowThreads >= 4 * PSR_WAVE && 13 * 3 >= 27, "the weights fit beside a wave's places");
-    return sh.place[q / 3][PSR_WAVE * (1 + q % 3) + t];
-}
-
-__device__ __forceinline__ RowMap row_map(RowShared& sh, const RowMapArgs& a, int bid, int r0, int rows, int M, bool oneWave,
-                                          float (&w)[27]) {
+__device__ __forceinline__ RowMap row_map(RowShared& sh, const RowMapArgs& a, int bid, int r0, int rows, int M, bool multi,
+                                          bool oneWave) {
     RowMap m;
     const int t = int(threadIdx.x), i = r0 + min(t, rows - 1);
     const bool own = t < rows;
     const RowHead& head = a.heads[bid];
     const int ghosts = __builtin_amdgcn_readfirstlane(head.ghosts);
-    m.slow = __builtin_amdgcn_readfirstlane(head.slow) != 0;
-#pragma unroll
-    for (int q = 0; q < 27; ++q) w[q] = uniform(head.w[q]);
+    m.form = __builtin_amdgcn_readfirstlane(head.form);
+    m.lanes = oneWave && m.form == RowHead::kOwnWeights;
 #pragma unroll
     for (int e = 0; e < 13; ++e) {
-        const unsigned p = a.places[size_t(e) * M + i];
-        if (e == 12) m.boundary = own && (p & kBoundaryBit) != 0u;
-        // the other waves of a one-wave group have no rows, and wave 0 keeps its weights in their words
-        if (!oneWave || t < PSR_WAVE) sh.place[e][t] = p & ~(e == 12 ? kBoundaryBit : 0u);
+        unsigned p = a.places[size_t(e) * M + i];
+        if (e == 12) {
+            m.boundary = multi && own && (p & kBoundaryBit) != 0u;
+            p &= ~kBoundaryBit;
+        }
+        // the other waves of a one-wave group have no rows, and write none of its words
+        if (m.lanes && t < PSR_WAVE) lane_word(sh, kLanePlaces + e, t) = p;
+        else if (!oneWave || t < PSR_WAVE) sh.place[e][t] = p;
     }
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
         const int e = t + g * kRowThreads;
         m.ghostRow[g] = e < ghosts ? a.ghosts[size_t(bid) * kGhostMax + e] : -1;
     }
-    if (m.slow && oneWave && t < PSR_WAVE) {
-        // such a group may take thousands of sweeps: its weights beside its values
+    if (m.lanes && t < PSR_WAVE) {
 #pragma unroll 1
-        for (int q = 0; q < 27; ++q) row_own_weight(sh, q, t) = own ? __float_as_uint(a.val[size_t(q) * M + i]) : 0u;
+        for (int q = 0; q < 27; ++q) lane_word(sh, q, t) = own ? __float_as_uint(a.val[size_t(q) * M + i]) : 0u;
     }
     if (t == 0) sh.fail = 0, sh.v[kPlaceZero / 4] = 0.f;
     __syncthreads();
     return m;
 }
 
+// The solves are compiled twice, for workgroups of form 0 (OWN false: the slots'
+// weights) and for the others (OWN: each row's own), so that what the others need
+// costs the first no registers: a spilled one is read back every sweep (300k
+// points at depth 8, mixed, 242 us a solve, 324 with one loop for both).
+// The others have missing entries and, where they are one wave at a coarse depth,
+// thousands of sweeps: solves of four bent clouds in the FP32 form with weights
+// and places in LDS by computed address and two branches an entry 41-52 ms, in
+// this straight line 7.3-18.5 ms; mixed 2.0-4.7 and 0.4-1.6 ms.
+template <bool OWN>
+__device__ __forceinline__ void slot_weights(const RowHead& head, float (&w)[27]) {
+#pragma unroll
+    for (int q = 0; q < 27; ++q) w[q] = OWN ? 0.f : uniform(head.w[q]);
+}
+
 // sum over the slots in order of weight x value, acc = term(acc, weight, value),
 // the values from LDS (`self`: the row's own); a thread without a row gets
-// something, which it must not use.  memory(e): the value of the
-// neighbour in entry e of the table where it has no place (slow form only).
-template <class T, class Term, class Memory>
+// something, which it must not use.  An entry that is not stored adds zero times
+// zero.  memory(e): the value of the neighbour in entry e of the table where it
+// has no place.
+template <bool OWN, class T, class Term, class Memory>
 __device__ __forceinline__ T row_product(const RowMap& m, const RowMapArgs& a, RowShared& sh, const float (&w)[27],
-                                         float self, bool own, bool oneWave, int i, int M, T acc, Term term, Memory memory) {
+                                         float self, bool own, int i, int M, T acc, Term term, Memory memory) {
+    const int t = int(threadIdx.x);
     auto placed = [&](unsigned p) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(sh.v) + p); };
-    if (!m.slow) {
+    if constexpr (!OWN) {
         // half of the neighbours' values are read together, then summed
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
@@ -521,7 +544,7 @@ __device__ __forceinline__ T row_product(const RowMap& m, const RowMapArgs& a, R
             float n[14];
 #pragma unroll
             for (int e = 0; e < count; e += 2) {
-                const unsigned p = sh.place[(first + e) / 2][threadIdx.x];
+                const unsigned p = sh.place[(first + e) / 2][t];
                 n[e] = placed(p & 0xffffu);
                 n[e + 1] = placed(p >> 16);
             }
@@ -534,15 +557,71 @@ __device__ __forceinline__ T row_product(const RowMap& m, const RowMapArgs& a, R
         }
         return acc;
     }
+    // slots 0-14 (entries 0-13 and the row itself), then 15-26: the values of a
+    // part are read together, then summed.  words(k, p): words k.. of the row's
+    // places; weights(q, v): the weights of slots q..
+    auto in_parts = [&](auto words, auto weights) {
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+            const int count = part ? 12 : 14;
+            unsigned p[7];
+            float v[15], n[14];
+            words(part * 7, p);
+            weights(part * 15, v);
+#pragma unroll
+            for (int e = 0; e < count; ++e) n[e] = placed(e % 2 ? p[e / 2] >> 16 : p[e / 2] & 0xffffu);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < (part ? 12 : 15); ++k)
+                acc = term(acc, v[k], part ? n[k] : (k < 13 ? n[k] : (k == 13 ? self : n[13])));
+        }
+    };
+    if (m.lanes) {
+        // such a group may take thousands of sweeps: its words come four at a time
+        const uint4* words = reinterpret_cast<const uint4*>(&sh.place[0][0]) + t;
+        auto word = [](const uint4& u, int k) { return k == 0 ? u.x : (k == 1 ? u.y : (k == 2 ? u.z : u.w)); };
+        in_parts(
+            [&](int first, unsigned (&p)[7]) {
+                const int k0 = kLanePlaces + first, c0 = k0 / 4;
+                uint4 u[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    if (c0 + c < kLaneChunks) u[c] = words[(c0 + c) * PSR_WAVE];
+#pragma unroll
+                for (int k = 0; k < 7; ++k)
+                    if (first + k < 13) p[k] = word(u[(k0 + k) / 4 - c0], (k0 + k) % 4);
+            },
+            [&](int first, float (&v)[15]) {
+                const int c0 = first / 4;
+                uint4 u[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) u[c] = words[(c0 + c) * PSR_WAVE];
+#pragma unroll
+                for (int k = 0; k < 15; ++k)
+                    if (first + k < 27) v[k] = __uint_as_float(word(u[(first + k) / 4 - c0], (first + k) % 4));
+            });
+        return acc;
+    }
     if (!own) return acc;
-    const int t = int(threadIdx.x);
+    asm volatile("" : "+v"(i));  // addresses are formed anew, not kept from sweep to sweep
+    if (m.form == RowHead::kOwnWeights) {
+        auto place_words = [&](int first, unsigned (&p)[7]) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k)
+                if (first + k < 13) p[k] = sh.place[first + k][t];
+        };
+        in_parts(place_words, [&](int first, float (&v)[15]) {
+#pragma unroll
+            for (int k = 0; k < 15; ++k)
+                if (first + k < 27) v[k] = (a.val + size_t(first + k) * M)[unsigned(i)];
+        });
+        return acc;
+    }
 #pragma unroll 1
     for (int c = 0; c < 27; c += 9) {
         float v[9];
-        asm volatile("" : "+v"(i));  // addresses are formed anew, not kept from sweep to sweep
 #pragma unroll
-        for (int k = 0; k < 9; ++k)
-            v[k] = oneWave ? __uint_as_float(row_own_weight(sh, c + k, t)) : (a.val + size_t(c + k) * M)[unsigned(i)];
+        for (int k = 0; k < 9; ++k) v[k] = (a.val + size_t(c + k) * M)[unsigned(i)];
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
             const int q = c + k;
@@ -617,8 +696,10 @@ __device__ __forceinline__ bool row_group_sum(double (&v)[N], RowShared& sh, Row
     const __amdgpu_buffer_rsrc_t rs = vec_rsrc(g.region + size_t(g.phase & 1u) * g.blocks * kSlotStride,
                                                sizeof(float4) * size_t(g.blocks) * kSlotStride);
     const float stamp = __uint_as_float(g.phase);
-    if (int(threadIdx.x) < N * g.ownBlocks) {
-        const int b = int(threadIdx.x) / N, n = int(threadIdx.x) % N;
+    int t = int(threadIdx.x);
+    asm volatile("" : "+v"(t));  // the slot's address is formed anew, not spilled from sum to sum
+    if (t < N * g.ownBlocks) {
+        const int b = t / N, n = t % N;
         const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(block_total(b, n)));
         st_vec4(rs, (g.firstBlock + b) * kSlotStride + n,
                 make_float4(__uint_as_float(unsigned(u)), __uint_as_float(unsigned(u >> 32)), stamp, 0.f));
@@ -693,23 +774,16 @@ __device__ __forceinline__ void row_sync(const RowGroup& g) {
 // iteration k the record of row i in buffer k & 1 holds {r_k, p_{k-1}}; a
 // ghost's p_k = r_k + beta p_{k-1} is formed from it, so the update of p and
 // the product A p need no group barrier in between (CGAlgorithm.cu:37-53).
-__device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& maps,
-                                                 const float* __restrict__ b, float* __restrict__ x, float2* state,
-                                                 float4* slots, int* __restrict__ iters, double* __restrict__ resid,
-                                                 int* errFlag) {
-    __shared__ RowShared sh;
-    int gi = 0;
-    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
-    const CgGroup G = P.g[gi];
-    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M;
-    const int r0 = G.rowBegin + local * G.rowsPerWg;
-    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0, i = r0 + t;
+template <bool OWN>
+__device__ __forceinline__ void cg_fp32_row_solve(int psr_bid, const CgParams& P, const CgGroup& G, const RowMapArgs& maps,
+                                                  const RowMap& m, RowGroup& g, RowShared& sh, int r0, int rows,
+                                                  const float* __restrict__ b, float* __restrict__ x, float2* state,
+                                                  int* __restrict__ iters, double* __restrict__ resid) {
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M, i = r0 + t;
     const bool own = t < rows;
-    RowGroup g = row_group(P, G, local, slots, errFlag);
-    float w[27];
-    const RowMap m = row_map(sh, maps, psr_bid, r0, rows, M, g.oneWave, w);
     const int* __restrict__ neigh = maps.neigh;
-    if (g.oneWave && t >= PSR_WAVE) return;
+    float w[27];
+    slot_weights<OWN>(maps.heads[psr_bid], w);
     const __amdgpu_buffer_rsrc_t st = vec_rsrc(state, sizeof(float2) * 2 * size_t(M));
     // x = 0, r = b, rr = r.r  (CGAlgorithm.cu:21-33 with x0 = 0)
     float xi = 0.f, ri = own ? b[i] : 0.f, pi = 0.f;
@@ -737,7 +811,7 @@ __device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, cons
             const float2 r = ld_vec2(st, cur + neigh[e]);
             return p_next(r.x, beta, r.y);
         };
-        const float api = row_product(m, maps, sh, w, pi, own, g.oneWave, i, M, 0.f, term, memory);
+        const float api = row_product<OWN>(m, maps, sh, w, pi, own, i, M, 0.f, term, memory);
         sum[0] = own ? double(pi * api) : 0.0;
         if (!row_group_sum<1>(sum, sh, g)) return;
         const float alpha = uniform(float(double(rr) / sum[0]));
@@ -756,6 +830,22 @@ __device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, cons
         iters[PSR_MAX_DEPTH + 1 + G.depth] = 1;
         resid[G.depth] = sqrt(double(rr));
     }
+}
+__device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& maps,
+                                                 const float* __restrict__ b, float* __restrict__ x, float2* state,
+                                                 float4* slots, int* __restrict__ iters, double* __restrict__ resid,
+                                                 int* errFlag) {
+    __shared__ RowShared sh;
+    int gi = 0;
+    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
+    const CgGroup G = P.g[gi];
+    const int local = psr_bid - G.firstWg, r0 = G.rowBegin + local * G.rowsPerWg;
+    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0;
+    RowGroup g = row_group(P, G, local, slots, errFlag);
+    const RowMap m = row_map(sh, maps, psr_bid, r0, rows, P.M, g.multi, g.oneWave);
+    if (g.oneWave && int(threadIdx.x) >= PSR_WAVE) return;
+    if (m.form == 0) cg_fp32_row_solve<false>(psr_bid, P, G, maps, m, g, sh, r0, rows, b, x, state, iters, resid);
+    else cg_fp32_row_solve<true>(psr_bid, P, G, maps, m, g, sh, r0, rows, b, x, state, iters, resid);
 }
 __global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kRowFp32Waves))) cg_fp32_row(
     CgParams P, RowMapArgs maps, const float* __restrict__ b, float* __restrict__ x, float2* state, float4* slots,
@@ -1030,23 +1120,17 @@ __device__ __forceinline__ Comp2 block_comp2(Comp2 v, Comp2* sh) {
 // bit.  Per inner iteration k the record of row i in buffer k & 1 holds
 // {r_k, w_k, s_{k-1}, x_k}; the row writes {r_{k+1}, w_{k+1}, s_k, x_{k+1}} to
 // the other buffer.
-__device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& maps,
-                                                  const float* __restrict__ b, float* x, float* rOut, float4* state,
-                                                  float4* slots, int* __restrict__ iters, double* __restrict__ resid,
-                                                  double* __restrict__ trueRel, int* errFlag) {
-    __shared__ RowShared sh;
-    int gi = 0;
-    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
-    const CgGroup G = P.g[gi];
-    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M;
-    const int r0 = G.rowBegin + local * G.rowsPerWg;
-    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0, i = r0 + t;
+template <bool OWN>
+__device__ __forceinline__ void cg_mixed_row_solve(int psr_bid, const CgParams& P, const CgGroup& G, const RowMapArgs& maps,
+                                                   const RowMap& m, RowGroup& g, RowShared& sh, int r0, int rows,
+                                                   const float* __restrict__ b, float* x, float* rOut, float4* state,
+                                                   int* __restrict__ iters, double* __restrict__ resid,
+                                                   double* __restrict__ trueRel) {
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M, i = r0 + t;
     const bool own = t < rows;
-    RowGroup g = row_group(P, G, local, slots, errFlag);
-    float w[27];
-    const RowMap m = row_map(sh, maps, psr_bid, r0, rows, M, g.oneWave, w);
     const int* __restrict__ neigh = maps.neigh;
-    if (g.oneWave && t >= PSR_WAVE) return;
+    float w[27];
+    slot_weights<OWN>(maps.heads[psr_bid], w);
     const __amdgpu_buffer_rsrc_t st = vec_rsrc(state, sizeof(float4) * 2 * size_t(M));
     auto term = [](float a, float wq, float v) { return __fmaf_rn(wq, v, a); };
     auto ghost_values = [&](auto value) {  // value(row) into the ghosts' places
@@ -1087,7 +1171,7 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
         row_sync(g);
         {
             auto memory = [&](size_t e) { return ld_shared(&rhs[neigh[e]]); };
-            wo = row_product(m, maps, sh, w, ro, own, g.oneWave, i, M, 0.f, term, memory);
+            wo = row_product<OWN>(m, maps, sh, w, ro, own, i, M, 0.f, term, memory);
             if (!own) wo = 0.f;
         }
         so = po = 0.f;
@@ -1129,7 +1213,7 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
                 const float4 r = ld_vec4(st, cur + neigh[e]);
                 return r_next(r.x, alpha, s_next(r.y, beta, r.z));
             };
-            wo = row_product(m, maps, sh, w, rni, own, g.oneWave, i, M, 0.f, term, memory);
+            wo = row_product<OWN>(m, maps, sh, w, rni, own, i, M, 0.f, term, memory);
             if (!own) wo = 0.f;
             ro = rni;
             so = si;
@@ -1172,7 +1256,7 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
             auto term64 = [](double a, float wq, float v) { return a - double(wq) * double(v); };
             auto memory = [&](size_t e) { return ld_vec4(st, last + neigh[e]).w; };
             asm volatile("" : "+v"(ii));
-            const double acc = row_product(m, maps, sh, w, xi, own, g.oneWave, i, M, double(b[ii]), term64, memory);
+            const double acc = row_product<OWN>(m, maps, sh, w, xi, own, i, M, double(b[ii]), term64, memory);
             st_shared(&rOut[ii], float(acc));
             loc[0] = acc * acc;
         }
@@ -1191,6 +1275,24 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
         resid[G.depth] = sqrt(double(gamma));
         trueRel[G.depth] = rel;
     }
+}
+__device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, const CgParams& P, const RowMapArgs& maps,
+                                                  const float* __restrict__ b, float* x, float* rOut, float4* state,
+                                                  float4* slots, int* __restrict__ iters, double* __restrict__ resid,
+                                                  double* __restrict__ trueRel, int* errFlag) {
+    __shared__ RowShared sh;
+    int gi = 0;
+    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
+    const CgGroup G = P.g[gi];
+    const int local = psr_bid - G.firstWg, r0 = G.rowBegin + local * G.rowsPerWg;
+    const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0;
+    RowGroup g = row_group(P, G, local, slots, errFlag);
+    const RowMap m = row_map(sh, maps, psr_bid, r0, rows, P.M, g.multi, g.oneWave);
+    if (g.oneWave && int(threadIdx.x) >= PSR_WAVE) return;
+    if (m.form == 0)
+        cg_mixed_row_solve<false>(psr_bid, P, G, maps, m, g, sh, r0, rows, b, x, rOut, state, iters, resid, trueRel);
+    else
+        cg_mixed_row_solve<true>(psr_bid, P, G, maps, m, g, sh, r0, rows, b, x, rOut, state, iters, resid, trueRel);
 }
 __global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(kRowMixedWaves))) cg_mixed_row(
     CgParams P, RowMapArgs maps, const float* __restrict__ b, float* x, float* rOut, float4* state, float4* slots,
