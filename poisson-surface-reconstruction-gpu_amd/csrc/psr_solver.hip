@@ -2232,8 +2232,26 @@ __device__ __forceinline__ void neighbour_columns_body(int psr_bid, int psr_nbid
         for (size_t i = t; i < nDense / 4; i += stride) dense4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (t < nDense % 4) dense[nDense - 1 - t] = 0.f;
     }
+    const size_t n = size_t(27) * M;
+    if (cols) {
+        // 16 bytes an entry: a workgroup's entries side by side, an entry a thread at a time
+#pragma unroll
+        for (int k = 0; k < kColumnItems; ++k) {
+            const size_t e = (size_t(psr_bid) * kColumnItems + k) * kThreads + threadIdx.x;
+            if (e >= n) break;
+            const int nb = neigh[e];
+            float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (nb >= 0) {
+                const float4 b = basis[nb];
+                col = make_float4(b.x, b.y, b.z, dx[nb]);
+            }
+            nbrCol[e] = col;
+            dCol[e] = col.w;
+        }
+        return;
+    }
     // four entries a thread (the columns are one array, 16-byte aligned)
-    const size_t n = size_t(27) * M, e = kColumnItems * t;
+    const size_t e = kColumnItems * t;
     if (e >= n) return;
     static_assert(kColumnItems == 4, "a 16-byte load and store");
     int nb[kColumnItems];
@@ -2246,11 +2264,6 @@ __device__ __forceinline__ void neighbour_columns_body(int psr_bid, int psr_nbid
     float d[kColumnItems];
 #pragma unroll
     for (int k = 0; k < kColumnItems; ++k) d[k] = nb[k] < 0 ? 0.f : dx[nb[k]];
-    if (cols)
-        for (int k = 0; k < kColumnItems && e + k < n; ++k) {
-            const float4 b = nb[k] < 0 ? make_float4(0.f, 0.f, 0.f, 0.f) : basis[nb[k]];
-            nbrCol[e + k] = make_float4(b.x, b.y, b.z, d[k]);
-        }
     if (e + kColumnItems <= n) *reinterpret_cast<float4*>(dCol + e) = make_float4(d[0], d[1], d[2], d[3]);
     else
         for (int k = 0; e + k < n; ++k) dCol[e + k] = d[k];
