@@ -281,6 +281,14 @@ __device__ __forceinline__ void dist_insert(float (&best)[K], float d) {
     best[0] = fminf(best[0], d);
 }
 
+// x into the ascending list of the K lowest indices.
+template <int K>
+__device__ __forceinline__ void index_insert(unsigned (&low)[K], unsigned x) {
+#pragma unroll
+    for (int j = K - 1; j > 0; --j) low[j] = max(low[j - 1], min(low[j], x));
+    low[0] = min(low[0], x);
+}
+
 // Orders a wave's LDS writes before its later reads of other lanes' values.
 __device__ __forceinline__ void wave_publish() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -382,40 +390,55 @@ __device__ __forceinline__ void knn_search(float3 p, int sub, int kk, const Grid
             if (j == kk - 1) dk = best[j];
         if (all || (dk < INFINITY && sqrtf(dk) * (1.0f + 1e-6f) + g.eps < cover)) break;
     }
+    int added = 0;
     for_points<LANES>(o, r, c, sub, g.G, spos, start, [&](float4 q) {
         const Cand e = candidate(q, p);
-        if (!(__uint_as_float(unsigned(e >> 32)) <= dk)) return;
+        if (!(__uint_as_float(unsigned(e >> 32)) <= dk) || added > kListCap) return;
         const int at = atomicAdd(cnt, 1);
+        ++added;
         if (at < kListCap) list[at] = e;
     });
     wave_publish();  // the lanes of p read each other's entries
-    const int m = *cnt;
-    if (m >= kk && m <= kListCap) {
-        for (int j = sub; j < m; j += LANES) {
-            const Cand e = list[j];
-            int rank = 0;
-            for (int i = 0; i < m; ++i) rank += list[i] < e ? 1 : 0;
-            if (rank < kk) found[rank * stride] = cand_index(e);
+    int m = *cnt;
+    const bool ties = m > kListCap;
+    unsigned tie[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) tie[j] = 0x7fffffffu;
+    if (ties) {
+        // more points at the kk-th distance than the list holds: once more, the
+        // nearer ones (fewer than kk) to the list and of those at the kk-th
+        // distance the lowest indices, a median a place as for the distances
+        wave_publish();
+        if (sub == 0) *cnt = 0;
+        wave_publish();
+        for_points<LANES>(o, r, c, sub, g.G, spos, start, [&](float4 q) {
+            const Cand e = candidate(q, p);
+            const float d = __uint_as_float(unsigned(e >> 32));
+            if (d < dk) list[atomicAdd(cnt, 1)] = e;
+            else if (d == dk) index_insert<K>(tie, unsigned(e));
+        });
+#pragma unroll
+        for (int w = 1; w < LANES; w <<= 1) {
+            unsigned other[K];
+#pragma unroll
+            for (int j = 0; j < K; ++j) other[j] = __shfl_xor(tie[j], w, PSR_WAVE);
+#pragma unroll
+            for (int j = 0; j < K; ++j) index_insert<K>(tie, other[j]);
         }
-        return;
+        wave_publish();
+        m = *cnt;
     }
-    // more ties at the kk-th distance than the list holds, or fewer than kk
-    // points with a distance at all: one smallest candidate after another
-    if (sub != 0) return;
-    Cand prev = 0;
-    for (int j = 0; j < kk; ++j) {
-        Cand next = kNone;
-        for (int x = o.x0; x <= o.x1; ++x)
-            for (int y = o.y0; y <= o.y1; ++y) {
-                const unsigned row = (unsigned(x) * unsigned(g.G) + unsigned(y)) * unsigned(g.G);
-                const int e = start[row + unsigned(o.z1) + 1];
-                for (int s = start[row + unsigned(o.z0)]; s < e; ++s) {
-                    const Cand q = candidate(spos[s], p);
-                    if ((j == 0 || q > prev) && q < next) next = q;
-                }
-            }
-        found[j * stride] = cand_index(next);
-        prev = next;
+    for (int j = sub; j < m; j += LANES) {
+        const Cand e = list[j];
+        int rank = 0;
+        for (int i = 0; i < m; ++i) rank += list[i] < e ? 1 : 0;
+        if (rank < kk) found[rank * stride] = cand_index(e);
+    }
+    // the places that are left: the ties, or no point (fewer than kk have a distance)
+    if (m < kk && sub == 0) {
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            if (m + j < kk) found[(m + j) * stride] = int(tie[j]);
     }
 }
 
