@@ -211,22 +211,33 @@ __global__ void __launch_bounds__(kThreads) ne_cell_starts(const unsigned* __res
         if (c0 + k <= cells) start[c0 + k] = first[k];
 }
 
+// 1 / sqrt(x) and 1 / x to FP64's last bit or two: the hardware's estimate and
+// two Newton steps.
+__device__ __forceinline__ double rsqrt_newton(double x) {
+    double r = __builtin_amdgcn_rsq(x);
+    r = __fma_rn(0.5 * r, __fma_rn(-x * r, r, 1.0), r);
+    return __fma_rn(0.5 * r, __fma_rn(-x * r, r, 1.0), r);
+}
+__device__ __forceinline__ double rcp_newton(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = __fma_rn(r, __fma_rn(-x, r, 1.0), r);
+    return __fma_rn(r, __fma_rn(-x, r, 1.0), r);
+}
+
 // Cyclic Jacobi on a symmetric 3 x 3 matrix, in FP64: eigenvalues on the
-// diagonal, eigenvectors in the columns of V.  The rotation's tangent is only
-// an estimate (FP32): any t leaves cos and sin orthonormal to FP64, and what it
-// leaves of the off-diagonal entry the next sweep takes; the matrix and V are
-// transformed in FP64 throughout.  A quarter of the instructions of the
-// rotation with two FP64 roots and three FP64 quotients, and as exact.
+// diagonal, eigenvectors in the columns of V.  With theta = (a_qq - a_pp) / (2
+// a_pq), t = sign(theta) / (|theta| + sqrt(theta^2 + 1)) is formed without the
+// quotient theta.  Roots and reciprocals by Newton steps in place of the
+// library's correctly rounded ones, whose instructions were three quarters of a
+// rotation's.
 template <int P, int Q>
 __device__ __forceinline__ void jacobi_rotate(double (&A)[3][3], double (&V)[3][3]) {
     constexpr int R = 3 - P - Q;
     if (A[P][Q] == 0.0) return;
-    const float theta = float((A[Q][Q] - A[P][P]) * __builtin_amdgcn_rcp(2.0 * A[P][Q]));
-    const float tf = copysignf(__builtin_amdgcn_rcpf(fabsf(theta) + __builtin_amdgcn_sqrtf(theta * theta + 1.0f)), theta);
-    const double t = double(tf), u = __fma_rn(t, t, 1.0);  // u in [1, 2]
-    double cs = __builtin_amdgcn_rsq(u);                    // 1 / sqrt(u), two Newton steps to FP64
-    cs = __fma_rn(0.5 * cs, __fma_rn(-u * cs, cs, 1.0), cs);
-    cs = __fma_rn(0.5 * cs, __fma_rn(-u * cs, cs, 1.0), cs);
+    const double dif = A[Q][Q] - A[P][P], h = 2.0 * A[P][Q], x = __fma_rn(dif, dif, h * h);
+    if (x == 0.0) return;  // the squares underflow: nothing to rotate beside the entries that do not
+    const double t = dif == 0.0 ? 1.0 : (dif > 0.0 ? h : -h) * rcp_newton(fabs(dif) + x * rsqrt_newton(x));
+    const double cs = rsqrt_newton(__fma_rn(t, t, 1.0));
     const double sn = t * cs;
     const double app = A[P][P], aqq = A[Q][Q], apq = A[P][Q], arp = A[R][P], arq = A[R][Q];
     const double cc = cs * cs, ss = sn * sn, sc = sn * cs;
