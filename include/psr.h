@@ -139,6 +139,8 @@ enum {
                                    S = 2^D + 1, (x, y, z) the edge's lower grid corner */
     PSR_ARRAY_WELDED_VERTICES,  /* float [welded n_vertices][3], after psr_weld_mesh */
     PSR_ARRAY_WELDED_TRIANGLES, /* int32 [n_triangles][3], after psr_weld_mesh */
+    PSR_ARRAY_SUBDIV_TILE_SIGNS, /* int32 per bounded one-root tile of the last subdivision working set: the sign of a
+                                    tile that the bound left out, else 0; empty where no bound was taken */
     PSR_ARRAY_COUNT_
 };
 

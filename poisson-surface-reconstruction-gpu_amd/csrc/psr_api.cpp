@@ -233,6 +233,8 @@ int psr_create(const psr_config* cfg, void* hip_stream, psr_ctx** out) {
         if (const char* e = std::getenv("PSR_CG_ROWS_PER_WG")) c.cgRowsPerWg = std::max(0, std::atoi(e));
         // test override of the CG barriers' spin bound (forces their time-out path)
         if (const char* e = std::getenv("PSR_CG_SPIN_LIMIT")) c.cgSpinLimit = std::max(0, std::atoi(e));
+        // test override of the number of subdivision tiles from which a bound leaves some out
+        if (const char* e = std::getenv("PSR_SUBDIV_BOUND_TILES")) c.boundTilesMin = std::max(0, std::atoi(e));
         PSR_HIP_CHECK(hipGetDevice(&c.device));
         if (hip_stream) {
             c.stream = static_cast<hipStream_t>(hip_stream);
@@ -554,6 +556,7 @@ int psr_export(psr_ctx* ctx, int id, void* dst, uint64_t bytes, uint64_t* needed
         case PSR_ARRAY_MESH_VERTEX_KEYS: src = {c.mesh.keys, size_t(4) * c.mesh.nv, 0}; break;
         case PSR_ARRAY_WELDED_VERTICES: src = {c.mesh.weldedVertices, size_t(12) * c.mesh.weldedNv, 0}; break;
         case PSR_ARRAY_WELDED_TRIANGLES: src = {c.mesh.weldedTriangles, size_t(12) * c.mesh.weldedNt, 0}; break;
+        case PSR_ARRAY_SUBDIV_TILE_SIGNS: src = {c.mc.tileState, size_t(4) * c.mc.boundTiles, 0}; break;
         case PSR_ARRAY_TABLE_DOT: src = {c.tables.dot, size_t(8) * c.tables.res * c.tables.res, 0}; break;
         case PSR_ARRAY_TABLE_DDOT: src = {c.tables.ddot, size_t(8) * c.tables.res * c.tables.res, 0}; break;
         case PSR_ARRAY_TABLE_D2DOT: src = {c.tables.d2dot, size_t(8) * c.tables.res * c.tables.res, 0}; break;

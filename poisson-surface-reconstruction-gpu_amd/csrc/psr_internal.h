@@ -173,6 +173,8 @@ struct MainMc {
     int nCross = 0, nTri = 0, nRoots = 0;
     int rootsPerDepth[PSR_MAX_DEPTH + 1] = {0};
     bool q1Fired = false;  // the level-local child 0 rule changed a parent somewhere
+    const int* tileState = nullptr;  // the bounded one-root tiles of the last working set: 0, or the sign of a left-out one
+    int boundTiles = 0;
 };
 
 // Small per-call results written by the kernels and read back in one copy.
@@ -241,6 +243,7 @@ struct Ctx {
     int cgRowsPerWg = 0;         // rows per CG workgroup (0: default)
     int cgRowTarget = 0;         // batch: rows a CG workgroup takes (0: the single-cloud plan)
     int cgSpinLimit = -1;        // spin bound of the CG barriers (-1: the default)
+    int boundTilesMin = -1;      // one-root subdivision tiles from which they are bounded (-1: the default)
     bool indefinite[PSR_MAX_DEPTH + 1] = {};  // the depth's operator after the 1e-6 drop is indefinite
     template <class T>
     T* buf(const char* name, size_t count) {

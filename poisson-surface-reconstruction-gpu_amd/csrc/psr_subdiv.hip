@@ -2063,7 +2063,8 @@ void extract_mesh_b(Ctx& c) {
         size_t oneTiles = 0;
         for (int k = 0; k < nSets; ++k)
             if (D - sets[k].rd >= 3) oneTiles += setCells[k] / kTile;
-        float* rootPoly = denseHalo && oneTiles >= size_t(current_recorder() ? 1 : kBoundTilesMin)
+        const size_t boundMin = c.boundTilesMin >= 0 ? size_t(c.boundTilesMin) : size_t(current_recorder() ? 1 : kBoundTilesMin);
+        float* rootPoly = denseHalo && oneTiles >= std::max<size_t>(1, boundMin)
                               ? c.buf<float>("sub_root_poly", size_t(kPolyWords) * nOneRoots)
                               : nullptr;
         for (const SetDesc& S : sets) {
@@ -2164,6 +2165,8 @@ void extract_mesh_b(Ctx& c) {
                 if (rootPoly) {
                     sign = c.buf<int>("sub_tile_sign", nOne);
                     state = c.buf<int>("sub_tile_state", nOne);
+                    c.mc.tileState = state;
+                    c.mc.boundTiles = nOne;
                     PSR_LAUNCH(sub_bound, div_up(nOne, kBoundTiles), 0, st, gr, dtiles, nOne,
                                static_cast<const float*>(rootPoly), isoDev, sign, state, tileCnt);
                 }
