@@ -392,8 +392,8 @@ __device__ __forceinline__ void divergence_leaf_nodes(int block, int offD, int n
     const int3 fo = decode_func_index(enc[o], D);
     const DivRows rows(ddotT, res, fo);
     double acc = 0;
-    const float sc = float(2 << D);
     if (*q1Fired == 0 && neigh[13 * M + o] == o) {
+        const float sc = float(2 << D);
         double wy[3], wz[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {  // past the domain: not used
@@ -423,23 +423,9 @@ __device__ __forceinline__ void divergence_leaf_nodes(int block, int offD, int n
             int nb[9];
 #pragma unroll
             for (int i = 0; i < 9; ++i) nb[i] = neigh[(9 * x + i) * M + o];
-            float3 v[9];
-            int f[9];
 #pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                const int j = nb[i] != -1 ? nb[i] - offD : 0;
-                v[i] = load_field(&vf[j], sc);
-                f[i] = enc[offD + j];
-            }
-#pragma unroll
-            for (int i = 0; i < 9; ++i) {
-                const int3 fj = decode_func_index(f[i], D);
-                double s = double(v[i].x) * rows.x[fj.x];
-                s += double(v[i].y) * rows.y[fj.y];
-                s += double(v[i].z) * rows.z[fj.z];
-                if (nb[i] != -1) acc += s;
-                if (i % 3 == 2) __builtin_amdgcn_sched_barrier(0);  // 27 table values in flight take 43 more registers
-            }
+            for (int i = 0; i < 9; ++i)
+                if (nb[i] != -1) acc += div_term(nb[i] - offD, offD, D, rows, enc, vf);
         }
     }
     div[o] = float(acc);
