@@ -454,6 +454,15 @@ __device__ __forceinline__ double uniform(double v) {
     const long long b = __double_as_longlong(v);
     return __hiloint2double(__builtin_amdgcn_readfirstlane(int(b >> 32)), __builtin_amdgcn_readfirstlane(int(b)));
 }
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// The group of workgroup `bid` (a batch's workgroups take bid and the arguments from memory).
+__device__ __forceinline__ CgGroup uniform_group(const CgParams& P, int bid) {
+    int gi = 0;
+    while (gi + 1 < P.ngroups && bid >= P.g[gi + 1].firstWg) ++gi;
+    const CgGroup& g = P.g[gi];
+    return CgGroup{uniform(g.depth),   uniform(g.rowBegin),  uniform(g.rows), uniform(g.firstWg),
+                   uniform(g.wgs),     uniform(g.rowsPerWg), uniform(g.indef)};
+}
 
 struct RowShared {
     // the rows' places; or, in a one-wave group with own weights, lane t's 27
@@ -610,10 +619,13 @@ __device__ __forceinline__ T row_product(const RowMap& m, const RowMapArgs& a, R
             for (int k = 0; k < 7; ++k)
                 if (first + k < 13) p[k] = sh.place[first + k][t];
         };
+        float rowWeights[27];  // all on their way at once
+#pragma unroll
+        for (int q = 0; q < 27; ++q) rowWeights[q] = (a.val + size_t(q) * M)[unsigned(i)];
         in_parts(place_words, [&](int first, float (&v)[15]) {
 #pragma unroll
             for (int k = 0; k < 15; ++k)
-                if (first + k < 27) v[k] = (a.val + size_t(first + k) * M)[unsigned(i)];
+                if (first + k < 27) v[k] = rowWeights[first + k];
         });
         return acc;
     }
@@ -670,7 +682,9 @@ __device__ __forceinline__ bool row_group_sum(double (&v)[N], RowShared& sh, Row
         wave_sync_memory();
         return true;
     }
-    const int lane = int(__lane_id()), wave = threadIdx.x / PSR_WAVE;
+    int t = int(threadIdx.x);
+    asm volatile("" : "+v"(t));  // lane, wave and addresses are formed anew, not spilled from sum to sum
+    const int lane = t % PSR_WAVE, wave = t / PSR_WAVE;
     g.parity ^= 1u;
     if (g.multi) __builtin_amdgcn_s_waitcnt(0);
     if (lane == 0) {
@@ -696,8 +710,6 @@ __device__ __forceinline__ bool row_group_sum(double (&v)[N], RowShared& sh, Row
     const __amdgpu_buffer_rsrc_t rs = vec_rsrc(g.region + size_t(g.phase & 1u) * g.blocks * kSlotStride,
                                                sizeof(float4) * size_t(g.blocks) * kSlotStride);
     const float stamp = __uint_as_float(g.phase);
-    int t = int(threadIdx.x);
-    asm volatile("" : "+v"(t));  // the slot's address is formed anew, not spilled from sum to sum
     if (t < N * g.ownBlocks) {
         const int b = t / N, n = t % N;
         const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(block_total(b, n)));
@@ -707,7 +719,7 @@ __device__ __forceinline__ bool row_group_sum(double (&v)[N], RowShared& sh, Row
     double part[N];
 #pragma unroll
     for (int n = 0; n < N; ++n) part[n] = 0.0;
-    for (int k = int(threadIdx.x); k - int(threadIdx.x) < g.blocks; k += kRowThreads) {
+    for (int k = t; k - t < g.blocks; k += kRowThreads) {
         const bool mine = k < g.blocks;
         float4 got[N];
         for (unsigned spins = 0;; ++spins) {
@@ -761,7 +773,7 @@ __device__ __forceinline__ RowGroup row_group(const CgParams& P, const CgGroup& 
     // whose other waves add exact zeros)
     g.oneWave = !g.multi && G.rows <= PSR_WAVE;
     g.phase = g.parity = 0u;
-    g.spinLimit = P.spinLimit;
+    g.spinLimit = unsigned(uniform(int(P.spinLimit)));
     g.errFlag = errFlag;
     return g;
 }
@@ -779,7 +791,7 @@ __device__ __forceinline__ void cg_fp32_row_solve(int psr_bid, const CgParams& P
                                                   const RowMap& m, RowGroup& g, RowShared& sh, int r0, int rows,
                                                   const float* __restrict__ b, float* __restrict__ x, float2* state,
                                                   int* __restrict__ iters, double* __restrict__ resid) {
-    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M, i = r0 + t;
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = uniform(P.M), i = r0 + t;
     const bool own = t < rows;
     const int* __restrict__ neigh = maps.neigh;
     float w[27];
@@ -836,9 +848,8 @@ __device__ __forceinline__ void cg_fp32_row_body(int psr_bid, int psr_nbid, cons
                                                  float4* slots, int* __restrict__ iters, double* __restrict__ resid,
                                                  int* errFlag) {
     __shared__ RowShared sh;
-    int gi = 0;
-    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
-    const CgGroup G = P.g[gi];
+    psr_bid = uniform(psr_bid);
+    const CgGroup G = uniform_group(P, psr_bid);
     const int local = psr_bid - G.firstWg, r0 = G.rowBegin + local * G.rowsPerWg;
     const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0;
     RowGroup g = row_group(P, G, local, slots, errFlag);
@@ -1126,7 +1137,7 @@ __device__ __forceinline__ void cg_mixed_row_solve(int psr_bid, const CgParams& 
                                                    const float* __restrict__ b, float* x, float* rOut, float4* state,
                                                    int* __restrict__ iters, double* __restrict__ resid,
                                                    double* __restrict__ trueRel) {
-    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = P.M, i = r0 + t;
+    const int local = psr_bid - G.firstWg, t = int(threadIdx.x), M = uniform(P.M), i = r0 + t;
     const bool own = t < rows;
     const int* __restrict__ neigh = maps.neigh;
     float w[27];
@@ -1281,9 +1292,8 @@ __device__ __forceinline__ void cg_mixed_row_body(int psr_bid, int psr_nbid, con
                                                   float4* slots, int* __restrict__ iters, double* __restrict__ resid,
                                                   double* __restrict__ trueRel, int* errFlag) {
     __shared__ RowShared sh;
-    int gi = 0;
-    while (gi + 1 < P.ngroups && int(psr_bid) >= P.g[gi + 1].firstWg) ++gi;
-    const CgGroup G = P.g[gi];
+    psr_bid = uniform(psr_bid);
+    const CgGroup G = uniform_group(P, psr_bid);
     const int local = psr_bid - G.firstWg, r0 = G.rowBegin + local * G.rowsPerWg;
     const int rows = min(G.rowBegin + G.rows, r0 + G.rowsPerWg) - r0;
     RowGroup g = row_group(P, G, local, slots, errFlag);
