@@ -448,6 +448,9 @@ int Batch::run(const psr_points* pts, uint32_t count, psr_mesh* outs, std::vecto
             },
             true);
         if (cand >= 0) tuner().report(tkey, cand, elapsed(b.ev[10], b.ev[11]));
+        size_t tiles = 0;
+        for (uint32_t i : live) tiles += bounded_tiles(clouds_[i]->c);
+        for (uint32_t i : live) clouds_[i]->c.batchTiles = tiles;
         phase([&](Ctx& c, uint32_t) { extract_mesh_b(c); }, false);
         for (uint32_t i : live) {
             psr_ctx* w = clouds_[i];

@@ -243,6 +243,7 @@ struct Ctx {
     int cgRowsPerWg = 0;         // rows per CG workgroup (0: default)
     int cgRowTarget = 0;         // batch: rows a CG workgroup takes (0: the single-cloud plan)
     int cgSpinLimit = -1;        // spin bound of the CG barriers (-1: the default)
+    size_t batchTiles = 0;       // batch: bounded_tiles of all its clouds
     int boundTilesMin = -1;      // one-root subdivision tiles from which they are bounded (-1: the default)
     bool indefinite[PSR_MAX_DEPTH + 1] = {};  // the depth's operator after the 1e-6 drop is indefinite
     template <class T>
@@ -339,6 +340,8 @@ void extract_mesh(Ctx& c);
 // the subdivision and the output
 void extract_mesh_a(Ctx& c);
 void extract_mesh_b(Ctx& c);
+// After that wait, before extract_mesh_b: the subdivision tiles that a bound could leave out.
+size_t bounded_tiles(Ctx& c);
 // Mesh counts of a deferred extraction, read from the mailbox after the final wait.
 void finish_mesh(Ctx& c);
 // Checks a cloud and resets a context's per-call state (PSR_OK, or a status

@@ -806,7 +806,9 @@ constexpr auto sub_corner_values_small = sub_corner_values<false, kSmallThreads>
 // 1127 us, the bounds included.  Below kBoundTilesMin tiles the GPU takes nearly
 // all of them at once and the bound is not taken: its launch costs more than the
 // tiles left out (a call with 284 tiles 523 us without and 538 with it, with 4282
-// tiles 650 and 630).  A batch has the tiles of all its clouds in one launch.
+// tiles 650 and 630).  A batch has the tiles of all its clouds in one launch, and
+// their sum decides (two clouds of 4k points at depth 5: 483 us without, 492 with
+// the bound).
 constexpr float kBoundMargin = 2e-4f;
 constexpr int kPolyWords = 32;  // per root: 27 coefficients, x-major, and the sum of the list's |d_x|
 constexpr int kBoundTilesMin = 2048;
@@ -1952,6 +1954,13 @@ int grid_tile_words(int D, int rd, int* haloOut = nullptr) {
     return halo + fac + ((27 * (rd + 1) + 3) & ~3) * kTw;
 }
 
+// Tiles of one root: of the roots 8 cells or more a side.
+size_t one_root_tiles(const MainMc& mm, int D) {
+    size_t n = 0;
+    for (int d = 0; d <= D - 3; ++d) n += (size_t(mm.rootsPerDepth[d]) << (3 * (D - d))) / kTile;
+    return n;
+}
+
 // Default depth-D virtual cells per chunk of subdivision sets; a set larger
 // than the chunk size forms a chunk of its own.
 constexpr size_t kChunkCells = size_t(1) << 24;
@@ -1969,6 +1978,11 @@ void extract_mesh_a(Ctx& c) {
     c.mc = MainMc{};
     c.mesh.deferred = false;
     depth_mc_launch(c, c.mc, mainV, mainKey, outT);
+}
+
+size_t bounded_tiles(Ctx& c) {
+    depth_mc_read(c, c.mc);
+    return c.mc.q1Fired ? 0 : one_root_tiles(c.mc, c.oct.L.D);
 }
 
 // After the wait for the depth-D counts: the subdivision and the output.
@@ -2060,11 +2074,10 @@ void extract_mesh_b(Ctx& c) {
         // tiles read d_x from dense per-depth grids when the octree is geometric
         const bool denseHalo = !mm.q1Fired;
         // the roots' polynomials, where the tiles are bounded
-        size_t oneTiles = 0;
-        for (int k = 0; k < nSets; ++k)
-            if (D - sets[k].rd >= 3) oneTiles += setCells[k] / kTile;
-        const size_t boundMin = c.boundTilesMin >= 0 ? size_t(c.boundTilesMin) : size_t(current_recorder() ? 1 : kBoundTilesMin);
-        float* rootPoly = denseHalo && oneTiles >= std::max<size_t>(1, boundMin)
+        const size_t oneTiles = one_root_tiles(mm, D);
+        const size_t launchTiles = current_recorder() ? c.batchTiles : oneTiles;  // of a batch's clouds together
+        const size_t boundMin = c.boundTilesMin >= 0 ? size_t(c.boundTilesMin) : size_t(kBoundTilesMin);
+        float* rootPoly = denseHalo && oneTiles > 0 && launchTiles >= boundMin
                               ? c.buf<float>("sub_root_poly", size_t(kPolyWords) * nOneRoots)
                               : nullptr;
         for (const SetDesc& S : sets) {
