@@ -411,8 +411,11 @@ __device__ __forceinline__ void divergence_leaf_nodes(int block, int offD, int n
             for (int i = 0; i < 9; ++i) v[i] = load_field(&vf[nb[i] != -1 ? nb[i] - offD : 0], sc);
 #pragma unroll
             for (int i = 0; i < 9; ++i) {
-                double s = double(v[i].x) * wx;
-                s += double(v[i].y) * wy[i / 3];
+                // rounded as div_term rounds it: y's product by itself, the other two fused onto it (here the
+                // compiler would choose x's, and one value in 170k differ in its last bit)
+                double p = double(v[i].y) * wy[i / 3];
+                asm("" : "+v"(p));
+                double s = p + double(v[i].x) * wx;
                 s += double(v[i].z) * wz[i % 3];
                 if (nb[i] != -1) acc += s;
             }
