@@ -496,16 +496,22 @@ void build_tables(Ctx& c) {
     Tables& t = c.tables;
     t.res = res;
     size_t n = size_t(res) * res;
-    t.dot = c.buf<double>("table_dot", n);
-    t.ddot = c.buf<double>("table_ddot", n);
-    t.ddotT = c.buf<double>("table_ddot_t", n);
-    t.d2dot = c.buf<double>("table_d2dot", n);
+    const int functions = res;  // of all depths
+    std::vector<float> weights(27 * size_t(D + 1), 0.f);
+    BlockParts parts;
+    const size_t oDot = parts.add(sizeof(double) * n), oDdot = parts.add(sizeof(double) * n), oDdotT = parts.add(sizeof(double) * n),
+                 oD2dot = parts.add(sizeof(double) * n), oBand = parts.add(sizeof(double2) * 3 * functions),
+                 oWeights = parts.add(sizeof(float) * weights.size());
+    char* block = c.buf<char>("tables", parts.bytes);
+    t.dot = reinterpret_cast<double*>(block + oDot);
+    t.ddot = reinterpret_cast<double*>(block + oDdot);
+    t.ddotT = reinterpret_cast<double*>(block + oDdotT);
+    t.d2dot = reinterpret_cast<double*>(block + oD2dot);
     build_tables_kernel<<<div_up(n, 256), 256, 0, c.stream>>>(res, t.dot, t.ddot, t.ddotT, t.d2dot);
     PSR_HIP_CHECK(hipGetLastError());
     // The inner products of each depth's functions with those at offsets -1, 0
     // and 1 (a depth's functions are consecutive), copied out in one piece.
-    const int functions = res;  // of all depths
-    double2* band = c.buf<double2>("table_band", size_t(3) * functions);
+    double2* band = reinterpret_cast<double2*>(block + oBand);
     gather_band<<<div_up(size_t(3) * functions, 256), 256, 0, c.stream>>>(res, D, t.dot, t.d2dot, band);
     std::vector<double2> hb(size_t(3) * functions);
     PSR_HIP_CHECK(hipMemcpyAsync(hb.data(), band, sizeof(double2) * hb.size(), hipMemcpyDeviceToHost, c.stream));
@@ -514,7 +520,6 @@ void build_tables(Ctx& c) {
     // offset differ from function to function in their last bits only, and the
     // entry rounds to one float for every triple of them or the depth has no
     // table of entries.
-    std::vector<float> weights(27 * size_t(D + 1), 0.f);
     bool unique = true;
     for (int d = 0; d <= D; ++d) {
         std::vector<double2> distinct[3];
@@ -541,7 +546,7 @@ void build_tables(Ctx& c) {
         }
     }
     if (unique) {
-        t.weights = c.buf<float>("table_weights", weights.size());
+        t.weights = reinterpret_cast<float*>(block + oWeights);
         PSR_HIP_CHECK(hipMemcpyAsync(t.weights, weights.data(), sizeof(float) * weights.size(), hipMemcpyHostToDevice, c.stream));
         PSR_HIP_CHECK(hipStreamSynchronize(c.stream));
     }

@@ -60,6 +60,17 @@ class Arena {
     int allocs_ = 0;
 };
 
+// Parts of one arena block, at multiples of 256 bytes: an allocation of its own
+// for each of a stage's buffers costs a context's first call 20 to 40 us.
+struct BlockParts {
+    size_t bytes = 0;
+    size_t add(size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    }
+};
+
 // 1-D inner-product tables for the configured depth, [a + res * b].
 struct Tables {
     int res = 0;
@@ -236,6 +247,7 @@ struct Ctx {
     void* hostStage = nullptr;          // pinned, mapped staging for small uploads
     void* stageDev = nullptr;           // device view of hostStage
     size_t hostStageBytes = 0;
+    int cus = 0;                 // compute units of the device
     int cgMaxWgs = 0;            // resident workgroups of the CG kernels with several rows per thread
     int cgMaxWgsRow = 0;         // resident workgroups of the one-row-per-thread CG kernels
     int cgMaxWgsMinres = 0;      // resident workgroups of the MINRES kernel (indefinite depths, mixed form)

@@ -610,17 +610,13 @@ void build_knn_grid(Ctx& c, const char* base, unsigned stride, int n, int k, Gri
     int bits = 1;
     while ((cells - 1) >> bits) ++bits;
     // one block of the arena: a context's first call allocates once
-    size_t at = 0;
-    auto part_of = [&](size_t bytes) {
-        const size_t o = at;
-        at += (bytes + 255) / 256 * 256;
-        return o;
-    };
+    BlockParts parts;
+    auto part_of = [&](size_t bytes) { return parts.add(bytes); };
     const size_t oPart = part_of(sizeof(float) * 6 * nb), oGrid = part_of(sizeof(GridSpec)), oKey = part_of(4 * size_t(n)),
                  oVal = part_of(4 * size_t(n)), oKt = part_of(4 * size_t(n)), oVt = part_of(4 * size_t(n)),
                  oPos = part_of(16 * size_t(n)), oSpos = part_of(16 * size_t(n)),
                  oStart = part_of(4 * (size_t(cells) + 1));
-    char* block = c.buf<char>("ne_grid", at);
+    char* block = c.buf<char>("ne_grid", parts.bytes);
     float* part = reinterpret_cast<float*>(block + oPart);
     grid = reinterpret_cast<GridSpec*>(block + oGrid);
     unsigned* key = reinterpret_cast<unsigned*>(block + oKey);

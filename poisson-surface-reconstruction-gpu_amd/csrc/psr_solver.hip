@@ -2387,37 +2387,37 @@ void solve_depths(Ctx& c) {
     // which the compiler may give other register counts: a budget is the
     // smaller occupancy of the two forms, so that a plan made for one cloud
     // also fits the merged launch.
+    auto occupancy = [](const void* single, const void* batched, int threads) {
+        int a = 0, b = 0;
+        PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, single, threads, 0));
+        PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, batched, threads, 0));
+        return std::min(a, b);
+    };
     if (c.cgMaxWgs <= 0) {
-        auto occupancy = [](const void* single, const void* batched, int threads) {
-            int a = 0, b = 0;
-            PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, single, threads, 0));
-            PSR_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, batched, threads, 0));
-            return std::min(a, b);
-        };
         const void* rowQueue = mixed ? multi_queue_kernel_of<cg_mixed_row_k>(cg_mixed_row)
                                      : multi_queue_kernel_of<cg_fp32_row_k>(cg_fp32_row);
         const void* genQueue = mixed ? multi_queue_kernel_of<cg_mixed_all_depths_k>(cg_mixed_all_depths)
                                      : multi_queue_kernel_of<cg_all_depths_k>(cg_all_depths);
-        int cus = 0;
         const int perRow = occupancy(rowKernel, rowQueue, kRowThreads), perGen = occupancy(genKernel, genQueue, kCgThreads);
-        const int perMinres = occupancy(reinterpret_cast<const void*>(cg_mixed_minres),
-                                        multi_queue_kernel_of<cg_mixed_minres_k>(cg_mixed_minres), kCgThreads);
-        PSR_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device));
-        c.cgMaxWgsRow = std::max(0, perRow * cus);
-        c.cgMaxWgs = std::max(1, perGen * cus);
-        c.cgMaxWgsMinres = std::max(1, perMinres * cus);
-        c.cgMaxWgsChip[0] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip4),
-                                            multi_queue_kernel_of<cg_minres_chip4_k>(cg_minres_chip4), kCgThreads);
-        c.cgMaxWgsChip[1] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip8),
-                                            multi_queue_kernel_of<cg_minres_chip8_k>(cg_minres_chip8), kCgThreads);
-        c.cgMaxWgsChip[2] = cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip16),
-                                            multi_queue_kernel_of<cg_minres_chip16_k>(cg_minres_chip16), kCgThreads);
+        PSR_HIP_CHECK(hipDeviceGetAttribute(&c.cus, hipDeviceAttributeMultiprocessorCount, c.device));
+        c.cgMaxWgsRow = std::max(0, perRow * c.cus);
+        c.cgMaxWgs = std::max(1, perGen * c.cus);
     }
     // the mixed form solves indefinite depths with MINRES, in a launch of its
     // own (the MINRES kernel) after the CG launch of the other depths
     bool isMinres[PSR_MAX_DEPTH + 1];
     bool anyIndef = false;
     for (int d = 0; d <= D; ++d) anyIndef |= (isMinres[d] = mixed && c.indefinite[d]);
+    if (anyIndef && c.cgMaxWgsMinres <= 0) {
+        c.cgMaxWgsMinres = std::max(1, c.cus * occupancy(reinterpret_cast<const void*>(cg_mixed_minres),
+                                                         multi_queue_kernel_of<cg_mixed_minres_k>(cg_mixed_minres), kCgThreads));
+        c.cgMaxWgsChip[0] = c.cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip4),
+                                              multi_queue_kernel_of<cg_minres_chip4_k>(cg_minres_chip4), kCgThreads);
+        c.cgMaxWgsChip[1] = c.cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip8),
+                                              multi_queue_kernel_of<cg_minres_chip8_k>(cg_minres_chip8), kCgThreads);
+        c.cgMaxWgsChip[2] = c.cus * occupancy(reinterpret_cast<const void*>(cg_minres_chip16),
+                                              multi_queue_kernel_of<cg_minres_chip16_k>(cg_minres_chip16), kCgThreads);
+    }
     auto need_of = [&](int rpw, bool minresSet) {
         long long w = 0;
         for (int d = 0; d <= D; ++d)
@@ -2484,11 +2484,11 @@ void solve_depths(Ctx& c) {
         const int want = widest <= 4 * kCgThreads ? 0 : (widest <= 8 * kCgThreads ? 1 : 2);
         if (widest <= 16 * kCgThreads && wgM <= c.cgMaxWgsChip[want] && wgM <= kFoldParts * kCgThreads) chip = want;
     }
-    const int capMinres = chip >= 0 ? c.cgMaxWgsChip[chip] : c.cgMaxWgsMinres;
+    const int capMinres = chip >= 0 ? c.cgMaxWgsChip[chip] : std::max(1, c.cgMaxWgsMinres);
     if (wg > (rowForm ? c.cgMaxWgsRow : c.cgMaxWgs) || wgM > capMinres)
         throw std::runtime_error("CG launch exceeds the resident workgroup budget");
     c.stats.cg_workgroups = uint32_t(wg + wgM);
-    double* partial = c.buf<double>("cg_partial", size_t(2) * (wg + wgM));
+    double* partial = rowForm ? nullptr : c.buf<double>("cg_partial", size_t(2) * (wg + wgM));
     GroupCtl* ctl = c.buf<GroupCtl>("cg_ctl", PSR_MAX_DEPTH + 1);
     const int ctlWords = int(sizeof(GroupCtl) / 4) * (PSR_MAX_DEPTH + 1);
     int* iters = res->cgIters;  // [inner iterations | outer steps] per depth
@@ -2513,10 +2513,19 @@ void solve_depths(Ctx& c) {
     c.cgSlots = slots;
     c.cgSlotWords = slotWords;
     RowMapArgs maps{o.neigh, val, c.tables.weights, o.q1Fired, nullptr, nullptr, nullptr};
+    char* rowState = nullptr;  // of the row form: the rows' records
+    float* rowOut = nullptr;   // and the mixed form's outer residual
     if (rowForm) {
-        maps.places = c.buf<unsigned>("cg_places", size_t(13) * M);
-        maps.ghosts = c.buf<int>("cg_ghosts", size_t(kGhostMax) * wg);
-        maps.heads = c.buf<RowHead>("cg_heads", wg);
+        BlockParts parts;
+        const size_t oPlaces = parts.add(sizeof(unsigned) * 13 * M), oGhosts = parts.add(sizeof(int) * kGhostMax * wg),
+                     oHeads = parts.add(sizeof(RowHead) * wg),
+                     oState = parts.add((mixed ? sizeof(float4) : sizeof(float2)) * 2 * M), oOut = parts.add(sizeof(float) * M);
+        char* block = c.buf<char>("cg_rows", parts.bytes);
+        maps.places = reinterpret_cast<unsigned*>(block + oPlaces);
+        maps.ghosts = reinterpret_cast<int*>(block + oGhosts);
+        maps.heads = reinterpret_cast<RowHead*>(block + oHeads);
+        rowState = block + oState;
+        rowOut = reinterpret_cast<float*>(block + oOut);
     }
     const CoarsePlan& coarse = c.fld.foldArgs.plan;
     const int mapBlocks = rowForm ? wg : 0;
@@ -2561,13 +2570,12 @@ void solve_depths(Ctx& c) {
     if (mixed) {
         P.relTol = PM.relTol = c.cfg.refine_rel_tol;
         P.maxOuter = PM.maxOuter = std::max(1, c.cfg.refine_max_outer);
-        float* rOut = c.buf<float>("cg_rout", M);
-        Comp2* partialC = c.buf<Comp2>("cg_partial_c", size_t(2) * (wg + wgM));
         if (rowForm) {
-            float4* state = c.buf<float4>("cg_state4", size_t(2) * M);
             launch_kernel<cg_mixed_row_k>(&siteMixedRow, cg_mixed_row, wg, 0, s, true, P, maps, c.fld.div, c.fld.dx,
-                                          rOut, state, slots, iters, resid, trueRel, err);
+                                          rowOut, reinterpret_cast<float4*>(rowState), slots, iters, resid, trueRel, err);
         } else {
+            float* rOut = c.buf<float>("cg_rout", M);
+            Comp2* partialC = c.buf<Comp2>("cg_partial_c", size_t(2) * (wg + wgM));
             // also the on-chip MINRES's two buffers of records
             float* rbuf = c.buf<float>("cg_rbuf", size_t(chip >= 0 ? 4 : 2) * M);
             float* wbuf = c.buf<float>("cg_wbuf", size_t(2) * M);
@@ -2593,9 +2601,8 @@ void solve_depths(Ctx& c) {
                                                  ctl + P.ngroups, iters, resid, trueRel, err, res->cgSlotMask);
         }
     } else if (rowForm) {
-        float2* state = c.buf<float2>("cg_state2", size_t(2) * M);
-        launch_kernel<cg_fp32_row_k>(&siteRow, cg_fp32_row, wg, 0, s, true, P, maps, c.fld.div, c.fld.dx, state, slots,
-                                     iters, resid, err);
+        launch_kernel<cg_fp32_row_k>(&siteRow, cg_fp32_row, wg, 0, s, true, P, maps, c.fld.div, c.fld.dx,
+                                     reinterpret_cast<float2*>(rowState), slots, iters, resid, err);
     } else {
         float* r = c.buf<float>("cg_r", M);
         float* pA = c.buf<float>("cg_pa", M);

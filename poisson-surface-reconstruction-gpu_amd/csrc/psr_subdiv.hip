@@ -2062,24 +2062,28 @@ void extract_mesh_b(Ctx& c) {
         const int* rootPos = mm.rootPos;
         float* isoDev = &c.results()->iso;
         const float4* nbrCol = c.fld.nbrCol;
-        int* rootNbr = c.buf<int>("sub_root_nbr", size_t(27) * mm.nRoots);
-        int* rootChain = c.buf<int>("sub_root_chain", size_t(kChain) * mm.nRoots);
-        int4* rootCell = c.buf<int4>("sub_root_cell", mm.nRoots);
-        unsigned* rootSet = c.buf<unsigned>("sub_root_set", mm.nRoots);
-        const RootRecArgs ra{mm.nRoots, M,        L,       finerDepth, mm.roots, rootPos,  o.neigh,
-                             o.parent,  o.key,    rootNbr, rootChain,  rootCell, rootSet};
-        const int rootBlocks = int(div_up(size_t(27) * mm.nRoots, kThreads));
         int nOneRoots = 0;  // roots of one-root tiles
         for (int d = 0; d <= D - 3; ++d) nOneRoots += mm.rootsPerDepth[d];
         // tiles read d_x from dense per-depth grids when the octree is geometric
         const bool denseHalo = !mm.q1Fired;
-        // the roots' polynomials, where the tiles are bounded
+        // whether the tiles are bounded, by their roots' polynomials
         const size_t oneTiles = one_root_tiles(mm, D);
         const size_t launchTiles = current_recorder() ? c.batchTiles : oneTiles;  // of a batch's clouds together
         const size_t boundMin = c.boundTilesMin >= 0 ? size_t(c.boundTilesMin) : size_t(kBoundTilesMin);
-        float* rootPoly = denseHalo && oneTiles > 0 && launchTiles >= boundMin
-                              ? c.buf<float>("sub_root_poly", size_t(kPolyWords) * nOneRoots)
-                              : nullptr;
+        const bool bounded = denseHalo && oneTiles > 0 && launchTiles >= boundMin;
+        BlockParts rootParts;
+        const size_t nR = size_t(mm.nRoots), oCell = rootParts.add(sizeof(int4) * nR), oNbr = rootParts.add(sizeof(int) * 27 * nR),
+                     oChain = rootParts.add(sizeof(int) * kChain * nR), oSet = rootParts.add(sizeof(unsigned) * nR),
+                     oPoly = rootParts.add(bounded ? sizeof(float) * kPolyWords * nOneRoots : 0);
+        char* rootBlock = c.buf<char>("sub_roots", rootParts.bytes);
+        int4* rootCell = reinterpret_cast<int4*>(rootBlock + oCell);
+        int* rootNbr = reinterpret_cast<int*>(rootBlock + oNbr);
+        int* rootChain = reinterpret_cast<int*>(rootBlock + oChain);
+        unsigned* rootSet = reinterpret_cast<unsigned*>(rootBlock + oSet);
+        float* rootPoly = bounded ? reinterpret_cast<float*>(rootBlock + oPoly) : nullptr;
+        const RootRecArgs ra{mm.nRoots, M,        L,       finerDepth, mm.roots, rootPos,  o.neigh,
+                             o.parent,  o.key,    rootNbr, rootChain,  rootCell, rootSet};
+        const int rootBlocks = int(div_up(size_t(27) * mm.nRoots, kThreads));
         for (const SetDesc& S : sets) {
             int halo = 0;
             if (denseHalo && D - S.rd >= 3 &&
@@ -2173,11 +2177,15 @@ void extract_mesh_b(Ctx& c) {
                 int words = 0;
                 for (int k = 0; k < nCs; ++k)
                     if (D - cs[k].rd >= 3) words = std::max(words, grid_tile_words(D, cs[k].rd));
-                ptOwner = c.buf<unsigned>("sub_point_owner", size_t(nOne) * kTilePoints);
+                BlockParts parts;
+                const size_t oOwner = parts.add(sizeof(unsigned) * kTilePoints * nOne),
+                             oSign = parts.add(bounded ? sizeof(int) * nOne : 0), oState = parts.add(bounded ? sizeof(int) * nOne : 0);
+                char* block = c.buf<char>("sub_one_root_tiles", parts.bytes);
+                ptOwner = reinterpret_cast<unsigned*>(block + oOwner);
                 int* sign = nullptr;
-                if (rootPoly) {
-                    sign = c.buf<int>("sub_tile_sign", nOne);
-                    state = c.buf<int>("sub_tile_state", nOne);
+                if (bounded) {
+                    sign = reinterpret_cast<int*>(block + oSign);
+                    state = reinterpret_cast<int*>(block + oState);
                     c.mc.tileState = state;
                     c.mc.boundTiles = nOne;
                     PSR_LAUNCH(sub_bound, div_up(nOne, kBoundTiles), 0, st, gr, dtiles, nOne,
