@@ -437,6 +437,7 @@ int Batch::run(const psr_points* pts, uint32_t count, psr_mesh* outs, std::vecto
             target = std::max(64, (target + 63) / 64 * 64);
         }
         for (uint32_t i : live) clouds_[i]->c.cgRowTarget = target;
+        const size_t planned = live.size();
         phase(
             [&](Ctx& c, uint32_t) {
                 build_octree_b(c);
@@ -447,7 +448,8 @@ int Batch::run(const psr_points* pts, uint32_t count, psr_mesh* outs, std::vecto
                 extract_mesh_a(c);
             },
             true);
-        if (cand >= 0) tuner().report(tkey, cand, elapsed(b.ev[10], b.ev[11]));
+        // (the time of a phase that lost a cloud says nothing of the plan)
+        if (cand >= 0 && live.size() == planned) tuner().report(tkey, cand, elapsed(b.ev[10], b.ev[11]));
         size_t tiles = 0;
         for (uint32_t i : live) tiles += bounded_tiles(clouds_[i]->c);
         for (uint32_t i : live) clouds_[i]->c.batchTiles = tiles;

@@ -2445,16 +2445,20 @@ void solve_depths(Ctx& c) {
     // A batch sets the rows a workgroup takes instead (cgRowTarget, from the
     // batch's total rows and the resident budget): a depth of n rows gets
     // ceil(n / target) workgroups of equal shares; one row per thread when
-    // every share fits the workgroup's threads.
+    // every share fits the workgroup's threads.  The target is the whole batch's,
+    // in several waves of the budget: a cloud whose own workgroups would not all
+    // be resident doubles it until they are.
     int capRows[PSR_MAX_DEPTH + 1];
-    if (c.cgRowTarget > 0) {
-        rowForm = true;
+    for (long long target = c.cgRowTarget; target > 0; target *= 2) {
+        rowForm = !anyIndef;
+        long long w[2] = {0, 0};  // workgroups of the CG and of the MINRES launch
         for (int d = 0; d <= D; ++d) {
-            const int w = std::max(1, int(div_up(L.count[d], unsigned(c.cgRowTarget))));
-            capRows[d] = std::max(1, int(div_up(L.count[d], unsigned(w))));
+            const int n = std::max(1, int(div_up(L.count[d], unsigned(target))));
+            capRows[d] = std::max(1, int(div_up(L.count[d], unsigned(n))));
             if (capRows[d] > kRowThreads || blocks_of(L.count[d], capRows[d]) > kRowMaxBlocks) rowForm = false;
+            w[isMinres[d] ? 1 : 0] += std::max(1, int(div_up(L.count[d], unsigned(capRows[d]))));
         }
-        if (anyIndef) rowForm = false;
+        if (w[0] <= (rowForm ? c.cgMaxWgsRow : c.cgMaxWgs) && w[1] <= std::max(1, c.cgMaxWgsMinres)) break;
     }
     // largest depths first so their groups start on separate CUs early; the
     // MINRES depths form a second launch (PM) with its own workgroup numbering
