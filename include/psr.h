@@ -141,6 +141,8 @@ enum {
     PSR_ARRAY_WELDED_TRIANGLES, /* int32 [n_triangles][3], after psr_weld_mesh */
     PSR_ARRAY_SUBDIV_TILE_SIGNS, /* int32 per bounded one-root tile of the last subdivision working set: the sign of a
                                     tile that the bound left out, else 0; empty where no bound was taken */
+    PSR_ARRAY_CG_FORM,          /* int32 [D+1], how each depth was solved: 1 CG with a row per thread, 0 CG with several;
+                                   4, 8 or 16 MINRES with that many rows a thread on chip, -1 MINRES from memory */
     PSR_ARRAY_COUNT_
 };
 

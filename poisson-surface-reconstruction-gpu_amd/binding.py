@@ -26,7 +26,7 @@ ARRAYS = ["SORTED_POS", "SORTED_NRM", "CODES", "ORDER", "POINT2NODE", "NODE_KEY"
           "LEVEL_COUNT", "NORM_PARAMS", "VFIELD", "DIVERGENCE", "DX", "CHI_POINTS", "VERTS", "EDGES", "FACES",
           "NODE_VERTICES", "NODE_EDGES", "NODE_FACES", "VVALUE", "MESH_VERTICES", "MESH_TRIANGLES", "TABLE_DOT",
           "TABLE_DDOT", "TABLE_D2DOT", "CUBE", "MESH_VERTEX_KEYS", "WELDED_VERTICES", "WELDED_TRIANGLES",
-          "SUBDIV_TILE_SIGNS"]
+          "SUBDIV_TILE_SIGNS", "CG_FORM"]
 ARRAY_ID = {n: i for i, n in enumerate(ARRAYS)}
 _ARRAY_LAYOUT = {
     "SORTED_POS": (np.float32, 4), "SORTED_NRM": (np.float32, 4), "NODE_CHILDREN": (np.int32, 8),

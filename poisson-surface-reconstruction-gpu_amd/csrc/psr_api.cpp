@@ -233,6 +233,8 @@ int psr_create(const psr_config* cfg, void* hip_stream, psr_ctx** out) {
         if (const char* e = std::getenv("PSR_CG_ROWS_PER_WG")) c.cgRowsPerWg = std::max(0, std::atoi(e));
         // test override of the CG barriers' spin bound (forces their time-out path)
         if (const char* e = std::getenv("PSR_CG_SPIN_LIMIT")) c.cgSpinLimit = std::max(0, std::atoi(e));
+        // test override: the MINRES reads and writes its vectors in memory at every size
+        if (const char* e = std::getenv("PSR_CG_MINRES_IN_MEMORY")) c.minresInMemory = std::atoi(e) != 0;
         // test override of the number of subdivision tiles from which a bound leaves some out
         if (const char* e = std::getenv("PSR_SUBDIV_BOUND_TILES")) c.boundTilesMin = std::max(0, std::atoi(e));
         PSR_HIP_CHECK(hipGetDevice(&c.device));
@@ -452,12 +454,13 @@ int psr_export(psr_ctx* ctx, int id, void* dst, uint64_t bytes, uint64_t* needed
             return PSR_OK;
         }
         case PSR_ARRAY_LEVEL_BASE:
-        case PSR_ARRAY_LEVEL_COUNT: {
+        case PSR_ARRAY_LEVEL_COUNT:
+        case PSR_ARRAY_CG_FORM: {
             size_t n = (id == PSR_ARRAY_LEVEL_BASE) ? D + 2 : D + 1;
             if (needed) *needed = 4 * n;
             if (!dst) return PSR_OK;
             if (bytes < 4 * n) return PSR_ERR_CAPACITY;
-            std::memcpy(dst, id == PSR_ARRAY_LEVEL_BASE ? o.L.base : o.L.count, 4 * n);
+            std::memcpy(dst, id == PSR_ARRAY_LEVEL_BASE ? o.L.base : (id == PSR_ARRAY_LEVEL_COUNT ? o.L.count : c.cgForm), 4 * n);
             return PSR_OK;
         }
         case PSR_ARRAY_NORM_PARAMS: src = {o.normParams, 16, 0}; break;

@@ -256,6 +256,8 @@ struct Ctx {
     int cgRowTarget = 0;         // batch: rows a CG workgroup takes (0: the single-cloud plan)
     int cgSpinLimit = -1;        // spin bound of the CG barriers (-1: the default)
     size_t batchTiles = 0;       // batch: bounded_tiles of all its clouds
+    bool minresInMemory = false; // the MINRES never keeps its vectors on chip
+    int cgForm[PSR_MAX_DEPTH + 1] = {};  // how each depth was solved (PSR_ARRAY_CG_FORM)
     int boundTilesMin = -1;      // one-root subdivision tiles from which they are bounded (-1: the default)
     bool indefinite[PSR_MAX_DEPTH + 1] = {};  // the depth's operator after the 1e-6 drop is indefinite
     template <class T>

@@ -2486,7 +2486,8 @@ void solve_depths(Ctx& c) {
         int widest = 0;
         for (int k = 0; k < PM.ngroups; ++k) widest = std::max(widest, PM.g[k].rowsPerWg);
         const int want = widest <= 4 * kCgThreads ? 0 : (widest <= 8 * kCgThreads ? 1 : 2);
-        if (widest <= 16 * kCgThreads && wgM <= c.cgMaxWgsChip[want] && wgM <= kFoldParts * kCgThreads) chip = want;
+        if (!c.minresInMemory && widest <= 16 * kCgThreads && wgM <= c.cgMaxWgsChip[want] && wgM <= kFoldParts * kCgThreads)
+            chip = want;
     }
     const int capMinres = chip >= 0 ? c.cgMaxWgsChip[chip] : std::max(1, c.cgMaxWgsMinres);
     if (wg > (rowForm ? c.cgMaxWgsRow : c.cgMaxWgs) || wgM > capMinres)
@@ -2616,6 +2617,7 @@ void solve_depths(Ctx& c) {
                                        pA, pB, Ap, partial, ctl, iters, resid, err, res->cgSlotMask);
     }
     c.stats.cg_row_form = rowForm ? 1 : 0;
+    for (int d = 0; d <= D; ++d) c.cgForm[d] = isMinres[d] ? (chip >= 0 ? 4 << chip : -1) : (rowForm ? 1 : 0);
     if (!recording) {
         PSR_HIP_CHECK(hipEventRecord(c.ev[9], s));
         std::lock_guard<std::mutex> order(cg_order_lock());
