@@ -131,44 +131,60 @@ def cpu_baseline(xyz, nrm, depth, reps, threads):
 
 
 
-def cg_kernel_name(st, precision):
-    """The CG kernel(s) of the solve: a mixed solve with several rows per
-    thread and a depth 9 or deeper (the indefinite depth solved with MINRES,
-    in a launch of its own) runs two kernels, named "a+b"."""
-    if st["cg_row_form"]:
+def cg_kernel_name(forms, precision):
+    """The CG kernel(s) of the solve, by the form the library reports for each
+    depth (CG_FORM): a mixed solve with an indefinite depth runs the MINRES in
+    a launch of its own and is named "a+b"."""
+    if forms[0] == 1:
         return "cg_mixed_row" if precision == "mixed" else "cg_fp32_row"
-    if precision == "mixed":
-        return "cg_mixed_all_depths+cg_minres_chip16" if st["depth"] >= 9 else "cg_mixed_all_depths"
-    return "cg_all_depths"
+    if precision != "mixed":
+        return "cg_all_depths"
+    minres = {f: "cg_minres_chip%d" % f if f > 0 else "cg_mixed_minres" for f in forms if f not in (0, 1)}
+    return "+".join(["cg_mixed_all_depths"] + [minres[f] for f in sorted(minres)])
 
 
-def cg_algorithmic_bytes(st, precision):
+ROW_WORKGROUP = 512  # rows of a workgroup of the one-row form
+
+
+def rows_read_elsewhere(rec, st):
+    """Per depth, the rows with a neighbour outside their workgroup of the
+    one-row form: those whose records other workgroups read every sweep."""
+    base, nb = rec.export("LEVEL_BASE"), rec.export("NODE_NEIGHS")
+    out = []
+    for d, n in enumerate(st["nodes_per_depth"]):
+        own = np.arange(n) // ROW_WORKGROUP
+        j = nb[base[d]:base[d] + n]
+        out.append(int(((j >= 0) & ((j - base[d]) // ROW_WORKGROUP != own[:, None])).any(1).sum()))
+    return out
+
+
+def cg_algorithmic_bytes(st, precision, forms, shared):
     """HBM bytes the CG launch must move, per depth with z stored operator
-    entries (4 B value + 4 B column) and n rows, each array read once per pass.
-    One row per thread (stencil held on chip, read once): FP32 8z + 16n (b in,
-    records out, x out) + 16n per iteration (8-byte records {r, p} read and
-    written); mixed 8z + 8n (b, x) + 28n per outer step (rhs, 12-byte records
-    out; b, x, residual) + 28n per inner iteration (records {r, w, s} read and
-    written, x out).  Several rows per thread (stencil read every sweep):
-    FP32 (CGAlgorithm.cu:10-80) 8z + 48n per iteration; mixed 8n, then
-    16z + 32n per outer step and 8z + 40n per inner iteration; a depth solved
-    with MINRES (9 and deeper) keeps stencil and vectors on chip, so that its
-    inner iterations move only the workgroups' outer records, which are not
-    counted."""
+    entries and n rows, each array read or written once per pass.
+    One row per thread: vectors, columns and weights stay on chip; 4z + 8n (a
+    column per entry, b in, x out), mixed 8n more per outer step (right-hand
+    side in, residual out), and per iteration the records of the s rows that
+    other workgroups read, out and in: FP32 16s ({r, p}, 8 bytes), mixed 32s
+    ({r, w, s, x}, 16 bytes; one more per outer step).
+    Several rows per thread (stencil read every sweep, 4 B value and 4 B column
+    an entry): FP32 (CGAlgorithm.cu:10-80) 8z + 48n per iteration; mixed, and a
+    depth solved with MINRES from memory, 8n, then 16z + 32n per outer step and
+    8z + 40n per inner iteration.  None where a depth's MINRES runs on chip:
+    what it must move is not known here."""
     total = 0
-    row = bool(st["cg_row_form"])
-    per_depth = zip(st["cg_iterations"], st["cg_nnz"], st["nodes_per_depth"], st["cg_outer"])
-    for d, (k, z, n, o) in enumerate(per_depth):
-        if row and precision == "mixed":
-            total += 8 * z + 8 * n + o * 28 * n + k * 28 * n
-        elif row:
-            total += 8 * z + 16 * n + k * 16 * n
+    per_depth = zip(st["cg_iterations"], st["cg_nnz"], st["nodes_per_depth"], st["cg_outer"], forms, shared)
+    for k, z, n, o, form, s in per_depth:
+        if form > 1:
+            return None
+        if form == 1 and precision == "mixed":
+            total += 4 * z + 8 * n + o * 8 * n + (o + k) * 32 * s
+        elif form == 1:
+            total += 4 * z + 8 * n + k * 16 * s
         elif precision == "mixed":
-            inner = 0 if d >= 9 else k * (8 * z + 40 * n)
-            total += 8 * n + o * (16 * z + 32 * n) + inner
+            total += 8 * n + o * (16 * z + 32 * n) + k * (8 * z + 40 * n)
         else:
             total += k * (8 * z + 48 * n)
-    return total
+    return float(total)
 
 
 def measure(pkg, tx, tn, depth, precision, steps, warmup):
@@ -191,11 +207,13 @@ def measure(pkg, tx, tn, depth, precision, steps, warmup):
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
     st = rec.stats()
+    forms = [int(f) for f in rec.export("CG_FORM")]
+    shared = rows_read_elsewhere(rec, st) if forms[0] == 1 else [0] * len(forms)
     rec.close()
     assert st["n_runs"] - before["n_runs"] == steps
     cg_ms = (st["ms_cg_kernel_sum"] - before["ms_cg_kernel_sum"]) / steps
     return {"value": steps / dt, "ms_per_step": dt * 1e3 / steps, "cg_ms": cg_ms,
-            "cg_bytes": float(cg_algorithmic_bytes(st, precision)), "stats": st}
+            "cg_bytes": cg_algorithmic_bytes(st, precision, forms, shared), "cg_forms": forms, "stats": st}
 
 
 # Non-CG algorithmic bytes of one reconstruction of the 200k-point torus at
@@ -390,8 +408,8 @@ def main():
     head = forms[-1]  # the headline form: mixed precision when both run
     h = res[head]
     st = h["stats"]
-    kernel = cg_kernel_name(st, head)
-    achieved = h["cg_bytes"] / (h["cg_ms"] * 1e-3) / 1e9
+    kernel = cg_kernel_name(h["cg_forms"], head)
+    achieved = h["cg_bytes"] / (h["cg_ms"] * 1e-3) / 1e9 if h["cg_bytes"] is not None else None
     metric = ("reconstructions/sec at depth 7, 200k pts; mixed-prec vs FP32 at <=1e-5 residual" if a.workload == "torus"
               else "reconstructions/sec, %s" % WORKLOADS[a.workload])
     line = {
@@ -411,7 +429,7 @@ def main():
                    "precision": head, "nodes": st["n_nodes"], "cg_iterations": st["cg_iterations"],
                    "mesh_triangles": st["mesh_triangles"]},
         "roofline": {"kernel": kernel, "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                     "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS if achieved is not None else None,
                      "traffic": measured_traffic(a.workload, head, kernel),
                      "ms_per_launch": h["cg_ms"], "bytes_per_launch": h["cg_bytes"]},
         "stage_ms": {k: st[k] for k in ("ms_octree", "ms_field", "ms_solve", "ms_mesh", "ms_total")},
