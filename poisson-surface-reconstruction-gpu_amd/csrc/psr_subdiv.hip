@@ -2051,8 +2051,13 @@ void extract_mesh_b(Ctx& c) {
     size_t triTotal = mm.nTri, keptSub = 0, keptMainHost = 0;
     float* outV = c.buf_keep<float>("mesh_vertices", 3 * (deferred ? vCap : size_t(std::max(mm.nCross, 1))), 0);
     unsigned* outKey = c.buf_keep<unsigned>("mesh_vertex_keys", deferred ? vCap : size_t(std::max(mm.nCross, 1)), 0);
-    // the depth-D batch's kept vertices: compacted by the first set-up launch
+    // the depth-D batch's kept vertices: compacted by the first set-up launch.
+    // The tile scans' state is reserved with it: grown between two launches of a
+    // recording it would clear the counters that the first is still to use.
     const int keepBlocks = std::max(1, int(div_up(mm.nCross, kThreads)));
+    size_t tilesAll = 0;
+    for (int k = 0; k < nSets; ++k) tilesAll += div_up(setCells[k], unsigned(kTile));
+    c.scan_for_tiles(std::max<size_t>(keepBlocks, size_t(3) * div_up(tilesAll, kScanThreads * kScanPer)));
     const KeepArgs ka{mainV, mainKey, mm.nCross,
                       scan_ticket(c.scan_for_tiles(size_t(keepBlocks)), keepBlocks, keptMain), outV, outKey};
     if (nSets == 0) PSR_LAUNCH(sub_setup, keepBlocks, 0, st, ka, keepBlocks, RootRecArgs{}, 0, RootPolyArgs{}, 0,
