@@ -51,7 +51,7 @@ typedef struct {
     uint32_t batch_workers;      /* psr_reconstruct_batch: clouds merged into each launch (a pass);
                                     0 = 64 */
     int32_t batch_cg_plan;       /* psr_reconstruct_batch, how the clouds' CG solves are laid out:
-                                    0 = the single-cloud plan (256 rows a workgroup, in as many waves
+                                    0 = the single-cloud plan (512 rows a workgroup, in as many waves
                                     of the resident budget as needed: meshes equal psr_reconstruct's
                                     bit for bit); w >= 1 = every depth's rows split evenly over
                                     workgroups so that all solves fit w waves; -1 (default) = picked
@@ -92,7 +92,7 @@ typedef struct {
     uint32_t cg_workgroups;
     int cg_nnz[PSR_STATS_MAX_DEPTH + 1]; /* stored operator entries per depth */
     int cg_outer[PSR_STATS_MAX_DEPTH + 1]; /* PSR_PRECISION_MIXED: outer refinement steps per depth; 1 otherwise */
-    int cg_row_form;      /* 1: one row per CG thread, stencil held in registers; 0: several rows per thread */
+    int cg_row_form;      /* 1: one row per CG thread, its vectors on chip; 0: several rows per thread */
     double ms_cg_kernel_sum; /* ms_cg_kernel summed over the context's completed runs */
     uint32_t n_runs;         /* completed runs of the context */
     uint64_t device_bytes;   /* device memory the run's buffers needed (the context's fixed tables and

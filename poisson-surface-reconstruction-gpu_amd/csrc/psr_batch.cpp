@@ -40,7 +40,7 @@ namespace {
 // between events), then keeps the fastest.  The shape's first call runs the
 // first candidate untimed.
 struct BatchTuner {
-    // 0: the single-cloud plan (256 rows a workgroup); w: all solves in w
+    // 0: the single-cloud plan (512 rows a workgroup); w: all solves in w
     // waves of the resident budget
     static constexpr int kCandidates[] = {0, 1, 2, 4, 8};
     static constexpr int kCount = int(sizeof(kCandidates) / sizeof(int));

@@ -268,9 +268,9 @@ __device__ __forceinline__ void jacobi3(double (&A)[3][3], double (&V)[3][3]) {
 
 // A candidate as one ordered word: its squared distance (never negative, so
 // its bits order as it does) above its point index, so the smaller word is the
-// closer point, ties to the lower index.  A NaN distance orders behind kNone.
+// closer point, ties to the lower index.
 typedef unsigned long long Cand;
-constexpr Cand kNone = (Cand(0x7f800000u) << 32) | 0x7fffffffu;
+constexpr unsigned kNoPoint = 0x7fffffffu;  // the index of a place without a point
 
 __device__ __forceinline__ int cand_index(Cand c) { return int(unsigned(c)); }
 
@@ -414,7 +414,7 @@ __device__ __forceinline__ void knn_search(float3 p, int sub, int kk, const Grid
     const bool ties = m > kListCap;
     unsigned tie[K];
 #pragma unroll
-    for (int j = 0; j < K; ++j) tie[j] = 0x7fffffffu;
+    for (int j = 0; j < K; ++j) tie[j] = kNoPoint;
     if (ties) {
         // more points at the kk-th distance than the list holds: once more, the
         // nearer ones (fewer than kk) to the list and of those at the kk-th
@@ -489,7 +489,7 @@ __global__ void __launch_bounds__(kThreads) ne_estimate(const char* __restrict__
     const float4 p4 = spos[at];
     const float3 p = make_float3(p4.x, p4.y, p4.z);
     const int i = __float_as_int(p4.w);
-    // kNone's index (fewer than kk points have a distance: NaN coordinates) reads as NaN
+    // kNoPoint (fewer than kk points have a distance: NaN coordinates) reads as NaN
     auto point = [&](int q) {
         return q < n ? load_point(xyz, stride, q) : make_float3(NAN, NAN, NAN);
     };

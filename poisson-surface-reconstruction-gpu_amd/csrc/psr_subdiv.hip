@@ -2175,7 +2175,7 @@ void extract_mesh_b(Ctx& c) {
             int4* tileCnt = c.buf<int4>("sub_tile_cnt", nTiles);
             int4* tileBase = c.buf<int4>("sub_tile_base", nTiles);
             // the one-root tiles' point owners, found by sub_corner_values_grid
-            // and reused by sub_classify (value indices slot * nVD + cell fit 32 bits)
+            // and reused by sub_classify (cell << 3 | slot: a set has less than 2^31 / 12 cells)
             unsigned* ptOwner = nullptr;
             int* state = nullptr;
             if (nOne > 0 && denseHalo) {
